@@ -27,6 +27,24 @@ struct SymvBlock {
     double *xb = nullptr, *ypart = nullptr;
 };
 
+// row of the coarse basis (row-major, k values) and coarse offset of a lambda entry
+struct LamCoarse {
+    int64_t row;
+    int off, k;
+};
+
+// PCG scalars per load case (device) and what the host reads of them (pinned)
+constexpr int PCG_SLOTS = 16, PCG_YW = 0, PCG_YW_PREV = 1, PCG_PAP = 2, PCG_WW = 3, PCG_TOL = 4,
+              PCG_STOP = 5,  // the case rests in this iteration
+              PCG_NEXT = 6,  // ... from the next one on
+              PCG_ITERS = 7, PCG_COUNT = 8;
+struct PcgRecord {
+    int count;   // iterations whose stop test is known
+    int active;  // cases left after it (0 or 1)
+    int iters[16];
+    double ww[16], tol[16], bb[16];
+};
+
 struct DualDev {
     int nsub = 0, nlam = 0, ncoarse = 0, max_m = 0;
     int64_t nbnd = 0;                // sum of m_s
@@ -46,6 +64,8 @@ struct DualDev {
     int *bl_lam = nullptr;
     double *bl_sign = nullptr;
     double *bl_sscale = nullptr;     // sign * scaling weight
+    int *bl_row = nullptr;           // boundary index of every entry
+    int64_t nle = 0;                 // entries
     // lambda -> boundary entries (1 or 2 per lambda, slots 2l, 2l+1)
     int *le_cnt = nullptr;
     int64_t *le_b = nullptr;
@@ -83,6 +103,9 @@ struct DualDev {
     int *cblk = nullptr, *ck = nullptr, *blk_ptr = nullptr, *blk_sub = nullptr;
     int64_t *rtoff = nullptr, *dsub_off = nullptr, *noff = nullptr;
     double *Rt = nullptr, *N = nullptr, *dsub = nullptr;
+    double *RbT = nullptr, *RtT = nullptr;  // R_b and Rt with row-major subdomain blocks
+    LamCoarse *le_coarse = nullptr;         // per lambda entry (2 per lambda)
+    bool coarse_direct = false;             // dsub is the coarse vector (one subdomain per block, in order)
     int64_t *asub = nullptr;          // offset of kernel amplitudes of subdomain s (sum of kdim)
 };
 
@@ -133,59 +156,76 @@ struct PrimalDev {
 // ev0/ev1 (optional) are recorded around the SYMV kernel alone.
 void launch_symv(const DualDev &D, bool sd, int prec, const double *x, int gather, bool scaled, hipStream_t st,
                  hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
-// nr right-hand sides at once on MFMA (1 <= nr <= 16; FP64 storage): x is
-// lambda-space, nr vectors of n_lambda (gathered with sign, or sign*scale when
-// `scaled`); yb receives nr boundary vectors of nbnd; stride nr in the scratch.
-// ev0/ev1 bracket the SYMV kernel.
-void launch_symv_mfma(const DualDev &D, const SymvBlock &B, bool sd, int nr, const double *x, bool scaled,
-                      double *yb, hipStream_t st, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
-void launch_lambda_gather(const DualDev &D, const double *yb, bool scaled, double *y, hipStream_t st);
-void launch_boundary_gather(const DualDev &D, const double *x, bool scaled, double *xb, hipStream_t st);
-void launch_kbb(const DualDev &D, const double *xb, double *yb, hipStream_t st);
-// mode 0: y = x - G^T GGinv G x; mode 1: y = G^T GGinv x (x coarse); mode 2: y = GGinv G x (y coarse)
-void launch_project(const DualDev &D, const double *x, double *y, int mode, hipStream_t st);
+// nr right-hand sides at once on MFMA (1 <= nr <= 16; FP64 storage): xb and
+// yb are boundary vectors interleaved by case.  ev0/ev1 bracket the SYMV kernel.
+void launch_symv_mfma(const DualDev &D, const SymvBlock &B, bool sd, int nr, const double *xb, double *yb,
+                      hipStream_t st, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
+// yb = sum of the SYMV partials (K interleaved cases)
+void launch_part_reduce(const DualDev &D, const SymvItem *items, const int *item0, const int *nitems, int R, int K,
+                        const double *ypart, double *yb, hipStream_t st);
+
+// ---- pcg.hip: K interleaved vectors (x[l K + v]); K = 1 is the single solve ----
+void launch_entry_rows(int64_t nb, const int64_t *bl_ptr, int *bl_row, hipStream_t st);
+void launch_basis_rows(int nsub, int max_m, const int *M, const int *kcols, const int64_t *roff, const double *R,
+                       double *RT, hipStream_t st);
+void launch_lambda_coarse(const DualDev &D, LamCoarse *le, hipStream_t st);
+// partials per dot product over n lines (one per workgroup, K values each)
+int dot_blocks(int64_t n, int K);
+// y = B y_b; with `part` the partial dot products of y with a
+void launch_lambda_gather(const DualDev &D, int K, const double *yb, bool scaled, double *y, hipStream_t st,
+                          const double *a = nullptr, double *part = nullptr);
+void launch_boundary_gather(const DualDev &D, int K, const double *x, bool scaled, double *xb, hipStream_t st);
+void launch_kbb(const DualDev &D, int K, const double *xb, double *yb, hipStream_t st);
+// SUPER_DIRICHLET: yb = K_bb xb - K_bn diag(K_nn)^-1 K_nb xb (n: interior DOFs
+// next to the boundary; t holds n_near K values of scratch)
+void launch_superdir(const DualDev &D, int K, int64_t n_near, const int64_t *sib_ptr, const int64_t *sib_col,
+                     const double *sib_val, const double *sdiag, const int64_t *sbi_ptr, const int64_t *sbi_col,
+                     const double *sbi_val, double *t, const double *xb, double *yb, hipStream_t st);
+// mode 0: y = x - G^T GGinv G x; mode 1: y = G^T GGinv x (x coarse); mode 2: y = GGinv G x (y coarse).
+// D.dsub, D.cd and D.ce hold K values per entry.  With `part` (modes 0, 1): partial dot
+// products of y with a (null: with y); stop: see k_apply_G
+void launch_project(const DualDev &D, int K, const double *x, double *y, int mode, hipStream_t st,
+                    const double *a = nullptr, double *part = nullptr, double *stop = nullptr);
+void launch_sub_lines(int64_t n, int K, double *y, const double *c, hipStream_t st);  // y_v -= c
+void launch_dot_lines(int64_t n, int K, const double *a, const double *b, double *part, hipStream_t st);
+void launch_pcg_init(int K, const double *part_r, const double *part_b, int np, double precision, double tol_abs,
+                     double *scal, PcgRecord *rec, hipStream_t st);
+void launch_p_update(int64_t n, int K, double *p, const double *y, const double *part_yw, const double *part_ww,
+                     int np, bool first, double *scal, PcgRecord *rec, hipStream_t st);
+void launch_xr_update(int64_t n, int K, double *x, double *r, const double *p, const double *Ap,
+                      const double *part_pAp, int np, double *scal, hipStream_t st);
 // out[asub[s] + a] = -R_s^T (B_s^T x) with the subdomain kernel (hybrid FETI e0)
-void launch_subdomain_kernel_dots(const DualDev &D, const double *x, double *out, hipStream_t st);
+void launch_subdomain_kernel_dots(const DualDev &D, int K, const double *x, double *out, hipStream_t st);
 // y_b += -K^+ B0^T lambda0 (+ R alphaK when addR) after solving the cluster problems
 // lowp: apply -F_i B0^T lambda0 with FB0f (the inner iterations on the FP32/BF16 F_i)
 void launch_cluster_correction(const DualDev &D, const ClusterDev &C, const double *e0s, double *yb, int addR,
                                hipStream_t st, bool lowp = false);
 // FB0f = FB0 rounded to FP32 (for the inner iterations on FP32/BF16 storage)
 void launch_fb0_round(const DualDev &D, const ClusterDev &C, hipStream_t st);
-// the correction for nr cases of a block (case strides ystr, tstr/lstr, astr):
-// t_v = F0^-1 B0 y_b,v into t (the lambda0 layout), then per case alpha and
-// lambda0 (launch_cluster_alpha), then y_b,v += -F B0^T lambda0_v + R alphaK_v
-void launch_cluster_t_multi(const DualDev &D, const ClusterDev &C, int nr, const double *yb, int64_t ystr, double *t,
-                            int64_t tstr, hipStream_t st);
-void launch_cluster_alpha(const ClusterDev &C, const double *e0s, double *lam0, double *alphaK, hipStream_t st);
-void launch_cluster_apply_multi(const DualDev &D, const ClusterDev &C, int nr, const double *lam0, int64_t lstr,
-                                const double *alphaK, int64_t astr, int addR, double *yb, int64_t ystr,
-                                hipStream_t st);
+// the correction for nr interleaved cases: yb and e0s interleaved, lambda0 and
+// alpha of the cases at strides lstr and astr
+void launch_cluster_correction_multi(const DualDev &D, const ClusterDev &C, int nr, const double *e0s, double *lam0,
+                                     int64_t lstr, double *alphaK, int64_t astr, double *yb, int addR,
+                                     hipStream_t st);
 // set-up: F0 (into C.F0inv) from the corner blocks; H = F0^-1 G0^T and the
 // regularised Sa (into Sa) once C.F0inv holds the inverse
 void launch_cluster_setup_f0(const ClusterDev &C, hipStream_t st);
 void launch_cluster_setup_sa(const ClusterDev &C, double *Sa, hipStream_t st);
-// alpha_tot(s) = alphaK(s) (hybrid) + N_s alpha_coarse
-void launch_alpha_combine(const DualDev &D, const ClusterDev &C, bool hybrid, const double *alpha_coarse,
-                          double *alpha_tot, hipStream_t st);
+// alpha_tot_v(s) = alphaK_v(s) (hybrid) + N_s alpha_coarse,v: alpha_coarse interleaved, the others at stride astr
+void launch_alpha_combine(const DualDev &D, int K, const double *alphaK, int64_t astr, bool hybrid,
+                          const double *alpha_coarse, double *alpha_tot, hipStream_t st);
 void launch_dot(const double *a, const double *b, int64_t n, double *partial, double *out, hipStream_t st);
-void launch_p_update(double *p, const double *y, int64_t n, const double *num, const double *den, int first,
-                     hipStream_t st);
-void launch_xr_update(double *x, double *r, const double *p, const double *Ap, int64_t n, const double *num,
-                      const double *den, hipStream_t st);
 void launch_axpby(double *y, const double *a, const double *b, int64_t n, double alpha, double beta, hipStream_t st);
-void launch_copy_scalar(const double *src, double *dst, hipStream_t st);
 void launch_symmetrize(double *A, int n, hipStream_t st);
 void launch_primal(const PrimalDev &P, int nsub, const double *ub, double *u, hipStream_t st);
 // new loads f (local DOF order, all subdomains): P.yf = L^-1 f_int, hf = f_b - K_bi K_ii^-1 f_int
 void launch_rhs_prepare(const PrimalDev &P, int nsub, const double *f, double *hf, hipStream_t st);
-// nr load vectors at once (strides between vectors fstr, hstr, ystr; work:
+// nr load vectors at once (strides fstr, ystr; hf and ub interleaved; work:
 // 16 values per interior row, P.work_off layout)
 void launch_rhs_prepare_multi(const PrimalDev &P, int nsub, int nr, const double *f, int64_t fstr, double *hf,
-                              int64_t hstr, double *yf, int64_t ystr, double *work, hipStream_t st);
-void launch_primal_multi(const PrimalDev &P, int nsub, int nr, const double *ub, int64_t bstr, const double *yf,
-                         int64_t ystr, const double *alpha, int64_t astr, double *u, int64_t ustr, double *work,
-                         hipStream_t st);
+                              double *yf, int64_t ystr, double *work, hipStream_t st);
+void launch_primal_multi(const PrimalDev &P, int nsub, int nr, const double *ub, const double *yf, int64_t ystr,
+                         const double *alpha, int64_t astr, double *u, int64_t ustr, double *work, hipStream_t st);
 // sens[e] = -w_e^T Ke0 u_e over the NE[0] x NE[1] x NE[2] HEXA8 grid (nodal fields, ndof nd)
 void launch_element_sensitivity(const int *NE, int nd, const double *Ke0, const double *u, const double *w,
                                 double *sens, hipStream_t st);
@@ -201,11 +241,6 @@ void launch_copy(const double *src, double *dst, int64_t n, hipStream_t st);
 // read-only stream over n doubles (n even) with `wgs` workgroups (out: wgs doubles)
 void launch_stream_read(const double *src, int64_t n, int wgs, double *out, hipStream_t st);
 
-// SUPER_DIRICHLET: yb = K_bb xb - K_bn diag(K_nn)^-1 K_nb xb (n: interior DOFs
-// next to the boundary; t holds n_near values of scratch)
-void launch_superdir(const DualDev &D, int64_t n_near, const int64_t *sib_ptr, const int64_t *sib_col,
-                     const double *sib_val, const double *sdiag, const int64_t *sbi_ptr, const int64_t *sbi_col,
-                     const double *sbi_val, double *t, const double *xb, double *yb, hipStream_t st);
 // KKT sums per subdomain (out: 2 per subdomain) and the boundary values of u
 // (ub); part holds 2 nsub kkt_groups(max_n) partial sums (max_n: the largest
 // subdomain's DOF count)

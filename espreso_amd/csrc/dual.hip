@@ -168,23 +168,6 @@ __global__ void __launch_bounds__(256) k_symv(const SymvItem *__restrict__ items
         ypart[it.part_off + j] = finite ? ldexp((double)(long long)ys[j], -k) * sc : __builtin_nan("");
 }
 
-// yb[boff+j] = sum of the partials of the items of subdomain s covering j
-__global__ void k_part_reduce(const SymvItem *items, const int *item0, const int *nitems, const int *M,
-                              const int64_t *boff, int R, const double *ypart, double *yb) {
-    const int s = blockIdx.x;
-    const int m = M[s];
-    const int i0 = item0[s], ni = nitems[s];
-    for (int j = threadIdx.x; j < m; j += blockDim.x) {
-        double v = 0.0;
-        for (int q = 0; q < ni; q++) {
-            const SymvItem it = items[i0 + q];
-            const int j0 = it.t0 * R;
-            if (j >= j0) v += ypart[it.part_off + j - j0];
-        }
-        yb[boff[s] + j] = v;
-    }
-}
-
 // Block SYMV on MFMA (v_mfma_f64_16x16x4f64): up to 16 right-hand sides, the
 // MFMA's N dimension (lanes of right-hand sides past nr carry zeros).  An
 // item is at most BLOCK_STRIPS strips of one subdomain; wave w owns the
@@ -310,67 +293,6 @@ __global__ void __launch_bounds__(256) k_symv_mfma(const SymvItem *__restrict__ 
     }
 }
 
-// yb[v * nbnd + boff + j] = sum of the block partials covering j (fixed order)
-__global__ void k_part_reduce_mfma(const SymvItem *items, const int *item0, const int *nitems, const int *M,
-                                   const int64_t *boff, int64_t nbnd, int nr, const double *ypart, double *yb) {
-    const int s = blockIdx.x;
-    const int m = M[s];
-    const int i0 = item0[s], ni = nitems[s];
-    for (int i = threadIdx.x; i < m * nr; i += blockDim.x) {
-        const int j = i / nr, v = i % nr;
-        double acc = 0.0;
-        for (int q = 0; q < ni; q++) {
-            const SymvItem it = items[i0 + q];
-            const int j0 = it.t0 * STRIP_F64;
-            if (j >= j0) acc += ypart[(it.part_off + j - j0) * nr + v];
-        }
-        yb[v * nbnd + boff[s] + j] = acc;
-    }
-}
-
-// xb[j nr + v] = sum coef * x[v nlam + lambda], v < nr
-__global__ void k_boundary_gather_multi(int64_t nb, int nr, const int64_t *bl_ptr, const int *bl_lam,
-                                        const double *coef, const double *x, int64_t nlam, double *xb) {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nb * nr;
-         i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t j = i / nr;
-        const int v = (int)(i % nr);
-        double acc = 0.0;
-        for (int64_t q = bl_ptr[j]; q < bl_ptr[j + 1]; q++) acc += coef[q] * x[v * nlam + bl_lam[q]];
-        xb[i] = acc;
-    }
-}
-
-// lambda-space y = sum_e coef_e * yb[b_e]
-__global__ void k_lambda_gather(int nlam, const int *cnt, const int64_t *lb, const double *coef, const double *yb,
-                                double *y) {
-    for (int l = blockIdx.x * blockDim.x + threadIdx.x; l < nlam; l += gridDim.x * blockDim.x) {
-        double v = 0.0;
-        for (int e = 0; e < cnt[l]; e++) v += coef[2 * l + e] * yb[lb[2 * l + e]];
-        y[l] = v;
-    }
-}
-
-// boundary gather xb = B^T x with coefficients
-__global__ void k_boundary_gather(int64_t nb, const int64_t *bl_ptr, const int *bl_lam, const double *coef,
-                                  const double *x, double *xb) {
-    for (int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < nb; j += (int64_t)gridDim.x * blockDim.x) {
-        double v = 0.0;
-        for (int64_t q = bl_ptr[j]; q < bl_ptr[j + 1]; q++) v += coef[q] * x[bl_lam[q]];
-        xb[j] = v;
-    }
-}
-
-// boundary SpMV with K_bb (lumped preconditioner): yb = K_bb xb
-__global__ void k_kbb(int64_t nb, const int64_t *ptr, const int64_t *col, const double *val, const double *xb,
-                      double *yb) {
-    for (int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < nb; j += (int64_t)gridDim.x * blockDim.x) {
-        double v = 0.0;
-        for (int64_t q = ptr[j]; q < ptr[j + 1]; q++) v += val[q] * xb[col[q]];
-        yb[j] = v;
-    }
-}
-
 __device__ __forceinline__ double block_sum(double v, double *red) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -381,98 +303,6 @@ __device__ __forceinline__ double block_sum(double v, double *red) {
     const int nw = blockDim.x >> 6;
     for (int w = 0; w < nw; w++) r += red[w];
     return r;
-}
-
-// per subdomain s: out[off[s] + a] = -sum_j R_s[j, a] (B_s^T x)_j for a < k[s]
-// (R_s: m_s x k_s column-major at R + roff[s]); one workgroup of 1024 threads
-// per subdomain (enough loads in flight for a latency-bound gather).
-// With the coarse basis this is G x = -(B R)^T x per subdomain.
-constexpr int APPLY_G_THREADS = 1024;
-__global__ void __launch_bounds__(APPLY_G_THREADS) k_apply_G(const int *M, const int64_t *boff, const int *kcols,
-                                                             const int64_t *outoff, const int64_t *roff,
-                                                             const double *R, const int64_t *bl_ptr,
-                                                             const int *bl_lam, const double *sign, const double *x,
-                                                             double *out) {
-    constexpr int KB = 8;  // columns per pass
-    constexpr int NW = APPLY_G_THREADS / 64;
-    __shared__ double red[KB][NW];
-    const int s = blockIdx.x, m = M[s], k = kcols[s];
-    const int64_t b0 = boff[s];
-    const double *Rs = R + roff[s];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int a0 = 0; a0 < k; a0 += KB) {
-        const int kb = min(KB, k - a0);
-        double acc[KB];
-#pragma unroll
-        for (int a = 0; a < KB; a++) acc[a] = 0.0;
-        for (int j = threadIdx.x; j < m; j += APPLY_G_THREADS) {
-            double xb = 0.0;
-            for (int64_t q = bl_ptr[b0 + j]; q < bl_ptr[b0 + j + 1]; q++) xb += sign[q] * x[bl_lam[q]];
-#pragma unroll
-            for (int a = 0; a < KB; a++)
-                if (a < kb) acc[a] += Rs[j + (int64_t)(a0 + a) * m] * xb;
-        }
-#pragma unroll
-        for (int a = 0; a < KB; a++) {
-            double v = acc[a];
-            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-            if (lane == 0) red[a][w] = v;
-        }
-        __syncthreads();
-        if (threadIdx.x < kb) {
-            double v = 0.0;
-            for (int q = 0; q < NW; q++) v += red[threadIdx.x][q];
-            out[outoff[s] + a0 + threadIdx.x] = -v;
-        }
-        __syncthreads();
-    }
-}
-
-// d[coff[b] + a] = sum over the subdomains of coarse block b of their partials
-__global__ void k_block_sum(int nblk, const int *blk_ptr, const int *blk_sub, const int64_t *subpart_off,
-                            const int *ck, const int *coff, const double *part, double *d) {
-    // one thread per (block, column); blocks hold at most 64 columns
-    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < nblk * 64; e += gridDim.x * blockDim.x) {
-        const int b = e >> 6, a = e & 63;
-        const int q0 = blk_ptr[b], q1 = blk_ptr[b + 1];
-        const int k = ck[blk_sub[q0]];
-        if (a >= k) continue;
-        double v = 0.0;
-        for (int q = q0; q < q1; q++) v += part[subpart_off[blk_sub[q]] + a];
-        d[coff[b] + a] = v;
-    }
-}
-
-// e = GGinv d (symmetric, column access)
-__global__ void __launch_bounds__(256) k_coarse_gemv(int nc, const double *Ginv, const double *d, double *e) {
-    __shared__ double red[4];
-    const int i = blockIdx.x;
-    const double *col = Ginv + (int64_t)i * nc;
-    double v = 0.0;
-    for (int j = threadIdx.x; j < nc; j += 256) v += col[j] * d[j];
-    v = block_sum(v, red);
-    if (threadIdx.x == 0) e[i] = v;
-}
-
-// mode 0: y = x - G^T e ; mode 1: y = G^T e   (G^T e)_l = -sum_entries sign Rt_s[j,:] e_blk(s)
-__global__ void k_project_finish(int nlam, const int *cnt, const int64_t *lb, const int *lsub, const double *sign,
-                                 const int64_t *boff, const int *M, const int *ck, const int *cblk, const int *coff,
-                                 const int64_t *rtoff, const double *Rt, const double *e, const double *x, double *y,
-                                 int mode) {
-    for (int l = blockIdx.x * blockDim.x + threadIdx.x; l < nlam; l += gridDim.x * blockDim.x) {
-        double g = 0.0;
-        for (int q = 0; q < cnt[l]; q++) {
-            const int s = lsub[2 * l + q];
-            const int64_t j = lb[2 * l + q] - boff[s];
-            const int m = M[s];
-            const double *R = Rt + rtoff[s];
-            const double *es = e + coff[cblk[s]];
-            double acc = 0.0;
-            for (int a = 0; a < ck[s]; a++) acc += R[j + (int64_t)a * m] * es[a];
-            g -= sign[2 * l + q] * acc;
-        }
-        y[l] = mode == 0 ? x[l] - g : g;
-    }
 }
 
 // ---- hybrid FETI: cluster correction of K^+ (cluster.cpp:796-916) ----
@@ -519,23 +349,26 @@ __global__ void __launch_bounds__(256) k_cluster_t(const ClusterDev C, const dou
     }
 }
 
-// one workgroup per cluster: alpha = Sa^-1 (G0 t - e0), lambda0 = t - H alpha (in place over t)
+// one workgroup per cluster and case: alpha = Sa^-1 (G0 t - e0), lambda0 = t - H alpha (in place over t);
+// e0s interleaved by case, lam0 and alphaK at strides lstr and astr
 __global__ void __launch_bounds__(1024) k_cluster_alpha(const ClusterDev C, const double *e0s, double *lam0,
-                                                        double *alphaK) {
+                                                        int64_t lstr, double *alphaK, int64_t astr) {
     extern __shared__ double sh[];
-    const int c = blockIdx.x;
+    const int c = blockIdx.x, K = gridDim.y;
+    lam0 += blockIdx.y * lstr;
+    alphaK += blockIdx.y * astr;
     const int n0 = C.n0[c], kt = C.kt[c];
     double *t2 = sh, *al = sh + C.max_kt;
     const int64_t ro = C.rowoff[c];
     const double *t = lam0 + ro;
     const double *G0T = C.G0T + C.g0off[c];  // n0 x kt
-    const double *e0 = e0s + C.eoff[c];      // cluster-contiguous subdomain partials
+    const double *e0 = e0s + C.eoff[c] * K + blockIdx.y;  // cluster-contiguous subdomain partials
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     for (int a = w; a < kt; a += 16) {
         double v = 0.0;
         for (int r = lane; r < n0; r += 64) v += G0T[r + (int64_t)a * n0] * t[r];
         v = wave_sum(v);
-        if (lane == 0) t2[a] = v - e0[a];
+        if (lane == 0) t2[a] = v - e0[(int64_t)a * K];
     }
     __syncthreads();
     const double *Sai = C.Sainv + C.saoff[c];
@@ -696,7 +529,7 @@ void launch_fb0_round(const DualDev &D, const ClusterDev &C, hipStream_t st) {
 // F0^-1 and F_i B0^T are read once per pass instead of once per case.
 // t_v = F0^-1 g0_v, g0_v gathered from the case's SYMV output; 4 rows per
 // wave, kc <= 8 cases (g0 of the kc cases in LDS); grid (rows/16, clusters).
-__global__ void __launch_bounds__(256) k_cluster_t_multi(const ClusterDev C, const double *yb, int64_t ystr,
+__global__ void __launch_bounds__(256) k_cluster_t_multi(const ClusterDev C, const double *yb, int64_t K,
                                                          int kc, double *t, int64_t tstr) {
     extern __shared__ double g0[];  // n0 x kc
     const int c = blockIdx.y;
@@ -707,7 +540,7 @@ __global__ void __launch_bounds__(256) k_cluster_t_multi(const ClusterDev C, con
     for (int e = threadIdx.x; e < n0 * kc; e += 256) {
         const int r = e / kc, v = e % kc;
         double g = 0.0;
-        for (int64_t q = C.re_ptr[ro + r]; q < C.re_ptr[ro + r + 1]; q++) g += C.re_c[q] * yb[v * ystr + C.re_b[q]];
+        for (int64_t q = C.re_ptr[ro + r]; q < C.re_ptr[ro + r + 1]; q++) g += C.re_c[q] * yb[C.re_b[q] * K + v];
         g0[e] = g;
     }
     __syncthreads();
@@ -749,7 +582,7 @@ __global__ void __launch_bounds__(256) k_cluster_apply_multi(const ClusterDev C,
                                                              const int *kdim, const int64_t *rboff, const double *Rb,
                                                              const double *lambda0, int64_t lstr,
                                                              const double *alphaK, int64_t astr, int addR, int kc,
-                                                             double *yb, int64_t ystr) {
+                                                             double *yb, int64_t K) {
     __shared__ double lam[256 * 8];
     const int s = blockIdx.y, m = M[s];
     if (blockIdx.x * 256 >= m) return;  // uniform
@@ -779,22 +612,24 @@ __global__ void __launch_bounds__(256) k_cluster_apply_multi(const ClusterDev C,
             const double *al = alphaK + v * astr + C.asub[s];
             for (int a = 0; a < kdim[s]; a++) val += R[(int64_t)a * m] * al[a];
         }
-        yb[v * ystr + boff[s] + j] += val;
+        yb[(boff[s] + j) * K + v] += val;
     }
 }
 
-// alpha_tot(s) = addK * alphaK(s) + N_s alpha_coarse(block(s))
-__global__ void k_alpha_combine(int nsub, const int *kdim, const int *ck, const int *cblk, const int *coff,
+// alpha_tot_v(s) = addK * alphaK_v(s) + N_s alpha_coarse,v(block(s)), a thread per subdomain and case
+// (alpha_coarse interleaved by case, alphaK and alpha_tot at stride astr)
+__global__ void k_alpha_combine(int nsub, int K, const int *kdim, const int *ck, const int *cblk, const int *coff,
                                 const int64_t *asub, const int64_t *noff, const double *N, const double *alphaK,
-                                int addK, const double *alpha_coarse, double *alpha_tot) {
-    for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < nsub; s += gridDim.x * blockDim.x) {
+                                int addK, const double *alpha_coarse, double *alpha_tot, int64_t astr) {
+    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < nsub * K; e += gridDim.x * blockDim.x) {
+        const int s = e / K, v = e % K;
         const int k = kdim[s], kc = ck[s];
         const double *Ns = N + noff[s];  // k x kc column-major
-        const double *ac = alpha_coarse + coff[cblk[s]];
+        const double *ac = alpha_coarse + (int64_t)coff[cblk[s]] * K + v;
         for (int a = 0; a < k; a++) {
-            double v = addK ? alphaK[asub[s] + a] : 0.0;
-            for (int b = 0; b < kc; b++) v += Ns[a + (int64_t)b * k] * ac[b];
-            alpha_tot[asub[s] + a] = v;
+            double t = addK ? alphaK[v * astr + asub[s] + a] : 0.0;
+            for (int b = 0; b < kc; b++) t += Ns[a + (int64_t)b * k] * ac[(int64_t)b * K];
+            alpha_tot[v * astr + asub[s] + a] = t;
         }
     }
 }
@@ -816,27 +651,10 @@ __global__ void __launch_bounds__(256) k_dot_final(const double *partial, int np
     if (threadIdx.x == 0) *out = v;
 }
 
-// p = y + beta p with beta = num/den (first: p = y)
-__global__ void k_p_update(double *p, const double *y, int64_t n, const double *num, const double *den, int first) {
-    const double beta = first ? 0.0 : (*num) / (*den);
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = first ? y[i] : y[i] + beta * p[i];
-}
-// alpha = num/den; x += alpha p; r -= alpha Ap
-__global__ void k_xr_update(double *x, double *r, const double *p, const double *Ap, int64_t n, const double *num,
-                            const double *den) {
-    const double alpha = (*num) / (*den);
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        x[i] += alpha * p[i];
-        r[i] -= alpha * Ap[i];
-    }
-}
 __global__ void k_axpby(double *y, const double *a, const double *b, int64_t n, double alpha, double beta) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         y[i] = alpha * a[i] + beta * b[i];
 }
-__global__ void k_copy_scalar(const double *src, double *dst) { *dst = *src; }
-
 __global__ void k_symmetrize(double *A, int n) {
     const int64_t nn = (int64_t)n * n;
     for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < nn; e += (int64_t)gridDim.x * blockDim.x) {
@@ -874,61 +692,19 @@ void launch_symv(const DualDev &D, bool sd, int prec, const double *x, int gathe
                            D.bl_lam, coef, x, gather, D.ypart);
     }
     if (ev1) (void)hipEventRecord(ev1, st);
-    const int R = strip_rows(prec);
-    hipLaunchKernelGGL(k_part_reduce, dim3(D.nsub), dim3(256), 0, st, items, D.item0[prec], D.nitems[prec], D.m,
-                       D.boff, R, D.ypart, D.yb);
+    launch_part_reduce(D, items, D.item0[prec], D.nitems[prec], strip_rows(prec), 1, D.ypart, D.yb, st);
 }
 
-void launch_symv_mfma(const DualDev &D, const SymvBlock &B, bool sd, int nr, const double *x, bool scaled,
-                      double *yb, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
+void launch_symv_mfma(const DualDev &D, const SymvBlock &B, bool sd, int nr, const double *xb, double *yb,
+                      hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
     if (nr < 1 || nr > 16) throw Error(ESPRESO_ERR_ARG, "block SYMV: 1 to 16 right-hand sides");
-    const double *coef = scaled ? D.bl_sscale : D.bl_sign;
     const double *pool = sd ? D.SD : D.Fd;
     const int64_t *off = sd ? D.sdoff : D.foff;
-    const unsigned gg = (unsigned)std::max<int64_t>(1, std::min<int64_t>(cdiv(D.nbnd * nr, 256), 8192));
-    hipLaunchKernelGGL(k_boundary_gather_multi, dim3(gg), dim3(256), 0, st, D.nbnd, nr, D.bl_ptr, D.bl_lam, coef, x,
-                       (int64_t)D.nlam, B.xb);
     if (ev0) (void)hipEventRecord(ev0, st);
-    hipLaunchKernelGGL(k_symv_mfma, dim3(B.n_items), dim3(256), 0, st, B.items, D.m, D.boff, pool, off, B.xb, nr,
+    hipLaunchKernelGGL(k_symv_mfma, dim3(B.n_items), dim3(256), 0, st, B.items, D.m, D.boff, pool, off, xb, nr,
                        B.ypart);
     if (ev1) (void)hipEventRecord(ev1, st);
-    hipLaunchKernelGGL(k_part_reduce_mfma, dim3(D.nsub), dim3(256), 0, st, B.items, B.item0, B.nitems, D.m, D.boff,
-                       D.nbnd, nr, B.ypart, yb);
-}
-
-void launch_lambda_gather(const DualDev &D, const double *yb, bool scaled, double *y, hipStream_t st) {
-    hipLaunchKernelGGL(k_lambda_gather, dim3(vgrid(D.nlam)), dim3(256), 0, st, D.nlam, D.le_cnt, D.le_b,
-                       scaled ? D.le_sscale : D.le_sign, yb, y);
-}
-
-void launch_boundary_gather(const DualDev &D, const double *x, bool scaled, double *xb, hipStream_t st) {
-    hipLaunchKernelGGL(k_boundary_gather, dim3(vgrid(D.nbnd)), dim3(256), 0, st, D.nbnd, D.bl_ptr, D.bl_lam,
-                       scaled ? D.bl_sscale : D.bl_sign, x, xb);
-}
-
-void launch_kbb(const DualDev &D, const double *xb, double *yb, hipStream_t st) {
-    hipLaunchKernelGGL(k_kbb, dim3(vgrid(D.nbnd)), dim3(256), 0, st, D.nbnd, D.kbb_ptr, D.kbb_col, D.kbb_val, xb, yb);
-}
-
-void launch_project(const DualDev &D, const double *x, double *y, int mode, hipStream_t st) {
-    // mode 0: y = P x;  mode 1: y = G^T GGinv x (x coarse);  mode 2: y = GGinv G x (coarse out)
-    if (mode != 1) {
-        hipLaunchKernelGGL(k_apply_G, dim3(D.nsub), dim3(APPLY_G_THREADS), 0, st, D.m, D.boff, D.ck, D.dsub_off, D.rtoff, D.Rt,
-                           D.bl_ptr, D.bl_lam, D.bl_sign, x, D.dsub);
-        hipLaunchKernelGGL(k_block_sum, dim3(vgrid((int64_t)D.nblk * 64)), dim3(256), 0, st, D.nblk, D.blk_ptr,
-                           D.blk_sub, D.dsub_off, D.ck, D.coff, D.dsub, D.cd);
-    }
-    const double *din = mode == 1 ? x : D.cd;
-    double *eout = mode == 2 ? y : D.ce;
-    hipLaunchKernelGGL(k_coarse_gemv, dim3(D.ncoarse), dim3(256), 0, st, D.ncoarse, D.GGinv, din, eout);
-    if (mode == 2) return;
-    hipLaunchKernelGGL(k_project_finish, dim3(vgrid(D.nlam)), dim3(256), 0, st, D.nlam, D.le_cnt, D.le_b, D.le_sub,
-                       D.le_sign, D.boff, D.m, D.ck, D.cblk, D.coff, D.rtoff, D.Rt, D.ce, x, y, mode);
-}
-
-void launch_subdomain_kernel_dots(const DualDev &D, const double *x, double *out, hipStream_t st) {
-    hipLaunchKernelGGL(k_apply_G, dim3(D.nsub), dim3(APPLY_G_THREADS), 0, st, D.m, D.boff, D.kdim, D.asub, D.rboff, D.Rb,
-                       D.bl_ptr, D.bl_lam, D.bl_sign, x, out);
+    launch_part_reduce(D, B.items, B.item0, B.nitems, STRIP_F64, nr, B.ypart, yb, st);
 }
 
 void launch_cluster_correction(const DualDev &D, const ClusterDev &C, const double *e0s, double *yb, int addR,
@@ -937,7 +713,7 @@ void launch_cluster_correction(const DualDev &D, const ClusterDev &C, const doub
         hipLaunchKernelGGL(k_cluster_t, dim3((C.max_n0 + 31) / 32, C.ncl), dim3(256), (size_t)C.max_n0 * 8, st, C, yb,
                            C.lambda0);
     hipLaunchKernelGGL(k_cluster_alpha, dim3(C.ncl), dim3(1024), 2 * (size_t)std::max(C.max_kt, 1) * 8, st, C, e0s,
-                       C.lambda0, C.alphaK);
+                       C.lambda0, (int64_t)0, C.alphaK, (int64_t)0);
     if (lowp && C.FB0f)
         hipLaunchKernelGGL(k_cluster_apply<float>, dim3((D.max_m + 255) / 256, D.nsub), dim3(256), 0, st, C,
                            (const float *)C.FB0f, D.m, D.boff, D.kdim, D.rboff, D.Rb, C.lambda0, C.alphaK, addR, yb);
@@ -946,33 +722,25 @@ void launch_cluster_correction(const DualDev &D, const ClusterDev &C, const doub
                            (const double *)C.FB0, D.m, D.boff, D.kdim, D.rboff, D.Rb, C.lambda0, C.alphaK, addR, yb);
 }
 
-// t_v = F0^-1 B0 y_b,v for nr cases (case stride ystr in yb, tstr in t)
-void launch_cluster_t_multi(const DualDev &D, const ClusterDev &C, int nr, const double *yb, int64_t ystr, double *t,
-                            int64_t tstr, hipStream_t st) {
-    if (C.max_n0 <= 0) return;
-    const int kc_max = (int)std::max<int64_t>(1, std::min<int64_t>(8, 6144 / C.max_n0));
-    for (int v0 = 0; v0 < nr; v0 += kc_max) {
-        const int kc = std::min(kc_max, nr - v0);
-        hipLaunchKernelGGL(k_cluster_t_multi, dim3((C.max_n0 + 15) / 16, C.ncl), dim3(256),
-                           (size_t)C.max_n0 * kc * 8, st, C, yb + v0 * ystr, ystr, kc, t + v0 * tstr, tstr);
+// the correction of nr interleaved cases: F0^-1 and F_i B0^T read once per 8 cases
+void launch_cluster_correction_multi(const DualDev &D, const ClusterDev &C, int nr, const double *e0s, double *lam0,
+                                     int64_t lstr, double *alphaK, int64_t astr, double *yb, int addR,
+                                     hipStream_t st) {
+    if (C.max_n0 > 0) {
+        const int kc_max = (int)std::max<int64_t>(1, std::min<int64_t>(8, 6144 / C.max_n0));
+        for (int v0 = 0; v0 < nr; v0 += kc_max) {
+            const int kc = std::min(kc_max, nr - v0);
+            hipLaunchKernelGGL(k_cluster_t_multi, dim3((C.max_n0 + 15) / 16, C.ncl), dim3(256),
+                               (size_t)C.max_n0 * kc * 8, st, C, yb + v0, (int64_t)nr, kc, lam0 + v0 * lstr, lstr);
+        }
     }
-    (void)D;
-}
-
-// alpha and lambda0 of one case from its t (in lam0) and e0s
-void launch_cluster_alpha(const ClusterDev &C, const double *e0s, double *lam0, double *alphaK, hipStream_t st) {
-    hipLaunchKernelGGL(k_cluster_alpha, dim3(C.ncl), dim3(1024), 2 * (size_t)std::max(C.max_kt, 1) * 8, st, C, e0s,
-                       lam0, alphaK);
-}
-
-void launch_cluster_apply_multi(const DualDev &D, const ClusterDev &C, int nr, const double *lam0, int64_t lstr,
-                                const double *alphaK, int64_t astr, int addR, double *yb, int64_t ystr,
-                                hipStream_t st) {
+    hipLaunchKernelGGL(k_cluster_alpha, dim3(C.ncl, nr), dim3(1024), 2 * (size_t)std::max(C.max_kt, 1) * 8, st, C, e0s,
+                       lam0, lstr, alphaK, astr);
     for (int v0 = 0; v0 < nr; v0 += 8) {
         const int kc = std::min(8, nr - v0);
         hipLaunchKernelGGL(k_cluster_apply_multi, dim3((D.max_m + 255) / 256, D.nsub), dim3(256), 0, st, C, D.m,
                            D.boff, D.kdim, D.rboff, D.Rb, lam0 + v0 * lstr, lstr, alphaK + v0 * astr, astr, addR, kc,
-                           yb + v0 * ystr, ystr);
+                           yb + v0, (int64_t)nr);
     }
 }
 
@@ -986,10 +754,10 @@ void launch_cluster_setup_sa(const ClusterDev &C, double *Sa, hipStream_t st) {
     hipLaunchKernelGGL(k_cluster_sa, dim3(C.ncl), dim3(256), 0, st, C, Sa);
 }
 
-void launch_alpha_combine(const DualDev &D, const ClusterDev &C, bool hybrid, const double *alpha_coarse,
-                          double *alpha_tot, hipStream_t st) {
-    hipLaunchKernelGGL(k_alpha_combine, dim3(vgrid(D.nsub)), dim3(256), 0, st, D.nsub, D.kdim, D.ck, D.cblk, D.coff,
-                       D.asub, D.noff, D.N, C.alphaK, hybrid ? 1 : 0, alpha_coarse, alpha_tot);
+void launch_alpha_combine(const DualDev &D, int K, const double *alphaK, int64_t astr, bool hybrid,
+                          const double *alpha_coarse, double *alpha_tot, hipStream_t st) {
+    hipLaunchKernelGGL(k_alpha_combine, dim3(vgrid((int64_t)D.nsub * K)), dim3(256), 0, st, D.nsub, K, D.kdim, D.ck,
+                       D.cblk, D.coff, D.asub, D.noff, D.N, alphaK, hybrid ? 1 : 0, alpha_coarse, alpha_tot, astr);
 }
 
 void launch_dot(const double *a, const double *b, int64_t n, double *partial, double *out, hipStream_t st) {
@@ -998,22 +766,8 @@ void launch_dot(const double *a, const double *b, int64_t n, double *partial, do
     hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(256), 0, st, partial, np, out);
 }
 
-void launch_p_update(double *p, const double *y, int64_t n, const double *num, const double *den, int first,
-                     hipStream_t st) {
-    hipLaunchKernelGGL(k_p_update, dim3(vgrid(n)), dim3(256), 0, st, p, y, n, num, den, first);
-}
-
-void launch_xr_update(double *x, double *r, const double *p, const double *Ap, int64_t n, const double *num,
-                      const double *den, hipStream_t st) {
-    hipLaunchKernelGGL(k_xr_update, dim3(vgrid(n)), dim3(256), 0, st, x, r, p, Ap, n, num, den);
-}
-
 void launch_axpby(double *y, const double *a, const double *b, int64_t n, double alpha, double beta, hipStream_t st) {
     hipLaunchKernelGGL(k_axpby, dim3(vgrid(n)), dim3(256), 0, st, y, a, b, n, alpha, beta);
-}
-
-void launch_copy_scalar(const double *src, double *dst, hipStream_t st) {
-    hipLaunchKernelGGL(k_copy_scalar, dim3(1), dim3(1), 0, st, src, dst);
 }
 
 void launch_symmetrize(double *A, int n, hipStream_t st) {
@@ -1163,11 +917,12 @@ __device__ __forceinline__ void band_upper_solve(const double *__restrict__ L, i
 
 // ---- new load vectors (K at once): y_f = L^-1 f_int (kept for the primal
 // recovery) and hf = f_b - K_bi K_ii^-1 f_int, so that (K^+ f)_b = F_i hf.
-// f, hf and yf hold the K vectors at strides fs, hs, ys; z is the interleaved
-// work area (K values per interior row).  One workgroup per subdomain.
+// f and yf hold the K vectors at strides fstr and ystr, hf is interleaved in
+// lines of hk cases; z is the interleaved work area (K values per interior
+// row).  One workgroup per subdomain.
 template <int K>
 __global__ void __launch_bounds__(256) k_rhs_prepare(const PrimalDev P, const double *f, int64_t fstr, double *hf,
-                                                     int64_t hstr, double *yf, int64_t ystr, double *work) {
+                                                     int hk, double *yf, int64_t ystr, double *work) {
     const int s = blockIdx.x;
     const int ni = P.ni[s], m = P.m[s], bw = P.bw[s];
     const int w = bw + 1;
@@ -1198,7 +953,7 @@ __global__ void __launch_bounds__(256) k_rhs_prepare(const PrimalDev P, const do
                 for (int r = 0; r < K; r++) v[r] -= kv[q] * z[(int64_t)pc * K + r];
         }
 #pragma unroll
-        for (int q = 0; q < K; q++) hf[q * hstr + P.boff[s] + j] = v[q];
+        for (int q = 0; q < K; q++) hf[(P.boff[s] + j) * hk + q] = v[q];
     }
 }
 
@@ -1210,7 +965,7 @@ __global__ void __launch_bounds__(256) k_rhs_prepare(const PrimalDev P, const do
 // per row would chain three dependent loads per entry).
 constexpr int PRIMAL_ROWS = 64;
 template <int K>
-__global__ void __launch_bounds__(256) k_primal_kib(const PrimalDev P, const double *ub, int64_t bstr, double *work) {
+__global__ void __launch_bounds__(256) k_primal_kib(const PrimalDev P, const double *ub, int bk, double *work) {
     const int s = blockIdx.y, g = blockIdx.x;
     const int ni = P.ni[s];
     const int *perm = P.perm + P.perm_off[s];
@@ -1218,7 +973,7 @@ __global__ void __launch_bounds__(256) k_primal_kib(const PrimalDev P, const dou
     const int *rp = P.rowptr + P.rp_off[s];
     const int *ci = P.colidx + P.nz_off[s];
     const double *kv = P.vals + P.nz_off[s];
-    const double *ubs = ub + P.boff[s];
+    const double *ubs = ub + P.boff[s] * bk;
     double *z = work + P.work_off[s] * K;
     const int grp = threadIdx.x >> 4, l = threadIdx.x & 15;
 #pragma unroll
@@ -1233,7 +988,7 @@ __global__ void __launch_bounds__(256) k_primal_kib(const PrimalDev P, const dou
             const int pc = iperm[ci[q]];
             if (pc >= ni)
 #pragma unroll
-                for (int t = 0; t < K; t++) v[t] += kv[q] * ubs[t * bstr + pc - ni];
+                for (int t = 0; t < K; t++) v[t] += kv[q] * ubs[(int64_t)(pc - ni) * bk + t];
         }
 #pragma unroll
         for (int t = 0; t < K; t++)
@@ -1251,7 +1006,7 @@ __global__ void __launch_bounds__(256) k_primal_kib(const PrimalDev P, const dou
 
 // then, one workgroup per subdomain, the band solves and the assembly of u
 template <int K>
-__global__ void __launch_bounds__(256) k_primal_interior(const PrimalDev P, const double *ub, int64_t bstr,
+__global__ void __launch_bounds__(256) k_primal_interior(const PrimalDev P, const double *ub, int bk,
                                                          const double *yf, int64_t ystr, const double *alpha,
                                                          int64_t astr, double *u, int64_t ustr, double *work) {
     const int s = blockIdx.x;
@@ -1259,7 +1014,7 @@ __global__ void __launch_bounds__(256) k_primal_interior(const PrimalDev P, cons
     const int w = bw + 1;
     const double *L = P.band + P.band_off[s];
     const int *perm = P.perm + P.perm_off[s];
-    const double *ubs = ub + P.boff[s];
+    const double *ubs = ub + P.boff[s] * bk;
     double *z = work + P.work_off[s] * K;
     __shared__ double Ds[64 * BAND_DL];
     // z = K_ib u_b (k_primal_kib), then z <- y_f - L^-1 z = L^-1 (f_int - K_ib u_b)
@@ -1275,7 +1030,7 @@ __global__ void __launch_bounds__(256) k_primal_interior(const PrimalDev P, cons
 #pragma unroll
         for (int q = 0; q < K; q++) {
             const double *al = alpha + q * astr + P.asub[s];
-            double v = r < ni ? z[(int64_t)r * K + q] : ubs[q * bstr + r - ni];
+            double v = r < ni ? z[(int64_t)r * K + q] : ubs[(int64_t)(r - ni) * bk + q];
             for (int a = 0; a < k; a++) v += R[lr + (int64_t)a * n] * al[a];
             u[q * ustr + P.perm_off[s] + lr] = v;
         }
@@ -1283,21 +1038,21 @@ __global__ void __launch_bounds__(256) k_primal_interior(const PrimalDev P, cons
 }
 
 void launch_rhs_prepare(const PrimalDev &P, int nsub, const double *f, double *hf, hipStream_t st) {
-    hipLaunchKernelGGL(k_rhs_prepare<1>, dim3(nsub), dim3(256), 0, st, P, f, (int64_t)0, hf, (int64_t)0, P.yf,
+    hipLaunchKernelGGL(k_rhs_prepare<1>, dim3(nsub), dim3(256), 0, st, P, f, (int64_t)0, hf, 1, P.yf,
                        (int64_t)0, P.work);
 }
 
 // K vectors in chunks of 16, 8, 4, 2, 1; work holds 16 values per interior row
 void launch_rhs_prepare_multi(const PrimalDev &P, int nsub, int nr, const double *f, int64_t fstr, double *hf,
-                              int64_t hstr, double *yf, int64_t ystr, double *work, hipStream_t st) {
+                              double *yf, int64_t ystr, double *work, hipStream_t st) {
     for (int v0 = 0; v0 < nr;) {
         const int r = nr - v0;
         const int K = r >= 16 ? 16 : r >= 8 ? 8 : r >= 4 ? 4 : r >= 2 ? 2 : 1;
         const double *fv = f + v0 * fstr;
-        double *hv = hf + v0 * hstr, *yv = yf + v0 * ystr;
+        double *hv = hf + v0, *yv = yf + v0 * ystr;
 #define ESP_RHS_CASE(KK)                                                                                          \
     case KK:                                                                                                      \
-        hipLaunchKernelGGL(k_rhs_prepare<KK>, dim3(nsub), dim3(256), 0, st, P, fv, fstr, hv, hstr, yv, ystr, work); \
+        hipLaunchKernelGGL(k_rhs_prepare<KK>, dim3(nsub), dim3(256), 0, st, P, fv, fstr, hv, nr, yv, ystr, work);   \
         break;
         switch (K) { ESP_RHS_CASE(16) ESP_RHS_CASE(8) ESP_RHS_CASE(4) ESP_RHS_CASE(2) ESP_RHS_CASE(1) }
 #undef ESP_RHS_CASE
@@ -1410,65 +1165,30 @@ void launch_gather_values(int64_t n, const int64_t *pos, const double *src, doub
 
 void launch_primal(const PrimalDev &P, int nsub, const double *ub, double *u, hipStream_t st) {
     hipLaunchKernelGGL(k_primal_kib<1>, dim3((P.max_ni + PRIMAL_ROWS - 1) / PRIMAL_ROWS, nsub), dim3(256), 0, st, P,
-                       ub, (int64_t)0, P.work);
-    hipLaunchKernelGGL(k_primal_interior<1>, dim3(nsub), dim3(256), 0, st, P, ub, (int64_t)0, P.yf, (int64_t)0,
+                       ub, 1, P.work);
+    hipLaunchKernelGGL(k_primal_interior<1>, dim3(nsub), dim3(256), 0, st, P, ub, 1, P.yf, (int64_t)0,
                        P.alpha, (int64_t)0, u, (int64_t)0, P.work);
 }
 
-void launch_primal_multi(const PrimalDev &P, int nsub, int nr, const double *ub, int64_t bstr, const double *yf,
-                         int64_t ystr, const double *alpha, int64_t astr, double *u, int64_t ustr, double *work,
+void launch_primal_multi(const PrimalDev &P, int nsub, int nr, const double *ub, const double *yf, int64_t ystr,
+                         const double *alpha, int64_t astr, double *u, int64_t ustr, double *work,
                          hipStream_t st) {
     for (int v0 = 0; v0 < nr;) {
         const int r = nr - v0;
         const int K = r >= 16 ? 16 : r >= 8 ? 8 : r >= 4 ? 4 : r >= 2 ? 2 : 1;
-        const double *bv = ub + v0 * bstr, *yv = yf + v0 * ystr, *av = alpha + v0 * astr;
+        const double *bv = ub + v0, *yv = yf + v0 * ystr, *av = alpha + v0 * astr;
         double *uv = u + v0 * ustr;
 #define ESP_PRIMAL_CASE(KK)                                                                                        \
     case KK:                                                                                                       \
         hipLaunchKernelGGL(k_primal_kib<KK>, dim3((P.max_ni + PRIMAL_ROWS - 1) / PRIMAL_ROWS, nsub), dim3(256), 0,  \
-                           st, P, bv, bstr, work);                                                                 \
-        hipLaunchKernelGGL(k_primal_interior<KK>, dim3(nsub), dim3(256), 0, st, P, bv, bstr, yv, ystr, av, astr, uv, \
+                           st, P, bv, nr, work);                                                                   \
+        hipLaunchKernelGGL(k_primal_interior<KK>, dim3(nsub), dim3(256), 0, st, P, bv, nr, yv, ystr, av, astr, uv,   \
                            ustr, work);                                                                            \
         break;
         switch (K) { ESP_PRIMAL_CASE(16) ESP_PRIMAL_CASE(8) ESP_PRIMAL_CASE(4) ESP_PRIMAL_CASE(2) ESP_PRIMAL_CASE(1) }
 #undef ESP_PRIMAL_CASE
         v0 += K;
     }
-}
-
-// ---- SUPER_DIRICHLET preconditioner (clustercpu.cpp:243-314) ----
-// S = K_bb - K_bi diag(K_ii)^-1 K_ib applied from the sparse blocks: first
-// t = diag(K_nn)^-1 K_nb x_b for the interior DOFs next to the boundary,
-// then y_b = K_bb x_b - K_bn t.
-__global__ void k_superdir_near(int64_t n_near, const int64_t *ptr, const int64_t *col, const double *val,
-                                const double *diag, const double *xb, double *t) {
-    for (int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g < n_near; g += (int64_t)gridDim.x * blockDim.x) {
-        double v = 0.0;
-        for (int64_t q = ptr[g]; q < ptr[g + 1]; q++) v += val[q] * xb[col[q]];
-        t[g] = v / diag[g];
-    }
-}
-
-__global__ void k_superdir_bnd(int64_t nb, const int64_t *kptr, const int64_t *kcol, const double *kval,
-                               const int64_t *ptr, const int64_t *col, const double *val, const double *xb,
-                               const double *t, double *yb) {
-    for (int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < nb; j += (int64_t)gridDim.x * blockDim.x) {
-        double v = 0.0;
-        for (int64_t q = kptr[j]; q < kptr[j + 1]; q++) v += kval[q] * xb[kcol[q]];
-        double w = 0.0;
-        for (int64_t q = ptr[j]; q < ptr[j + 1]; q++) w += val[q] * t[col[q]];
-        yb[j] = v - w;
-    }
-}
-
-void launch_superdir(const DualDev &D, int64_t n_near, const int64_t *sib_ptr, const int64_t *sib_col,
-                     const double *sib_val, const double *sdiag, const int64_t *sbi_ptr, const int64_t *sbi_col,
-                     const double *sbi_val, double *t, const double *xb, double *yb, hipStream_t st) {
-    if (n_near > 0)
-        hipLaunchKernelGGL(k_superdir_near, dim3(vgrid(n_near)), dim3(256), 0, st, n_near, sib_ptr, sib_col, sib_val,
-                           sdiag, xb, t);
-    hipLaunchKernelGGL(k_superdir_bnd, dim3(vgrid(D.nbnd)), dim3(256), 0, st, D.nbnd, D.kbb_ptr, D.kbb_col, D.kbb_val,
-                       sbi_ptr, sbi_col, sbi_val, xb, t, yb);
 }
 
 // ---- KKT report (itersolver.cpp:199-251) ----

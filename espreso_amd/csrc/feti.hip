@@ -336,6 +336,35 @@ PinnedPool &pinned_pool() {
     return p;
 }
 
+// PCG records (pinned, one per instance with loaded inputs), kept for the
+// process and lent to the instances: pinning and unpinning a page costs more
+// than a small solve.  As many as instances were alive at once.
+struct RecordPool {
+    std::mutex mu;
+    std::vector<PcgRecord *> idle;
+    PcgRecord *acquire() {
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            if (!idle.empty()) {
+                PcgRecord *r = idle.back();
+                idle.pop_back();
+                return r;
+            }
+        }
+        void *p = nullptr;
+        ESP_HIP(hipHostMalloc(&p, sizeof(PcgRecord), hipHostMallocPortable));
+        return (PcgRecord *)p;
+    }
+    void give_back(PcgRecord *r) {
+        std::lock_guard<std::mutex> lock(mu);
+        idle.push_back(r);
+    }
+};
+RecordPool &record_pool() {
+    static RecordPool p;
+    return p;
+}
+
 struct espreso_feti_s {
     espreso_feti_options opt{};
     int nsub = 0, nlam = -1, ncoarse = 0;
@@ -371,7 +400,9 @@ struct espreso_feti_s {
     double *d_hf = nullptr, *d_ubf = nullptr, *d_fb = nullptr;  // boundary arrays
     double *d_x = nullptr, *d_r = nullptr, *d_w = nullptr, *d_y = nullptr, *d_z = nullptr, *d_p = nullptr,
            *d_Ap = nullptr, *d_b = nullptr, *d_tmp = nullptr, *d_r2 = nullptr, *d_partial = nullptr,
-           *d_scal = nullptr;
+           *d_scal = nullptr;  // PCG scalars of one case, then PCG_SLOTS of scratch
+    double *d_dots = nullptr;  // partial dot products of the PCG: 3 x dot_blocks
+    PcgRecord *rec = nullptr;  // what the running PCG reports (pinned host memory)
     double *d_u = nullptr;    // per-subdomain primal (local order), sum n
     double *d_f = nullptr, *d_Qm = nullptr, *d_GGt = nullptr, *d_c = nullptr;  // resident inputs
     std::vector<int64_t> h_poff[3], h_boff;
@@ -475,8 +506,6 @@ struct espreso_feti_s {
         if (asm_pool || !cached_allocs.empty()) {
             if (st) (void)hipStreamSynchronize(st);
             if (asm_st) (void)hipStreamSynchronize(asm_st);
-            for (Lane &l : lanes)
-                if (l.s) (void)hipStreamSynchronize(l.s);
         }
         if (asm_pool) {
             workspace_cache().give_back(opt.device, asm_pool);
@@ -485,11 +514,6 @@ struct espreso_feti_s {
         for (void *p : cached_allocs) workspace_cache().give_back(opt.device, p);
         cached_allocs.clear();
         drop_graphs();
-        for (Lane &l : lanes) {
-            if (l.ev) (void)hipEventDestroy(l.ev);
-            if (l.s) (void)hipStreamDestroy(l.s);
-        }
-        if (ev_main) (void)hipEventDestroy(ev_main);
         if (ev_fork) (void)hipEventDestroy(ev_fork);
         if (ev_join) (void)hipEventDestroy(ev_join);
         for (hipEvent_t e : asm_ev)
@@ -500,6 +524,7 @@ struct espreso_feti_s {
             (void)hipStreamSynchronize(st);
             (void)hipStreamDestroy(st);
         }
+        if (rec) record_pool().give_back(rec);  // its writers have finished
     }
     // Device memory comes from the device's stream-ordered pool, which keeps
     // what instances free for the next ones of the process (like a caching
@@ -680,12 +705,25 @@ struct espreso_feti_s {
         return upload(v);
     }
     void cluster_setup();
-    void pcg_step(double *x, double *r, int prec, bool first);
-    void pcg_step_graph(double *x, double *r, int prec);
+    // the vectors of a PCG over K interleaved cases; block: the block operators
+    // (MFMA SYMV, FP64 storage) and the block scratch, else the single solve
+    struct PcgVec {
+        int K;
+        bool block;
+        double *x, *r, *w, *z, *y, *p, *Ap, *scal, *dots;
+        DualDev E;  // operators with the coarse scratch of the K cases
+    };
+    PcgVec single_vec(double *x, double *r);
+    PcgVec block_vec(int K);
+    void pcg_step(const PcgVec &V, int prec, bool first);
+    void pcg_step_graph(const PcgVec &V, int prec);
+    void pcg_start(const PcgVec &V, const double *b, double tol_abs);
+    void pcg_loop(const PcgVec &V, int prec);
+    void wait_record(int count);
     void drop_graphs();
     struct StepGraph {
         double *x, *r;
-        int prec;
+        int K, prec;
         hipGraphExec_t exec;
     };
     std::vector<StepGraph> step_graphs;
@@ -703,24 +741,12 @@ struct espreso_feti_s {
         double *x = nullptr, *r = nullptr, *w = nullptr, *z = nullptr, *y = nullptr, *p = nullptr, *Ap = nullptr,
                *b = nullptr, *e = nullptr, *alpha_c = nullptr, *alpha_tot = nullptr, *e0f = nullptr, *hf = nullptr,
                *ubf = nullptr, *xbv = nullptr, *yb = nullptr, *f = nullptr, *yf = nullptr, *u = nullptr,
-               *scal = nullptr, *work = nullptr, *e0s = nullptr, *lam0 = nullptr, *alphaK = nullptr;
+               *scal = nullptr, *work = nullptr, *e0s = nullptr, *lam0 = nullptr, *alphaK = nullptr, *dsub = nullptr,
+               *cd = nullptr, *ce = nullptr, *dots = nullptr, *snear = nullptr;
     } BB;
     SymvBlock SB;
     int64_t nyf = 0;  // interior DOFs (length of P.yf)
-    int64_t n_dsub = 1, n_lambda0 = 1, n_e0s = 1;  // scratch sizes (per-case lanes)
-    // per-case work of a block runs on NLANE streams (default priority), each
-    // with its own copies of the scratch the projector, the cluster correction
-    // and the dot products use
-    static constexpr int NLANE = 4;
-    struct Lane {
-        hipStream_t s = nullptr;
-        hipEvent_t ev = nullptr;
-        double *dsub = nullptr, *cd = nullptr, *ce = nullptr, *lambda0 = nullptr, *alphaK = nullptr,
-               *e0s = nullptr, *partial = nullptr;
-        DualDev D;
-        ClusterDev C;
-    } lanes[NLANE];
-    hipEvent_t ev_main = nullptr;
+    int64_t n_dsub = 1, n_lambda0 = 1, n_e0s = 1;  // scratch sizes per case
     // assembly kernels that only read what an earlier step wrote run on asm_st
     // beside the main stream's work: fork (asm_st behind st) and join (st
     // behind asm_st)
@@ -741,22 +767,8 @@ struct espreso_feti_s {
     hipStream_t asm_st = nullptr;
     std::vector<hipEvent_t> asm_ev;
     void factor_solve(const DenseDesc *desc, int nb, int which, int nt, int band, int ntc);
-    bool lanes_ready = false;
-    void lanes_setup();
-    void fork_lanes();
-    void join_lanes();
     void block_setup(int K);
-    void apply_F_block(int K, const double *x, double *y);
-    void cluster_block(int K, const double *x);
-    void step_block(int K, const std::vector<char> &active, bool first);
-    // iterations with every case of a group active replay a HIP graph of
-    // step_block (the lanes are forked and joined inside the graph)
-    struct BlockGraph {
-        int K;
-        hipGraphExec_t exec;
-    };
-    std::vector<BlockGraph> block_graphs;
-    void step_block_graph(int K);
+    void apply_F_block(const PcgVec &V, const double *x, double *y, bool dot);
     bool resolve_block(int nrhs, const double *f, double *u, int32_t *iters, double *norms,
                        espreso_feti_stats *stats);
     void resolve_group(int K, const double *f, double *u, int32_t *iters, double *norms, espreso_feti_stats &tot);
@@ -788,8 +800,9 @@ struct espreso_feti_s {
     void upload_items(int prec, int64_t target);
     void tune_symv();
     // dual operators on device vectors
-    void apply_F(const double *x, double *y, int prec);
+    void apply_F(const double *x, double *y, int prec, const double *dot_with = nullptr, double *part = nullptr);
     void apply_prec(const double *x, double *y);
+    void apply_prec(const DualDev &E, int K, bool block, const double *x, double *y);
     void solve(espreso_feti_stats *st_out);
     void pcg(const double *b, double *x, double *r, int prec, int &iters, double &norm, double &tol, bool quiet_tol,
              double tol_abs, double *norm_b = nullptr);
@@ -1274,6 +1287,9 @@ void espreso_feti_s::load() {
     D.bl_lam = upload(bl_lam);
     D.bl_sign = upload(bl_sign);
     D.bl_sscale = upload(bl_ss);
+    D.nle = nle;
+    D.bl_row = alloc<int>(nle);
+    launch_entry_rows(nb, D.bl_ptr, D.bl_row, st);
     D.le_cnt = upload(le_cnt);
     D.le_b = upload(le_b);
     D.le_sub = upload(le_sub);
@@ -1298,6 +1314,8 @@ void espreso_feti_s::load() {
         d_snear = alloc<double>(n_near);
     }
     D.Rb = upload(Rb);
+    D.RbT = alloc<double>(rboff[nsub]);
+    launch_basis_rows(nsub, max_m, D.m, D.kdim, D.rboff, D.Rb, D.RbT, st);
     D.yb = alloc<double>(nb);
     D.xb = alloc<double>(nb);
 
@@ -1407,6 +1425,8 @@ void espreso_feti_s::load() {
     note("load: upload", t0);
     if (hybrid) load_clusters();
     else coarse_layout_subdomains();
+    D.le_coarse = alloc<LamCoarse>(2 * (size_t)nlam);
+    launch_lambda_coarse(D, D.le_coarse, st);
     note("load: coarse space, GG^T", t0);
 
     // ---- SYMV work lists (the item size is tuned at the first set-up) ----
@@ -1436,7 +1456,9 @@ void espreso_feti_s::load() {
     d_tmp = alloc<double>(nlam);
     d_r2 = alloc<double>(nlam);
     d_partial = alloc<double>(1024);
-    d_scal = alloc<double>(16);
+    d_scal = alloc<double>(2 * PCG_SLOTS);
+    d_dots = alloc<double>(3 * (size_t)dot_blocks(nlam, 1));
+    rec = record_pool().acquire();
     d_c = upload(c);
     for (int s = 0; s < nsub; s++) kkt_max_n = std::max(kkt_max_n, sub[s].n);
     d_kkt = alloc<double>(2 * nb + nlam + 2 * (int64_t)nsub + 8 + 2 * (int64_t)nsub * kkt_groups(kkt_max_n));
@@ -1537,7 +1559,7 @@ void espreso_feti_s::compute_b_into(const double *hf, double *ubf, const double 
     launch_symv(D, false, 0, hf, 0, false, st);
     ESP_HIP(hipMemcpyAsync(ubf, D.yb, D.nbnd * sizeof(double), hipMemcpyDeviceToDevice, st));
     if (hybrid) launch_cluster_correction(D, CL, e0f, D.yb, 1, st);
-    launch_lambda_gather(D, D.yb, false, b, st);
+    launch_lambda_gather(D, 1, D.yb, false, b, st);
     launch_axpby(b, b, d_c, nlam, 1.0, -1.0, st);
 }
 
@@ -2021,88 +2043,103 @@ void espreso_feti_s::tune_symv() {
 }
 
 // ------------------------------------------------------ dual operators ----
-void espreso_feti_s::apply_F(const double *x, double *y, int prec) {
+void espreso_feti_s::apply_F(const double *x, double *y, int prec, const double *dot_with, double *part) {
     launch_symv(D, false, prec, x, 1, false, st);
     if (hybrid) {
         // K~^+ = K^+ - K^+ B0^T lambda0 + R alpha (cluster.cpp:796-916), e0 = -R^T B^T x
-        launch_subdomain_kernel_dots(D, x, d_e0s, st);
+        launch_subdomain_kernel_dots(D, 1, x, d_e0s, st);
         launch_cluster_correction(D, CL, d_e0s, D.yb, 1, st, prec != 0);
     }
-    launch_lambda_gather(D, D.yb, false, y, st);
+    launch_lambda_gather(D, 1, D.yb, false, y, st, dot_with, part);
 }
 
-void espreso_feti_s::apply_prec(const double *x, double *y) {
+void espreso_feti_s::apply_prec(const double *x, double *y) { apply_prec(D, 1, false, x, y); }
+
+// K interleaved cases; block: with the block scratch and the block SYMV
+void espreso_feti_s::apply_prec(const DualDev &E, int K, bool block, const double *x, double *y) {
+    double *xb = block ? SB.xb : D.xb, *yb = block ? BB.yb : D.yb;
     switch (opt.preconditioner) {
     case ESPRESO_PREC_NONE:
-        ESP_HIP(hipMemcpyAsync(y, x, nlam * sizeof(double), hipMemcpyDeviceToDevice, st));
+        ESP_HIP(hipMemcpyAsync(y, x, (size_t)K * nlam * sizeof(double), hipMemcpyDeviceToDevice, st));
         break;
     case ESPRESO_PREC_LUMPED:
-        launch_boundary_gather(D, x, true, D.xb, st);
-        launch_kbb(D, D.xb, D.yb, st);
-        launch_lambda_gather(D, D.yb, true, y, st);
+        launch_boundary_gather(E, K, x, true, xb, st);
+        launch_kbb(E, K, xb, yb, st);
+        launch_lambda_gather(E, K, yb, true, y, st);
         break;
     case ESPRESO_PREC_WEIGHT:
-        launch_boundary_gather(D, x, true, D.xb, st);
-        launch_lambda_gather(D, D.xb, true, y, st);
+        launch_boundary_gather(E, K, x, true, xb, st);
+        launch_lambda_gather(E, K, xb, true, y, st);
         break;
     case ESPRESO_PREC_DIRICHLET:
-        launch_symv(D, true, 0, x, 1, true, st);
-        launch_lambda_gather(D, D.yb, true, y, st);
+        if (block) {
+            launch_boundary_gather(E, K, x, true, xb, st);
+            launch_symv_mfma(E, SB, true, K, xb, yb, st);
+        } else {
+            launch_symv(D, true, 0, x, 1, true, st);
+        }
+        launch_lambda_gather(E, K, yb, true, y, st);
         break;
     case ESPRESO_PREC_SUPER_DIRICHLET:
-        launch_boundary_gather(D, x, true, D.xb, st);
-        launch_superdir(D, n_near, d_sib_ptr, d_sib_col, d_sib_val, d_sdiag, d_sbi_ptr, d_sbi_col, d_sbi_val, d_snear,
-                        D.xb, D.yb, st);
-        launch_lambda_gather(D, D.yb, true, y, st);
+        launch_boundary_gather(E, K, x, true, xb, st);
+        launch_superdir(E, K, n_near, d_sib_ptr, d_sib_col, d_sib_val, d_sdiag, d_sbi_ptr, d_sbi_col, d_sbi_val,
+                        block ? BB.snear : d_snear, xb, yb, st);
+        launch_lambda_gather(E, K, yb, true, y, st);
         break;
     default:
         throw Error(ESPRESO_ERR_ARG, "unknown preconditioner");
     }
 }
 
-// Projected PCG (itersolver.cpp:1537-1684) on device vectors.  r holds the
-// initial residual on entry.  Scalars stay on the device; the host reads
-// ||w|| once per iteration for the stop test.
+// Projected PCG (itersolver.cpp:1537-1684) on K interleaved device vectors, each
+// case with its own scalars and stop test.  The scalars stay on the device; the
+// kernel that finishes ||w||^2 reports it to pinned memory (PcgRecord) in the
+// middle of the iteration, so the host decides on the next iteration while the
+// dual operator of this one runs.
+espreso_feti_s::PcgVec espreso_feti_s::single_vec(double *x, double *r) {
+    return PcgVec{1, false, x, r, d_w, d_z, d_y, d_p, d_Ap, d_scal, d_dots, D};
+}
+
 // One iteration of Solve_RegCG (itersolver.cpp:1537-1684) as a launch sequence:
-// w = P r, y = P M w, beta, p, Ap = F p, alpha, x, r, ||w||^2.
-void espreso_feti_s::pcg_step(double *x, double *r, int prec, bool first) {
-    double *s_yw = d_scal + 0, *s_yw_prev = d_scal + 1, *s_pAp = d_scal + 2, *s_ww = d_scal + 3;
-    launch_project(D, r, d_w, 0, st);
+// w = P r, y = P M w, beta, p, Ap = F p, alpha, x, r.  The dot products are
+// summed by the passes that produce w, y and Ap.
+void espreso_feti_s::pcg_step(const PcgVec &V, int prec, bool first) {
+    const int K = V.K, np = dot_blocks(nlam, K);
+    double *ww = V.dots, *yw = V.dots + (size_t)np * K, *pAp = V.dots + 2 * (size_t)np * K;
+    launch_project(V.E, K, V.r, V.w, 0, st, nullptr, ww, V.scal);
     if (opt.preconditioner == ESPRESO_PREC_NONE) {
-        ESP_HIP(hipMemcpyAsync(d_y, d_w, nlam * sizeof(double), hipMemcpyDeviceToDevice, st));
+        ESP_HIP(hipMemcpyAsync(V.y, V.w, (size_t)K * nlam * sizeof(double), hipMemcpyDeviceToDevice, st));
+        launch_dot_lines(nlam, K, V.y, V.w, yw, st);
     } else {
-        apply_prec(d_w, d_z);
-        launch_project(D, d_z, d_y, 0, st);
+        apply_prec(V.E, K, V.block, V.w, V.z);
+        launch_project(V.E, K, V.z, V.y, 0, st, V.w, yw);
     }
-    if (!first) launch_copy_scalar(s_yw, s_yw_prev, st);
-    launch_dot(d_y, d_w, nlam, d_partial, s_yw, st);
-    launch_p_update(d_p, d_y, nlam, s_yw, s_yw_prev, first, st);
-    apply_F(d_p, d_Ap, prec);
-    launch_dot(d_p, d_Ap, nlam, d_partial, s_pAp, st);
-    launch_xr_update(x, r, d_p, d_Ap, nlam, s_yw, s_pAp, st);
-    launch_dot(d_w, d_w, nlam, d_partial, s_ww, st);
+    launch_p_update(nlam, K, V.p, V.y, yw, ww, np, first, V.scal, rec, st);
+    if (V.block) apply_F_block(V, V.p, V.Ap, true);
+    else apply_F(V.p, V.Ap, prec, V.p, pAp);
+    launch_xr_update(nlam, K, V.x, V.r, V.p, V.Ap, pAp, np, V.scal, st);
 }
 
 // iterations after the first replay a HIP graph of pcg_step, captured once
-// per (x, r, storage precision); graphs hold device pointers of the current
-// set-up and are dropped when the set-up is redone
-void espreso_feti_s::pcg_step_graph(double *x, double *r, int prec) {
+// per (x, r, cases, storage precision); graphs hold device pointers of the
+// current set-up and are dropped when the set-up is redone
+void espreso_feti_s::pcg_step_graph(const PcgVec &V, int prec) {
     for (const StepGraph &g : step_graphs)
-        if (g.x == x && g.r == r && g.prec == prec) {
+        if (g.x == V.x && g.r == V.r && g.K == V.K && g.prec == prec) {
             ESP_HIP(hipGraphLaunch(g.exec, st));
             return;
         }
     hipGraph_t graph = nullptr;
     ESP_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
     try {
-        pcg_step(x, r, prec, false);
+        pcg_step(V, prec, false);
     } catch (...) {
         (void)hipStreamEndCapture(st, &graph);
         if (graph) (void)hipGraphDestroy(graph);
         throw;
     }
     ESP_HIP(hipStreamEndCapture(st, &graph));
-    StepGraph g{x, r, prec, nullptr};
+    StepGraph g{V.x, V.r, V.K, prec, nullptr};
     const hipError_t e = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     ESP_HIP(e);
@@ -2114,43 +2151,60 @@ void espreso_feti_s::drop_graphs() {
     for (StepGraph &g : step_graphs)
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
     step_graphs.clear();
-    for (BlockGraph &g : block_graphs)
-        if (g.exec) (void)hipGraphExecDestroy(g.exec);
-    block_graphs.clear();
+}
+
+// tol = precision * min(||P r0||, ||b||) per case (tol_abs > 0: that), flags cleared
+void espreso_feti_s::pcg_start(const PcgVec &V, const double *b, double tol_abs) {
+    const int np = dot_blocks(nlam, V.K);
+    launch_project(V.E, V.K, V.r, V.w, 0, st, nullptr, V.dots);
+    launch_dot_lines(nlam, V.K, b, b, V.dots + (size_t)np * V.K, st);
+    rec->count = 0;  // no kernel of an earlier PCG is left that writes the record
+    rec->active = 1;
+    launch_pcg_init(V.K, V.dots, V.dots + (size_t)np * V.K, np, opt.precision, tol_abs, V.scal, rec, st);
+}
+
+// waits until the record holds the stop test of iteration `count` (1-based)
+void espreso_feti_s::wait_record(int count) {
+    for (unsigned n = 0; __atomic_load_n(&rec->count, __ATOMIC_ACQUIRE) < count; n++) {
+        if (n % 1024 != 1023) continue;
+        const hipError_t e = hipStreamQuery(st);
+        if (e == hipErrorNotReady) continue;
+        ESP_HIP(e);
+        // the stream has drained: the record is final
+        ESP_CHECK(__atomic_load_n(&rec->count, __ATOMIC_ACQUIRE) >= count, ESPRESO_ERR_HIP,
+                  "PCG iteration ended without its stop test");
+    }
+}
+
+// iterates until every case meets its stop test (rec: norms and iterations per case)
+void espreso_feti_s::pcg_loop(const PcgVec &V, int prec) {
+    for (int it = 0; it < opt.max_iterations; it++) {
+        if (it == 0 || !use_graphs) pcg_step(V, prec, it == 0);
+        else pcg_step_graph(V, prec);
+        wait_record(it + 1);
+        for (int v = 0; v < V.K; v++)
+            ESP_CHECK(std::isfinite(rec->ww[v]), ESPRESO_ERR_NUMERIC,
+                      V.block ? "block PCG produced a non-finite residual" : "PCG produced a non-finite residual");
+        if (!rec->active) break;
+    }
 }
 
 void espreso_feti_s::pcg(const double *b, double *x, double *r, int prec, int &iters, double &norm, double &tol,
                          bool use_abs, double tol_abs, double *norm_b) {
-    double *s_ww = d_scal + 3, *s_tmp = d_scal + 4;
-    // tol = precision * min(||P r0||, ||b||)
-    launch_project(D, r, d_w, 0, st);
-    launch_dot(d_w, d_w, nlam, d_partial, s_tmp, st);
-    launch_dot(b, b, nlam, d_partial, s_tmp + 1, st);
-    double hv[2];
-    ESP_HIP(hipMemcpyAsync(hv, s_tmp, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
-    sync();
-    tol = use_abs ? tol_abs : opt.precision * std::min(std::sqrt(hv[0]), std::sqrt(hv[1]));
-    if (norm_b) *norm_b = std::sqrt(hv[1]);
-    iters = 0;
-    norm = 0;
-    for (int it = 0; it < opt.max_iterations; it++) {
-        if (it == 0 || !use_graphs) pcg_step(x, r, prec, it == 0);
-        else pcg_step_graph(x, r, prec);
-        double ww = 0;
-        ESP_HIP(hipMemcpyAsync(&ww, s_ww, sizeof(double), hipMemcpyDeviceToHost, st));
-        sync();
-        ESP_CHECK(std::isfinite(ww), ESPRESO_ERR_NUMERIC, "PCG produced a non-finite residual");
-        norm = std::sqrt(ww);
-        iters = it + 1;
-        if (norm < tol) break;
-    }
+    const PcgVec V = single_vec(x, r);
+    pcg_start(V, b, use_abs ? tol_abs : 0.0);
+    pcg_loop(V, prec);
+    tol = rec->tol[0];
+    if (norm_b) *norm_b = std::sqrt(rec->bb[0]);
+    iters = rec->iters[0];
+    norm = std::sqrt(rec->ww[0]);
 }
 
 void espreso_feti_s::solve(espreso_feti_stats *out) {
     ESP_CHECK(ready, ESPRESO_ERR_STATE, "espreso_feti_setup not called");
     double t0 = wall();
     // lambda0 = G^T (GG^T)^-1 e ; r = b - F lambda0
-    launch_project(D, d_e, d_x, 1, st);
+    launch_project(D, 1, d_e, d_x, 1, st);
     apply_F(d_x, d_Ap, 0);
     launch_axpby(d_r, d_b, d_Ap, nlam, 1.0, -1.0, st);
     int iters = 0;
@@ -2164,11 +2218,11 @@ void espreso_feti_s::solve(espreso_feti_stats *out) {
     } else {
         // mixed precision: inner PCG on the low-precision F_i, outer FP64
         // residual r = b - F lambda with the FP64 F_i (iterative refinement)
-        launch_project(D, d_r, d_w, 0, st);
-        launch_dot(d_w, d_w, nlam, d_partial, d_scal + 4, st);
-        launch_dot(d_b, d_b, nlam, d_partial, d_scal + 5, st);
+        launch_project(D, 1, d_r, d_w, 0, st);
+        launch_dot(d_w, d_w, nlam, d_partial, d_scal + PCG_SLOTS, st);
+        launch_dot(d_b, d_b, nlam, d_partial, d_scal + PCG_SLOTS + 1, st);
         double hv[2];
-        ESP_HIP(hipMemcpyAsync(hv, d_scal + 4, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
+        ESP_HIP(hipMemcpyAsync(hv, d_scal + PCG_SLOTS, 2 * sizeof(double), hipMemcpyDeviceToHost, st));
         sync();
         const double tol64 = opt.precision * std::min(std::sqrt(hv[0]), std::sqrt(hv[1]));
         last.norm_b = std::sqrt(hv[1]);
@@ -2182,10 +2236,10 @@ void espreso_feti_s::solve(espreso_feti_stats *out) {
             int it = 0;
             double nn = 0, tt = 0;
             // inner tolerance: relative 1e-5 of the current projected residual, floor tol64
-            launch_project(D, d_r, d_w, 0, st);
-            launch_dot(d_w, d_w, nlam, d_partial, d_scal + 6, st);
+            launch_project(D, 1, d_r, d_w, 0, st);
+            launch_dot(d_w, d_w, nlam, d_partial, d_scal + PCG_SLOTS + 2, st);
             double cur = 0;
-            ESP_HIP(hipMemcpyAsync(&cur, d_scal + 6, sizeof(double), hipMemcpyDeviceToHost, st));
+            ESP_HIP(hipMemcpyAsync(&cur, d_scal + PCG_SLOTS + 2, sizeof(double), hipMemcpyDeviceToHost, st));
             sync();
             cur = std::sqrt(cur);
             if (cur < tol64) break;
@@ -2195,10 +2249,10 @@ void espreso_feti_s::solve(espreso_feti_stats *out) {
             apply_F(d_x, d_Ap, 0);
             launch_axpby(d_r, d_b, d_Ap, nlam, 1.0, -1.0, st);
         }
-        launch_project(D, d_r, d_w, 0, st);
-        launch_dot(d_w, d_w, nlam, d_partial, d_scal + 6, st);
+        launch_project(D, 1, d_r, d_w, 0, st);
+        launch_dot(d_w, d_w, nlam, d_partial, d_scal + PCG_SLOTS + 2, st);
         double fin = 0;
-        ESP_HIP(hipMemcpyAsync(&fin, d_scal + 6, sizeof(double), hipMemcpyDeviceToHost, st));
+        ESP_HIP(hipMemcpyAsync(&fin, d_scal + PCG_SLOTS + 2, sizeof(double), hipMemcpyDeviceToHost, st));
         sync();
         iters = total;
         norm = std::sqrt(fin);
@@ -2209,17 +2263,17 @@ void espreso_feti_s::solve(espreso_feti_stats *out) {
     double tp = wall();
     last.time_pcg = tp - t0;
     // amplitudes alpha = (GG^T)^-1 G r ; primal u = K~^+ (f - B^T lambda) + R alpha
-    launch_project(D, d_r, d_alpha_c, 2, st);
+    launch_project(D, 1, d_r, d_alpha_c, 2, st);
     // u_b = K^+ f|_b - F_i B^T lambda
     launch_symv(D, false, 0, d_x, 1, false, st);
     launch_axpby(D.xb, d_ubf, D.yb, D.nbnd, 1.0, -1.0, st);
     if (hybrid) {
         // e0 = -R^T (f - B^T lambda) = e0f - (-R^T B^T lambda)
-        launch_subdomain_kernel_dots(D, d_x, d_e0s, st);
+        launch_subdomain_kernel_dots(D, 1, d_x, d_e0s, st);
         launch_axpby(d_e0s, d_e0f, d_e0s, asubv[nsub], 1.0, -1.0, st);
         launch_cluster_correction(D, CL, d_e0s, D.xb, 0, st);
     }
-    launch_alpha_combine(D, CL, hybrid, d_alpha_c, d_alpha_tot, st);
+    launch_alpha_combine(D, 1, CL.alphaK, 0, hybrid, d_alpha_c, d_alpha_tot, st);
     launch_primal(P, nsub, D.xb, d_u, st);
     // KKT report of the solution (GetSolution_Primal_singular_parallel, itersolver.cpp:171-370)
     kkt(d_x, last);
@@ -2254,14 +2308,14 @@ void espreso_feti_s::kkt(const double *lambda, espreso_feti_stats &s) {
     const int64_t nb = D.nbnd;
     double *bt1 = d_kkt, *bt0 = d_kkt + nb, *yl = d_kkt + 2 * nb, *sums = d_kkt + 2 * nb + nlam;
     double *ub = D.yb;  // boundary values of u (scratch)
-    launch_boundary_gather(D, lambda, false, bt1, st);
+    launch_boundary_gather(D, 1, lambda, false, bt1, st);
     if (hybrid) {
         ESP_HIP(hipMemsetAsync(bt0, 0, nb * sizeof(double), st));
         launch_b0t(D, CL, bt0, st);
     }
     double *part = d_kkt + 2 * nb + nlam + 2 * (int64_t)nsub + 8;
     launch_kkt_primal(P, nsub, kkt_max_n, d_u, d_f, bt1, hybrid ? bt0 : nullptr, ub, part, sums, st);
-    launch_lambda_gather(D, ub, false, yl, st);
+    launch_lambda_gather(D, 1, ub, false, yl, st);
     launch_axpby(yl, yl, d_c, nlam, 1.0, -1.0, st);
     launch_dot(yl, yl, nlam, d_partial, sums + 2 * nsub, st);
     launch_dot(d_c, d_c, nlam, d_partial, sums + 2 * nsub + 1, st);
@@ -2321,7 +2375,7 @@ void espreso_feti_s::block_setup(int K) {
     drop_graphs();  // graphs hold the group's buffers
     for (double *q : {BB.x, BB.r, BB.w, BB.z, BB.y, BB.p, BB.Ap, BB.b, BB.e, BB.alpha_c, BB.alpha_tot, BB.e0f, BB.hf,
                       BB.ubf, BB.xbv, BB.yb, BB.f, BB.yf, BB.u, BB.scal, BB.work, BB.e0s, BB.lam0, BB.alphaK,
-                      SB.xb, SB.ypart})
+                      BB.dsub, BB.cd, BB.ce, BB.dots, BB.snear, SB.xb, SB.ypart})
         if (q) release(q);
     const int64_t nl = nlam, nb = D.nbnd, nc = std::max(ncoarse, 1), na = std::max<int64_t>(asubv[nsub], 1);
     BB.x = alloc<double>(K * nl);
@@ -2343,231 +2397,97 @@ void espreso_feti_s::block_setup(int K) {
     BB.f = alloc<double>(K * uoff[nsub]);
     BB.yf = alloc<double>(K * std::max<int64_t>(nyf, 1));
     BB.u = alloc<double>(K * uoff[nsub]);
-    BB.scal = alloc<double>(8 * K);
+    BB.scal = alloc<double>((size_t)PCG_SLOTS * K);
     BB.work = alloc<double>(16 * std::max<int64_t>(nyf, 1));
     BB.e0s = alloc<double>(K * n_e0s);
     BB.lam0 = alloc<double>(K * n_lambda0);
     BB.alphaK = alloc<double>(K * na);
+    BB.dsub = alloc<double>(K * n_dsub);
+    BB.cd = alloc<double>(K * nc);
+    BB.ce = alloc<double>(K * nc);
+    size_t dots = 0;  // any group of up to K cases uses these buffers
+    for (int k = 1; k <= K; k++) dots = std::max(dots, 3 * (size_t)dot_blocks(nlam, k) * k);
+    BB.dots = alloc<double>(dots);
+    BB.snear = n_near > 0 ? alloc<double>(K * n_near) : nullptr;
     SB.xb = alloc<double>(K * nb);
     SB.ypart = alloc<double>(K * std::max<int64_t>(SB.plen, 1));
     BB.K = K;
 }
 
-void espreso_feti_s::lanes_setup() {
-    if (!lanes_ready) {
-        for (Lane &l : lanes) {
-            ESP_HIP(hipStreamCreate(&l.s));
-            ESP_HIP(hipEventCreateWithFlags(&l.ev, hipEventDisableTiming));
-            l.dsub = alloc<double>(n_dsub);
-            l.cd = alloc<double>(std::max(ncoarse, 1));
-            l.ce = alloc<double>(std::max(ncoarse, 1));
-            l.lambda0 = alloc<double>(n_lambda0);
-            l.alphaK = alloc<double>(std::max<int64_t>(asubv[nsub], 1));
-            l.e0s = alloc<double>(n_e0s);
-            l.partial = alloc<double>(1024);
-        }
-        ESP_HIP(hipEventCreateWithFlags(&ev_main, hipEventDisableTiming));
-        lanes_ready = true;
-    }
-    // the operators of the current set-up with the lane's own scratch
-    for (Lane &l : lanes) {
-        l.D = D;
-        l.D.dsub = l.dsub;
-        l.D.cd = l.cd;
-        l.D.ce = l.ce;
-        l.C = CL;
-        l.C.lambda0 = l.lambda0;
-        l.C.alphaK = l.alphaK;
-    }
+// the vectors of a block of K cases (interleaved) with the current operators
+espreso_feti_s::PcgVec espreso_feti_s::block_vec(int K) {
+    PcgVec V{K, true, BB.x, BB.r, BB.w, BB.z, BB.y, BB.p, BB.Ap, BB.scal, BB.dots, D};
+    V.E.dsub = BB.dsub;
+    V.E.cd = BB.cd;
+    V.E.ce = BB.ce;
+    return V;
 }
 
-// lanes start after the work queued on the main stream; the main stream
-// continues after the lanes' work
-void espreso_feti_s::fork_lanes() {
-    ESP_HIP(hipEventRecord(ev_main, st));
-    for (Lane &l : lanes) ESP_HIP(hipStreamWaitEvent(l.s, ev_main, 0));
-}
-
-void espreso_feti_s::join_lanes() {
-    for (Lane &l : lanes) {
-        ESP_HIP(hipEventRecord(l.ev, l.s));
-        ESP_HIP(hipStreamWaitEvent(st, l.ev, 0));
+// Y = F X for the K interleaved cases: block SYMV, cluster correction, scatter
+void espreso_feti_s::apply_F_block(const PcgVec &V, const double *x, double *y, bool dot) {
+    const int K = V.K;
+    launch_boundary_gather(V.E, K, x, false, SB.xb, st);
+    launch_symv_mfma(V.E, SB, false, K, SB.xb, BB.yb, st);
+    if (hybrid) {
+        launch_subdomain_kernel_dots(V.E, K, x, BB.e0s, st);
+        launch_cluster_correction_multi(V.E, CL, K, BB.e0s, BB.lam0, n_lambda0, BB.alphaK,
+                                        std::max<int64_t>(asubv[nsub], 1), BB.yb, 1, st);
     }
-}
-
-// hybrid: the cluster correction of the block SYMV output BB.yb for the K
-// lambda-space vectors x: F0^-1 and F_i B0^T are read once for the group (main
-// stream), the kernel dots and the small alpha solves run per case on the lanes
-void espreso_feti_s::cluster_block(int K, const double *x) {
-    const int64_t na = std::max<int64_t>(asubv[nsub], 1);
-    fork_lanes();
-    for (int v = 0; v < K; v++)
-        launch_subdomain_kernel_dots(lanes[v % NLANE].D, x + (int64_t)v * nlam, BB.e0s + v * n_e0s,
-                                     lanes[v % NLANE].s);
-    join_lanes();
-    launch_cluster_t_multi(D, CL, K, BB.yb, D.nbnd, BB.lam0, n_lambda0, st);
-    fork_lanes();
-    for (int v = 0; v < K; v++)
-        launch_cluster_alpha(CL, BB.e0s + v * n_e0s, BB.lam0 + v * n_lambda0, BB.alphaK + v * na, lanes[v % NLANE].s);
-    join_lanes();
-    launch_cluster_apply_multi(D, CL, K, BB.lam0, n_lambda0, BB.alphaK, na, 1, BB.yb, D.nbnd, st);
-}
-
-// Y = F X for K lambda-space vectors: one block SYMV on the main stream, the
-// cluster correction, then the scatter of each vector on its lane
-void espreso_feti_s::apply_F_block(int K, const double *x, double *y) {
-    launch_symv_mfma(D, SB, false, K, x, false, BB.yb, st);
-    if (hybrid) cluster_block(K, x);
-    fork_lanes();
-    for (int v = 0; v < K; v++)
-        launch_lambda_gather(lanes[v % NLANE].D, BB.yb + v * D.nbnd, false, y + (int64_t)v * nlam, lanes[v % NLANE].s);
-    join_lanes();
-}
-
-// one PCG iteration of every active case (the block applies cover all K);
-// the per-case chains between the block applies run on the lanes
-void espreso_feti_s::step_block(int K, const std::vector<char> &active, bool first) {
-    const int64_t nl = nlam;
-    auto sc = [&](int v, int q) { return BB.scal + 8 * v + q; };  // 0 yw, 1 yw_prev, 2 pAp, 3 ww
-    auto lane = [&](int v) -> Lane & { return lanes[v % NLANE]; };
-    fork_lanes();
-    for (int v = 0; v < K; v++)
-        if (active[v]) launch_project(lane(v).D, BB.r + v * nl, BB.w + v * nl, 0, lane(v).s);
-    join_lanes();
-    const bool dir = opt.preconditioner == ESPRESO_PREC_DIRICHLET;
-    if (dir) {
-        launch_symv_mfma(D, SB, true, K, BB.w, true, BB.yb, st);
-    } else if (opt.preconditioner != ESPRESO_PREC_NONE) {
-        for (int v = 0; v < K; v++)
-            if (active[v]) apply_prec(BB.w + v * nl, BB.z + v * nl);  // main stream (shared boundary scratch)
-    }
-    fork_lanes();
-    for (int v = 0; v < K; v++) {
-        if (!active[v]) continue;
-        Lane &L = lane(v);
-        if (opt.preconditioner == ESPRESO_PREC_NONE) {
-            ESP_HIP(hipMemcpyAsync(BB.y + v * nl, BB.w + v * nl, nl * sizeof(double), hipMemcpyDeviceToDevice, L.s));
-        } else {
-            if (dir) launch_lambda_gather(L.D, BB.yb + v * D.nbnd, true, BB.z + v * nl, L.s);
-            launch_project(L.D, BB.z + v * nl, BB.y + v * nl, 0, L.s);
-        }
-        if (!first) launch_copy_scalar(sc(v, 0), sc(v, 1), L.s);
-        launch_dot(BB.y + v * nl, BB.w + v * nl, nl, L.partial, sc(v, 0), L.s);
-        launch_p_update(BB.p + v * nl, BB.y + v * nl, nl, sc(v, 0), sc(v, 1), first, L.s);
-    }
-    join_lanes();
-    launch_symv_mfma(D, SB, false, K, BB.p, false, BB.yb, st);
-    if (hybrid) cluster_block(K, BB.p);
-    fork_lanes();
-    for (int v = 0; v < K; v++) {
-        if (!active[v]) continue;
-        Lane &L = lane(v);
-        double *ybv = BB.yb + v * D.nbnd, *Apv = BB.Ap + v * nl;
-        launch_lambda_gather(L.D, ybv, false, Apv, L.s);
-        launch_dot(BB.p + v * nl, Apv, nl, L.partial, sc(v, 2), L.s);
-        launch_xr_update(BB.x + v * nl, BB.r + v * nl, BB.p + v * nl, Apv, nl, sc(v, 0), sc(v, 2), L.s);
-        launch_dot(BB.w + v * nl, BB.w + v * nl, nl, L.partial, sc(v, 3), L.s);
-    }
-    join_lanes();
-}
-
-void espreso_feti_s::step_block_graph(int K) {
-    for (const BlockGraph &g : block_graphs)
-        if (g.K == K) {
-            ESP_HIP(hipGraphLaunch(g.exec, st));
-            return;
-        }
-    const std::vector<char> all(K, 1);
-    hipGraph_t graph = nullptr;
-    ESP_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    try {
-        step_block(K, all, false);
-    } catch (...) {
-        (void)hipStreamEndCapture(st, &graph);
-        if (graph) (void)hipGraphDestroy(graph);
-        throw;
-    }
-    ESP_HIP(hipStreamEndCapture(st, &graph));
-    BlockGraph g{K, nullptr};
-    const hipError_t e = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(graph);
-    ESP_HIP(e);
-    block_graphs.push_back(g);
-    ESP_HIP(hipGraphLaunch(g.exec, st));
+    launch_lambda_gather(V.E, K, BB.yb, false, y, st, dot ? x : nullptr,
+                         dot ? V.dots + 2 * (size_t)dot_blocks(nlam, K) * K : nullptr);
 }
 
 void espreso_feti_s::resolve_group(int K, const double *f, double *u, int32_t *iters, double *norms,
                                    espreso_feti_stats &tot) {
     const double t0 = wall();
     block_setup(K);
-    lanes_setup();
+    const PcgVec V = block_vec(K);
     const int64_t nl = nlam, nb = D.nbnd, nt = uoff[nsub], na = std::max<int64_t>(asubv[nsub], 1);
-    const int64_t nc = std::max(ncoarse, 1);
-    // loads: e0f, e on the host; f, y_f, hf (one band-solve launch) and b on the device
-    hvec<double> e0f;
-    std::vector<double> e;
+    // loads: e0f, e on the host (interleaved by case); f, y_f, hf (one band-solve launch) and b on the device
     ESP_HIP(hipMemcpyAsync(BB.f, f, K * nt * sizeof(double), hipMemcpyHostToDevice, st));
+    std::vector<double> e0f_all((size_t)K * asubv[nsub]), e_all((size_t)K * ncoarse);
     for (int v = 0; v < K; v++) {
+        hvec<double> e0f;
+        std::vector<double> e;
         rhs_host(f + v * nt, e0f, e);
-        if (!e0f.empty())
-            ESP_HIP(hipMemcpyAsync(BB.e0f + v * na, e0f.data(), e0f.size() * sizeof(double), hipMemcpyHostToDevice, st));
-        if (!e.empty())
-            ESP_HIP(hipMemcpyAsync(BB.e + v * nc, e.data(), e.size() * sizeof(double), hipMemcpyHostToDevice, st));
-        sync();  // host vectors e0f, e are reused by the next case
+        for (size_t q = 0; q < e0f.size(); q++) e0f_all[q * K + v] = e0f[q];
+        for (size_t q = 0; q < e.size(); q++) e_all[q * K + v] = e[q];
     }
-    launch_rhs_prepare_multi(P, nsub, K, BB.f, nt, BB.hf, nb, BB.yf, nyf, BB.work, st);
-    for (int v = 0; v < K; v++) compute_b_into(BB.hf + v * nb, BB.ubf + v * nb, BB.e0f + v * na, BB.b + v * nl);
+    ESP_HIP(hipMemcpyAsync(BB.e0f, e0f_all.data(), e0f_all.size() * sizeof(double), hipMemcpyHostToDevice, st));
+    ESP_HIP(hipMemcpyAsync(BB.e, e_all.data(), e_all.size() * sizeof(double), hipMemcpyHostToDevice, st));
+    launch_rhs_prepare_multi(P, nsub, K, BB.f, nt, BB.hf, BB.yf, nyf, BB.work, st);
+    // K^+ f on the boundary: ubf = F_i hf, hybrid + cluster correction; b = B K^+ f - c
+    launch_symv_mfma(D, SB, false, K, BB.hf, BB.yb, st);
+    ESP_HIP(hipMemcpyAsync(BB.ubf, BB.yb, K * nb * sizeof(double), hipMemcpyDeviceToDevice, st));
+    if (hybrid)
+        launch_cluster_correction_multi(D, CL, K, BB.e0f, BB.lam0, n_lambda0, BB.alphaK, na, BB.yb, 1, st);
+    launch_lambda_gather(V.E, K, BB.yb, false, BB.b, st);
+    launch_sub_lines(nl, K, BB.b, d_c, st);
     // lambda0 = G^T (GG^T)^-1 e ; r = b - F lambda0 ; tol = precision * min(||P r0||, ||b||)
-    for (int v = 0; v < K; v++) launch_project(D, BB.e + v * nc, BB.x + v * nl, 1, st);
-    apply_F_block(K, BB.x, BB.Ap);
-    for (int v = 0; v < K; v++) {
-        launch_axpby(BB.r + v * nl, BB.b + v * nl, BB.Ap + v * nl, nl, 1.0, -1.0, st);
-        launch_project(D, BB.r + v * nl, BB.w + v * nl, 0, st);
-        launch_dot(BB.w + v * nl, BB.w + v * nl, nl, d_partial, BB.scal + 8 * v + 4, st);
-        launch_dot(BB.b + v * nl, BB.b + v * nl, nl, d_partial, BB.scal + 8 * v + 5, st);
-    }
-    std::vector<double> hs(8 * K);
-    ESP_HIP(hipMemcpyAsync(hs.data(), BB.scal, hs.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-    sync();
+    launch_project(V.E, K, BB.e, BB.x, 1, st);
+    apply_F_block(V, BB.x, BB.Ap, false);
+    launch_axpby(BB.r, BB.b, BB.Ap, K * nl, 1.0, -1.0, st);
+    pcg_start(V, BB.b, 0.0);
+    sync();  // the host vectors above are in use until here
     const double t1 = wall();
-    std::vector<double> tol(K), nrm(K, 0.0);
-    std::vector<char> active(K, 1);
-    std::vector<int> it_v(K, 0);
-    for (int v = 0; v < K; v++) tol[v] = opt.precision * std::min(std::sqrt(hs[8 * v + 4]), std::sqrt(hs[8 * v + 5]));
-    bool all_active = true;
-    for (int it = 0; it < opt.max_iterations; it++) {
-        if (it > 0 && all_active && use_graphs) step_block_graph(K);
-        else step_block(K, active, it == 0);
-        ESP_HIP(hipMemcpyAsync(hs.data(), BB.scal, hs.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-        sync();
-        bool any = false;
-        for (int v = 0; v < K; v++) {
-            if (!active[v]) continue;
-            ESP_CHECK(std::isfinite(hs[8 * v + 3]), ESPRESO_ERR_NUMERIC, "block PCG produced a non-finite residual");
-            nrm[v] = std::sqrt(hs[8 * v + 3]);
-            it_v[v] = it + 1;
-            if (nrm[v] < tol[v]) active[v] = 0;
-            any |= active[v] != 0;
-            all_active = all_active && active[v];
-        }
-        if (!any) break;
-    }
+    pcg_loop(V, 0);
+    std::vector<double> tol(rec->tol, rec->tol + K), nrm(K);
+    std::vector<int> it_v(rec->iters, rec->iters + K);
+    for (int v = 0; v < K; v++) nrm[v] = std::sqrt(rec->ww[v]);
     sync();
     const double t2 = wall();
     // primal per case: u = K~^+ (f - B^T lambda) + R~ alpha
-    for (int v = 0; v < K; v++) launch_project(D, BB.r + v * nl, BB.alpha_c + v * nc, 2, st);
-    launch_symv_mfma(D, SB, false, K, BB.x, false, BB.yb, st);
-    for (int v = 0; v < K; v++) {
-        double *xb = BB.xbv + v * nb;
-        launch_axpby(xb, BB.ubf + v * nb, BB.yb + v * nb, nb, 1.0, -1.0, st);
-        if (hybrid) {
-            launch_subdomain_kernel_dots(D, BB.x + v * nl, d_e0s, st);
-            launch_axpby(d_e0s, BB.e0f + v * na, d_e0s, asubv[nsub], 1.0, -1.0, st);
-            launch_cluster_correction(D, CL, d_e0s, xb, 0, st);
-        }
-        launch_alpha_combine(D, CL, hybrid, BB.alpha_c + v * nc, BB.alpha_tot + v * na, st);
+    launch_project(V.E, K, BB.r, BB.alpha_c, 2, st);
+    launch_boundary_gather(V.E, K, BB.x, false, SB.xb, st);
+    launch_symv_mfma(D, SB, false, K, SB.xb, BB.yb, st);
+    launch_axpby(BB.xbv, BB.ubf, BB.yb, K * nb, 1.0, -1.0, st);
+    if (hybrid) {
+        launch_subdomain_kernel_dots(V.E, K, BB.x, BB.e0s, st);
+        launch_axpby(BB.e0s, BB.e0f, BB.e0s, K * asubv[nsub], 1.0, -1.0, st);
+        launch_cluster_correction_multi(D, CL, K, BB.e0s, BB.lam0, n_lambda0, BB.alphaK, na, BB.xbv, 0, st);
     }
-    launch_primal_multi(P, nsub, K, BB.xbv, nb, BB.yf, nyf, BB.alpha_tot, na, BB.u, nt, BB.work, st);
+    launch_alpha_combine(D, K, BB.alphaK, na, hybrid, BB.alpha_c, BB.alpha_tot, st);
+    launch_primal_multi(P, nsub, K, BB.xbv, BB.yf, nyf, BB.alpha_tot, na, BB.u, nt, BB.work, st);
     ESP_HIP(hipMemcpyAsync(u, BB.u, K * nt * sizeof(double), hipMemcpyDeviceToHost, st));
     sync();
     for (int v = 0; v < K; v++) {
@@ -2710,6 +2630,8 @@ void espreso_feti_s::coarse_layout_subdomains() {
     D.blk_ptr = upload(bptr);
     D.blk_sub = upload(bsub);
     D.Rt = D.Rb;
+    D.RtT = D.RbT;
+    D.coarse_direct = true;  // asub is the coarse offset
     D.rtoff = D.rboff;
     D.dsub_off = D.asub;
     n_dsub = std::max<int64_t>(1, asubv[nsub]);
@@ -2962,6 +2884,8 @@ void espreso_feti_s::load_clusters() {
     D.blk_sub = upload(bsub);
     D.rtoff = upload(rtoff);
     D.Rt = upload(Rt);
+    D.RtT = alloc<double>(rtoff[nsub]);
+    launch_basis_rows(nsub, D.max_m, D.m, D.ck, D.rtoff, D.Rt, D.RtT, st);
     D.N = upload(Ns);
     D.noff = upload(noff);
     D.dsub_off = upload(dsub_off);
@@ -3334,8 +3258,8 @@ int espreso_feti_load_work(espreso_feti *h, double *c) {
     ESP_CHECK(h && c, ESPRESO_ERR_ARG, "null argument");
     ESP_CHECK(h->solved, ESPRESO_ERR_STATE, "no solution");
     ESP_HIP(hipSetDevice(h->opt.device));
-    launch_dot(h->d_f, h->d_u, h->uoff[h->nsub], h->d_partial, h->d_scal + 8, h->st);
-    ESP_HIP(hipMemcpyAsync(c, h->d_scal + 8, sizeof(double), hipMemcpyDeviceToHost, h->st));
+    launch_dot(h->d_f, h->d_u, h->uoff[h->nsub], h->d_partial, h->d_scal + PCG_SLOTS + 8, h->st);
+    ESP_HIP(hipMemcpyAsync(c, h->d_scal + PCG_SLOTS + 8, sizeof(double), hipMemcpyDeviceToHost, h->st));
     h->sync();
     ESP_API_END
 }
@@ -3354,7 +3278,7 @@ static int dual_op(espreso_feti *h, const double *x, double *y, int which) {
     ESP_HIP(hipMemcpyAsync(h->d_z, x, bytes, hipMemcpyHostToDevice, h->st));
     if (which == 0) h->apply_F(h->d_z, h->d_tmp, h->opt.sc_precision);
     else if (which == 1) h->apply_prec(h->d_z, h->d_tmp);
-    else launch_project(h->D, h->d_z, h->d_tmp, 0, h->st);
+    else launch_project(h->D, 1, h->d_z, h->d_tmp, 0, h->st);
     ESP_HIP(hipMemcpyAsync(y, h->d_tmp, bytes, hipMemcpyDeviceToHost, h->st));
     h->sync();
     ESP_API_END
@@ -3401,7 +3325,7 @@ int espreso_feti_project_device(espreso_feti *h, const double *x, double *y, voi
     E.dsub = sp;
     E.cd = sp + h->n_dsub;
     E.ce = sp + h->n_dsub + h->ncoarse;
-    launch_project(E, x, y, 0, stream ? (hipStream_t)stream : h->st);
+    launch_project(E, 1, x, y, 0, stream ? (hipStream_t)stream : h->st);
     h->check_launches("projector");
     ESP_API_END
 }
