@@ -35,6 +35,13 @@ __device__ __forceinline__ double gload(const double *p) {
     return *(const __attribute__((address_space(1))) double *)p;
 }
 
+// orders the LDS accesses of a wave's own lanes
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // C(MxN) = alpha * op(A)(MxK) * op(B)(KxN) + beta * C, M,N <= 64.
 // op(A)(i,k) = TA ? A[k + i*lda] : A[i + k*lda];  op(B)(k,j) = TB ? B[j + k*ldb] : B[k + j*ldb].
 // C may alias A or B when this tile is the only reader of the aliased tile:
@@ -445,11 +452,28 @@ __device__ __forceinline__ void pick(const DenseDesc &d, int which, double *&A, 
 }
 
 // ---- block Cholesky, step k ----
+__device__ __forceinline__ double read_lane(double v, int lane) {
+    const long long b = __builtin_bit_cast(long long, v);
+    const unsigned lo = __builtin_amdgcn_readlane((int)b, lane), hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    return __builtin_bit_cast(double, (long long)(((unsigned long long)hi << 32) | lo));
+}
+
 // diagonal tile: factor the tile and invert its factor (one workgroup per
 // subdomain).  Its updates by the block columns to its left, A_kk -= L_kj
 // L_kj^T, were applied by the panel steps j that produced L_kj, so this
 // latency-bound chain of launches carries no GEMM of its own.
-__global__ void __launch_bounds__(256) k_potrf_diag(const DenseDesc *D, int which, int step) {
+// What bounds it is the chain of 64 pivots.  Right-looking over four 16-column
+// blocks: wave 0 holds row r of the block column in lane r, so that one pass of
+// 16 pivots (left-looking inside the block, the multipliers broadcast with
+// v_readlane, the reciprocal root by v_rsq_f64 and one third-order step) factors
+// the diagonal block and solves the rows below it together; the rank-16 update of the trailing blocks
+// runs on MFMA over the four waves.  The inverse takes the four diagonal blocks
+// at once (a column per lane) and the blocks below by distance on MFMA, the sum
+// staying in the accumulators (their layout is the B operand of the product
+// with the inverted diagonal block).  60 -> 29 us a step at 64 subdomains of 5^3;
+// beside the MFMA work of the substitution 92 -> 50 us at 64 x 10^3 (wave priority
+// raised: this chain is what the other launches of a step wait for).
+__global__ void __launch_bounds__(256, 4) k_potrf_diag(const DenseDesc *D, int which, int step) {
     const DenseDesc &d = D[blockIdx.x];
     double *A, *B;
     int lda, n, band, nt, ncols, ntc;
@@ -458,146 +482,121 @@ __global__ void __launch_bounds__(256) k_potrf_diag(const DenseDesc *D, int whic
     if (k0 >= n) return;
     const int nb = min(TILE, n - k0);
     double *Akk = A + k0 + (size_t)k0 * lda;
-    __shared__ double T[TILE][TILE + 1];
-    __shared__ double xd[TILE];
-    __shared__ double tmp[3][16][17];
-    __shared__ int bad;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid == 0) bad = 0;
-    for (int q = tid; q < TILE * TILE; q += 256) {
-        int i = q & 63, j = q >> 6;
-        double v;
-        if (i < nb && j < nb) v = (i >= j) ? Akk[i + (size_t)j * lda] : 0.0;
-        else v = (i == j) ? 1.0 : 0.0;
-        T[i][j] = v;
+    __shared__ double T[TILE][TILE + 1];  // L below the diagonal; X = L^-1 above it: X(i, j), i > j, at T[j][i]
+    __shared__ double xd[TILE];           // X(i, i)
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, kq = lane >> 4;
+    __builtin_amdgcn_s_setprio(3);
+#pragma unroll 4
+    for (int it = 0; it < 16; it++) {
+        const int i = lane, j = wave + 4 * it;
+        const bool in = i < nb && j < nb && i >= j;
+        const double v = gload(Akk + (in ? i + (size_t)j * lda : 0));
+        T[i][j] = in ? v : (i == j ? 1.0 : 0.0);
     }
     __syncthreads();
-    // ---- T = L L^T, right-looking over four 16-column blocks ----
-    for (int kb = 0; kb < 4; kb++) {
-        const int c0 = kb * 16;
+    // ---- T = L L^T ----
+    int bad = 0;  // first failing column of the tile (wave 0; 1-based)
+    for (int c0 = 0; c0 < TILE; c0 += 16) {
         if (wave == 0) {
-            // diagonal block in registers: lane r < 16 holds row r
-            const int r = lane;
             double v[16];
 #pragma unroll
-            for (int c = 0; c < 16; c++) v[c] = (r < 16 && c <= r) ? T[c0 + r][c0 + c] : 0.0;
+            for (int c = 0; c < 16; c++) v[c] = T[lane][c0 + c];
 #pragma unroll
             for (int j = 0; j < 16; j++) {
-                double piv = __shfl(v[j], j, 64);
-                if (!(piv > 0.0) || !isfinite(piv)) {
-                    if (lane == 0 && bad == 0) bad = c0 + j + 1;
-                    piv = 1.0;
-                }
-                const double dd = sqrt(piv);
-                if (r == j) v[j] = dd;
-                else if (r > j) v[j] = v[j] / dd;
+                // the columns k < j of this block, each broadcast used at once
+                // (right-looking, the compiler would keep and spill them)
+                double a0 = v[j], a1 = 0.0;
 #pragma unroll
-                for (int c = j + 1; c < 16; c++) {
-                    const double lc = __shfl(v[j], c, 64);
-                    if (r >= c) v[c] -= v[j] * lc;
+                for (int k = 0; k < j; k++) {
+                    const double lk = read_lane(v[k], c0 + j);
+                    if ((j - k) & 1) a0 = fma(-v[k], lk, a0);
+                    else a1 = fma(-v[k], lk, a1);
                 }
+                a0 += a1;
+                double piv = read_lane(a0, c0 + j);
+                const bool ok = piv > 0.0 && piv <= 1.7976931348623157e308;
+                bad = (bad == 0 && !ok) ? c0 + j + 1 : bad;
+                piv = ok ? piv : 1.0;
+                // y = piv^-1/2: with e = 1 - piv y0^2, y0 (1 - e)^-1/2 = y0 (1 + e/2 + 3/8 e^2 + ...)
+                double y = __builtin_amdgcn_rsq(piv);
+                const double e = fma(-piv * y, y, 1.0);
+                y = fma(y * e, fma(0.375, e, 0.5), y);
+                double r = piv * y;  // the root, corrected by half its residual
+                r = fma(0.5 * y, fma(-r, r, piv), r);
+                v[j] = lane == c0 + j ? r : a0 * y;
+                xd[c0 + j] = y;  // the same value from every lane
+                __builtin_amdgcn_sched_barrier(0);
             }
-            if (r < 16) {
+            if (lane >= c0) {  // above the diagonal: overwritten by X below
 #pragma unroll
-                for (int c = 0; c < 16; c++)
-                    if (c <= r) T[c0 + r][c0 + c] = v[c];
+                for (int c = 0; c < 16; c++) T[lane][c0 + c] = v[c];
             }
         }
         __syncthreads();
-        const int rest = TILE - c0 - 16;
-        if (rest == 0) break;
-        // panel rows below: L_rb = A_rb L_bb^-T, one thread per row
-        if (tid < rest) {
-            const int r = c0 + 16 + tid;
-            double x[16];
+        // trailing blocks (I, J), c0/16 < J <= I, wave w every fourth of them
+        const int kb = c0 >> 4, rest = 3 - kb;
+        for (int q = wave; q < rest * (rest + 1) / 2; q += 4) {
+            const int I = q < 1 ? 0 : (q < 3 ? 1 : 2), J = q - I * (I + 1) / 2;
+            const int ri = 16 * (kb + 1 + I), rj = 16 * (kb + 1 + J);
+            d4 acc = d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-            for (int c = 0; c < 16; c++) {
-                double sv = T[r][c0 + c];
+            for (int s = 0; s < 4; s++)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(T[ri + l16][c0 + 4 * s + kq], T[rj + l16][c0 + 4 * s + kq],
+                                                           acc, 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < c; i++) sv -= x[i] * T[c0 + c][c0 + i];
-                x[c] = sv / T[c0 + c][c0 + c];
-            }
-#pragma unroll
-            for (int c = 0; c < 16; c++) T[r][c0 + c] = x[c];
+            for (int v = 0; v < 4; v++) T[ri + kq + 4 * v][rj + l16] -= acc[v];
         }
         __syncthreads();
-        // trailing lower block update (rank 16)
-        for (int q = tid; q < rest * rest; q += 256) {
-            const int rr = c0 + 16 + q % rest, cc = c0 + 16 + q / rest;
-            if (rr < cc) continue;
+    }
+    // ---- X = L^-1: diagonal blocks, wave w block w: row by row, column c in lanes
+    // c + 16 kq, which share the sum over k (rows of X above come from LDS) ----
+    {
+        const int c0 = wave * 16, c = l16;
+        for (int i = 0; i < 16; i++) {
             double sv = 0.0;
 #pragma unroll
-            for (int i = 0; i < 16; i++) sv += T[rr][c0 + i] * T[cc][c0 + i];
-            T[rr][cc] -= sv;
-        }
-        __syncthreads();
-    }
-    // ---- X = L^-1 (lower): X(i,j), i > j, kept at T[j][i]; X(i,i) in xd[i] ----
-    // diagonal 16x16 blocks: wave w inverts block w, lane c < 16 one column
-    {
-        const int c0 = wave * 16, c = lane;
-        if (c < 16) {
-            double x[16];
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                if (i < c) {
-                    x[i] = 0.0;
-                    continue;
-                }
-                double sv = (i == c) ? 1.0 : 0.0;
-#pragma unroll
-                for (int k = 0; k < i; k++)
-                    if (k >= c) sv -= T[c0 + i][c0 + k] * x[k];
-                x[i] = sv / T[c0 + i][c0 + i];
+            for (int t = 0; t < 4; t++) {
+                const int k = kq + 4 * t;
+                const double l = T[c0 + i][c0 + k], x = T[c0 + c][c0 + k], xk = xd[c0 + k];
+                // columns k < i of L, rows k >= c of X
+                sv = fma(k < i ? l : 0.0, k > c ? x : (k == c ? xk : 0.0), sv);
             }
-            xd[c0 + c] = x[c];
-#pragma unroll
-            for (int i = 0; i < 16; i++)
-                if (i > c) T[c0 + c][c0 + i] = x[i];
+            sv += __shfl_xor(sv, 16, 64);
+            sv += __shfl_xor(sv, 32, 64);
+            if (kq == 0 && i > c) T[c0 + c][c0 + i] = -sv * xd[c0 + i];
+            wave_lds_sync();
         }
     }
     __syncthreads();
-    // off-diagonal blocks by distance: X_IJ = -X_II sum_{K=J}^{I-1} L_IK X_KJ
+    // off-diagonal blocks by distance: X_IJ = -X_II sum_{K=J}^{I-1} L_IK X_KJ, wave J
+    auto xval = [&](int row, int col) {
+        const double v = T[min(row, col)][max(row, col)], w = xd[row];
+        return row > col ? v : (row == col ? w : 0.0);
+    };
     for (int dist = 1; dist < 4; dist++) {
         const int J = wave, I = wave + dist;
-        const bool act = I < 4;
-        const int a = lane & 15;
-        if (act) {
-            for (int t = 0; t < 4; t++) {
-                const int bcol = (lane >> 4) + 4 * t;
-                double sv = 0.0;
-                for (int K = J; K < I; K++)
-                    for (int k = 0; k < 16; k++) {
-                        const int row = K * 16 + k, col = J * 16 + bcol;
-                        double xv;
-                        if (row > col) xv = T[col][row];
-                        else xv = (row == col) ? xd[row] : 0.0;
-                        sv += T[I * 16 + a][K * 16 + k] * xv;
-                    }
-                tmp[wave][a][bcol] = sv;
-            }
-        }
-        __syncthreads();
-        if (act) {
-            for (int t = 0; t < 4; t++) {
-                const int bcol = (lane >> 4) + 4 * t;
-                double sv = 0.0;
-                for (int k = 0; k <= a; k++) {
-                    const int row = I * 16 + a, col = I * 16 + k;
-                    const double xv = (row == col) ? xd[row] : T[col][row];
-                    sv += xv * tmp[wave][k][bcol];
-                }
-                T[J * 16 + bcol][I * 16 + a] = -sv;
-            }
+        if (I < 4) {
+            d4 acc = d4{0.0, 0.0, 0.0, 0.0}, out = d4{0.0, 0.0, 0.0, 0.0};
+            for (int K = J; K < I; K++)
+#pragma unroll
+                for (int s = 0; s < 4; s++)
+                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(T[16 * I + l16][16 * K + 4 * s + kq],
+                                                               xval(16 * K + 4 * s + kq, 16 * J + l16), acc, 0, 0, 0);
+            // acc holds rows kq + 4 v, column l16: the B operand of the k-step over rows 4v..4v+3
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                out = __builtin_amdgcn_mfma_f64_16x16x4f64(xval(16 * I + l16, 16 * I + 4 * v + kq), acc[v], out, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; v++) T[16 * J + l16][16 * I + kq + 4 * v] = -out[v];
         }
         __syncthreads();
     }
-    __syncthreads();
     if (tid == 0 && bad && d.info[0] == 0) d.info[0] = k0 + bad;
     double *Dinv = d.Dinv + (size_t)step * TILE * TILE;
-    for (int q = tid; q < TILE * TILE; q += 256) {
-        int i = q & 63, j = q >> 6;
-        Dinv[q] = i > j ? T[j][i] : (i == j ? xd[i] : 0.0);
+#pragma unroll 4
+    for (int it = 0; it < 16; it++) {
+        const int q = tid + 256 * it, i = lane, j = wave + 4 * it;
+        Dinv[q] = xval(i, j);
         if (i < nb && j < nb && i >= j) Akk[i + (size_t)j * lda] = T[i][j];
     }
 }
@@ -1165,12 +1164,6 @@ __global__ void k_unpack(const T *pool, int64_t off, int m, float scale, double 
 // in its own LDS window of MAT_W rows; only wave-level synchronisation, so the
 // waves of a workgroup proceed independently.
 constexpr int MAT_W = 1024;
-
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 __global__ void __launch_bounds__(256) k_materialize(const DenseDesc *D, const int *rowptr, const int64_t *rp_off,
                                                      const int *colidx, const double *vals, const int64_t *nz_off,
