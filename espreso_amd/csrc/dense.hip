@@ -307,119 +307,198 @@ __device__ __forceinline__ void diag_update(const d4 (&o)[4], double *lds, doubl
         }
 }
 
-// ---- two column tiles per workgroup (forward substitution) ----
-// The tiles (i, J) and (i, J+1) of one block row share the A operand (rows i of
-// the factor) and the diagonal inverse: each wave owns 16 columns of both
-// tiles.  A tile's B rows before its own window start (kfirst[s]) are read as
-// zero: the other tile may start its window earlier.
-constexpr int FUSED2_LDS = 2 * 16 * (TILE + 1) + 2 * 16 * (2 * TILE + 1);  // doubles
+// ---- wave tiles: one 64 x 64 tile per wave, operands straight from memory ----
+// The FP64 MFMA and every VALU instruction share the issue of a SIMD (8 integer
+// adds per 16x16x4 MFMA cost it 21 % of its rate, measured), and one MFMA takes 64
+// cycles.  A wave that owns a whole 64 x 64 tile needs 8 operand values per lane
+// for 16 MFMAs and loads them from global memory into registers, so the loop has
+// no LDS traffic, no barrier and, with the operands at a uniform pointer plus a
+// constant 32-bit offset, almost no VALU: S = -Y^T Y at 3993 x 2598 (64 matrices)
+// runs at 66.7 TFLOP/s against 49-50 for the four-wave tile through LDS (72 is
+// what the MFMA reaches in registers).  The accumulators take 128 registers, two
+// chunks of 8 columns of K 64: two waves per SIMD.
+//
+// Operands: K-contiguous, element (i, k) at p[k + i ld] (a lane reads columns k0 +
+// 2 kq and + 1 of K as 16 bytes, the four lanes of a row one 64-byte piece), or
+// M-contiguous at p[i + k ld] (16 lanes read 128 consecutive bytes).  The MFMA's
+// k-step s takes K = k0 + 2 kq + s from lane quarter kq for both operands: any
+// order of K serves as long as A and B agree.  Rows past M repeat row M - 1; the
+// caller masks its results.
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+constexpr int WAVE_KC = 8;
 
-__device__ __forceinline__ void strip2_gemm(d4 (&acc)[2][4], double *lds, const double *A, int lda, const double *B,
-                                            int ldb, int M, int N, int K, const int (&kfirst)[2]) {
-    double(*As)[16][TILE + 1] = reinterpret_cast<double(*)[16][TILE + 1]>(lds);
-    double(*Bs)[16][2 * TILE + 1] = reinterpret_cast<double(*)[16][2 * TILE + 1]>(lds + 2 * 16 * (TILE + 1));
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    double ra[4], rb[8];
-    int fk = 0;
-    auto bok = [&](int j, int k) { return j < N && k < K && k >= kfirst[j >> 6]; };
-    auto fetch = [&](int k0) {
-        fk = k0;
+// values that are the same in every lane, kept in scalar registers (the compiler
+// cannot tell: they come out of descriptors that the kernel's stores might alias)
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ const double *uniform(const double *p) {
+    const unsigned long long b = (unsigned long long)p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+    return (const double *)(((unsigned long long)hi << 32) | lo);
+}
+
+template <bool KC>  // K-contiguous
+struct WaveOperand {
+    const char *p;  // uniform: the chunk's first element
+    unsigned off[4];
+    size_t step, next;  // bytes per chunk and per k
+    __device__ __forceinline__ void init(const double *a, int ld, int M) {
+        const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
+        p = (const char *)uniform(a);
+        ld = uniform(ld);
 #pragma unroll
-        for (int it = 0; it < 4; it++) {
-            const int q = tid + 256 * it, i = q & 63, kk = q >> 6;
-            const bool va = i < M && k0 + kk < K;
-            ra[it] = gload(A + (va ? i + (size_t)(k0 + kk) * lda : 0));
+        for (int r = 0; r < 4; r++) {
+            const unsigned i = min(16 * r + l16, M - 1);
+            off[r] = KC ? (i * (unsigned)ld + 2 * kq) * 8u : (i + 2u * kq * (unsigned)ld) * 8u;
         }
+        step = KC ? WAVE_KC * 8 : (size_t)ld * (WAVE_KC * 8);
+        next = KC ? 8 : (size_t)ld * 8;
+    }
+    __device__ __forceinline__ void load(double (&x)[4][2]) {
+        // opaque copies, so that pointer and offset stay apart (scalar pointer plus
+        // 32-bit lane offset is an addressing mode; a hoisted 64-bit sum per load is not)
+        asm volatile("" : "+s"(p));
+        const char *p1 = p + next;
 #pragma unroll
-        for (int it = 0; it < 8; it++) {
-            const int q = tid + 256 * it, kk = q & 15, j = q >> 4;
-            rb[it] = gload(B + (bok(j, k0 + kk) ? (k0 + kk) + (size_t)j * ldb : 0));
-        }
-    };
-    auto store = [&](int buf) {
-#pragma unroll
-        for (int it = 0; it < 4; it++) {
-            const int q = tid + 256 * it, i = q & 63, kk = q >> 6;
-            As[buf][kk][i] = (i < M && fk + kk < K) ? ra[it] : 0.0;
-        }
-#pragma unroll
-        for (int it = 0; it < 8; it++) {
-            const int q = tid + 256 * it, kk = q & 15, j = q >> 4;
-            Bs[buf][kk][j] = bok(j, fk + kk) ? rb[it] : 0.0;
-        }
-    };
-    fetch(0);
-    store(0);
-    __syncthreads();
-    if (16 < K) fetch(16);
-    for (int k0 = 0, cur = 0; k0 < K; k0 += 16, cur ^= 1) {
-#pragma unroll
-        for (int ks = 0; ks < 16; ks += 4) {
-            const int kr = ks + (lane >> 4);
-            double a[4];
-#pragma unroll
-            for (int r = 0; r < 4; r++) a[r] = As[cur][kr][16 * r + (lane & 15)];
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                const double b = Bs[cur][kr][TILE * t + 16 * wave + (lane & 15)];
-#pragma unroll
-                for (int r = 0; r < 4; r++) acc[t][r] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], b, acc[t][r], 0, 0, 0);
+        for (int r = 0; r < 4; r++) {
+            asm volatile("" : "+v"(off[r]));
+            const unsigned o = off[r];
+            if constexpr (KC) {
+                const d2u v = *(const __attribute__((address_space(1))) d2u *)(p + o);
+                x[r][0] = v[0];
+                x[r][1] = v[1];
+            } else {
+                x[r][0] = *(const __attribute__((address_space(1))) double *)(p + o);
+                x[r][1] = *(const __attribute__((address_space(1))) double *)(p1 + o);
             }
         }
-        if (k0 + 16 < K) store(cur ^ 1);
-        __syncthreads();  // after the last chunk: the operand buffers are free
-        if (k0 + 32 < K) fetch(k0 + 32);
+        p += step;
+    }
+    // the last, partial chunk: `left` columns of K, zeros after them
+    __device__ __forceinline__ void load_tail(double (&x)[4][2], int left) {
+        const int kq = (threadIdx.x & 63) >> 4;
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                const bool in = 2 * kq + s < left;
+                // a lane past the end reads its row's first column of the chunk
+                const unsigned o = in ? off[r] + (unsigned)(s * next) : off[r] - (unsigned)(2 * kq * next);
+                const double v = *(const __attribute__((address_space(1))) double *)(p + o);
+                x[r][s] = in ? v : 0.0;
+            }
+    }
+};
+
+// acc[r][c] += op(A)(rows of block r, :K) op(B)(:K, columns of block c): lane value v
+// of acc[r][c] is element (16 r + kq + 4 v, 16 c + l16)
+template <bool AK, bool BK>
+__device__ __forceinline__ void wave_gemm(d4 (&acc)[4][4], const double *A, int lda, const double *B, int ldb, int M,
+                                          int N, int K) {
+    WaveOperand<AK> oa;
+    WaveOperand<BK> ob;
+    oa.init(A, lda, M);
+    ob.init(B, ldb, N);
+    double a[2][4][2], b[2][4][2];
+    auto mul = [&](const double (&x)[4][2], const double (&y)[4][2]) {
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[r][s], y[c][s], acc[r][c], 0, 0, 0);
+    };
+    K = uniform(K);
+    int chunks = K / WAVE_KC;
+    const int left = K - chunks * WAVE_KC;
+    if (chunks > 0) {
+        oa.load(a[0]);
+        ob.load(b[0]);
+        // two chunks per round: the next one's loads fly while the MFMAs of the
+        // current one run
+        for (; chunks > 2; chunks -= 2) {
+            oa.load(a[1]);
+            ob.load(b[1]);
+            mul(a[0], b[0]);
+            oa.load(a[0]);
+            ob.load(b[0]);
+            mul(a[1], b[1]);
+        }
+        if (chunks == 2) {
+            oa.load(a[1]);
+            ob.load(b[1]);
+        }
+        mul(a[0], b[0]);
+        if (chunks == 2) mul(a[1], b[1]);
+    }
+    if (left) {
+        oa.load_tail(a[0], left);
+        ob.load_tail(b[0], left);
+        mul(a[0], b[0]);
     }
 }
 
-// R_t = beta C0 - acc_t on rows < M, columns < N of tile t (columns 64 t..64 t+63
-// of C, element (r, c) at C[r + c ldc]), then C = Dinv(:, :M) R_t for the valid tiles
-__device__ __forceinline__ void strip2_finish(d4 (&acc)[2][4], double *lds, double *C, int ldc, int M, int N,
-                                              const double *Dinv, double beta, const bool (&valid)[2]) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+__device__ __forceinline__ void wave_zero(d4 (&acc)[4][4]) {
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        double dv[8];
+    for (int r = 0; r < 4; r++)
 #pragma unroll
-        for (int it = 0; it < 8; it++) dv[it] = gload(Dinv + tid + 256 * (8 * h + it));
+        for (int c = 0; c < 4; c++) acc[r][c] = d4{0.0, 0.0, 0.0, 0.0};
+}
+
+// acc = -C on rows < M, columns < N (zero elsewhere): the accumulators start from the
+// tile, whose loads fly beside the first operands'.  TR: element (r, c) of the tile is
+// C[c + r ldc], else C[r + c ldc].
+template <bool TR>
+__device__ __forceinline__ void wave_start(d4 (&acc)[4][4], const double *C, int ldc, int M, int N) {
+    const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
 #pragma unroll
-        for (int it = 0; it < 8; it++) {
-            const int e = tid + 256 * (8 * h + it), i = e & 63, k = e >> 6;
-            lds[k * (TILE + 1) + i] = k < M ? dv[it] : 0.0;
-        }
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int i = 16 * r + kq + 4 * v, j = 16 * c + l16;
+                const bool ok = i < M && j < N;
+                const double c0 = gload(C + (ok ? (TR ? j + (size_t)i * ldc : i + (size_t)j * ldc) : 0));
+                acc[r][c][v] = ok ? -c0 : 0.0;
+            }
+}
+
+// C = -Dinv acc on rows < M, columns < N, with acc = op(A) op(B) - C on entry and
+// +-C on return.  Dinv is a lower triangular 64 x 64 tile (column-major).  A lane's
+// accumulators are the B operand of the product (value v of row block r: the k-step
+// over rows 16 r + 4 v .. + 3), and the output blocks go from the last row block up,
+// so that each replaces an accumulator nothing reads any more.
+template <bool TR>
+__device__ __forceinline__ void wave_finish(d4 (&acc)[4][4], double *C, int ldc, int M, int N, const double *Dinv) {
+    const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
+    if (M < TILE || N < TILE) {  // rows and columns past the tile repeat its last ones
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    if (16 * r + kq + 4 * v >= M || 16 * c + l16 >= N) acc[r][c][v] = 0.0;
     }
 #pragma unroll
-    for (int t = 0; t < 2; t++) {
-        const int c = TILE * t + 16 * wave + (lane & 15);
+    for (int o = 3; o >= 0; o--) {
+        d4 out[4] = {d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}};
 #pragma unroll
-        for (int rbk = 0; rbk < 4; rbk++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int r = 16 * rbk + (lane >> 4) + 4 * v;
-                const bool ok = valid[t] && r < M && c < N;
-                const double c0 = (beta != 0.0) ? gload(C + (ok ? (size_t)r + (size_t)c * ldc : 0)) : 0.0;
-                acc[t][rbk][v] = ok ? beta * c0 - acc[t][rbk][v] : 0.0;
-            }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int ob = 0; ob < 4; ob++) {
-        d4 out[2] = {d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}};
-#pragma unroll
-        for (int rbk = 0; rbk < 4; rbk++)
+        for (int r = 0; r <= o; r++)
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const double a = lds[(16 * rbk + 4 * v + (lane >> 4)) * (TILE + 1) + 16 * ob + (lane & 15)];
+                const double x = gload(Dinv + (16 * r + 4 * v + kq) * TILE + 16 * o + l16);
 #pragma unroll
-                for (int t = 0; t < 2; t++) out[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, acc[t][rbk][v], out[t], 0, 0, 0);
+                for (int c = 0; c < 4; c++) out[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, acc[r][c][v], out[c], 0, 0, 0);
             }
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
-            const int c = TILE * t + 16 * wave + (lane & 15);
+        for (int c = 0; c < 4; c++) {
+            acc[o][c] = out[c];
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const int r = 16 * ob + (lane >> 4) + 4 * v;
-                if (valid[t] && r < M && c < N) C[(size_t)r + (size_t)c * ldc] = out[t][v];
+                const int i = 16 * o + kq + 4 * v, j = 16 * c + l16;
+                if (i < M && j < N) C[TR ? j + (size_t)i * ldc : i + (size_t)j * ldc] = -out[c][v];
             }
         }
     }
@@ -441,13 +520,15 @@ __device__ __forceinline__ void xcd_tile(int &bx, int &by) {
 }
 
 // the factored matrix A (n x n, leading dimension lda) and the right-hand
-// sides B (n x ncols, leading dimension n) of a stage
+// sides B (n x ncols, leading dimension ldb) of a stage
 __device__ __forceinline__ void pick(const DenseDesc &d, int which, double *&A, int &lda, int &n, int &band, int &nt,
-                                     double *&B, int &ncols, int &ntc) {
+                                     double *&B, int &ldb, int &ncols, int &ntc) {
     if (which == 0) {
-        A = d.Kii; lda = d.ldk; n = d.ni; band = d.band_ii; nt = d.ntii; B = d.Kib; ncols = d.m + 1; ntc = d.ntc;
+        A = d.Kii; lda = d.ldk; n = d.ni; band = d.band_ii; nt = d.ntii;
+        B = d.Kib; ldb = d.ldb; ncols = d.m + 1; ntc = d.ntc;
     } else {
-        A = d.S; lda = d.m; n = d.m; band = d.ntm; nt = d.ntm; B = d.W; ncols = d.m; ntc = d.ntm;
+        A = d.S; lda = d.lds; n = d.m; band = d.ntm; nt = d.ntm;
+        B = d.W; ldb = d.lds; ncols = d.m; ntc = d.ntm;
     }
 }
 
@@ -476,8 +557,8 @@ __device__ __forceinline__ double read_lane(double v, int lane) {
 __global__ void __launch_bounds__(256, 4) k_potrf_diag(const DenseDesc *D, int which, int step) {
     const DenseDesc &d = D[blockIdx.x];
     double *A, *B;
-    int lda, n, band, nt, ncols, ntc;
-    pick(d, which, A, lda, n, band, nt, B, ncols, ntc);
+    int lda, n, band, nt, ldb, ncols, ntc;
+    pick(d, which, A, lda, n, band, nt, B, ldb, ncols, ntc);
     const int k0 = step * TILE;
     if (k0 >= n) return;
     const int nb = min(TILE, n - k0);
@@ -615,7 +696,7 @@ __global__ void __launch_bounds__(256) k_potrf_panel_rl(const DenseDesc *D, int 
     int bx, by;
     xcd_tile(bx, by);
     const DenseDesc &d = D[by];
-    const int nt = d.ntm, n = d.m, lda = d.m;
+    const int nt = d.ntm, n = d.m, lda = d.lds;
     const int i = step + 1 + bx;
     if (i >= nt) return;
     const int k0 = step * TILE, i0 = i * TILE;
@@ -637,7 +718,7 @@ __global__ void __launch_bounds__(256) k_potrf_trail(const DenseDesc *D, int ste
     const int J = q - I * (I + 1) / 2;
     const int i = step + 1 + I, j = step + 1 + J;
     if (i >= d.ntm) return;
-    const int n = d.m, lda = d.m, k0 = step * TILE, i0 = i * TILE, j0 = j * TILE;
+    const int n = d.m, lda = d.lds, k0 = step * TILE, i0 = i * TILE, j0 = j * TILE;
     const int nb = min(TILE, n - k0), mi = min(TILE, n - i0), mj = min(TILE, n - j0);
     tile_gemm<false, true>(d.S + i0 + (size_t)j0 * lda, lda, d.S + i0 + (size_t)k0 * lda, lda,
                            d.S + j0 + (size_t)k0 * lda, lda, mi, mj, nb, -1.0, 1.0);
@@ -648,8 +729,8 @@ __global__ void __launch_bounds__(256) k_potrf_panel(const DenseDesc *D, int whi
     xcd_tile(bx, by);
     const DenseDesc &d = D[by];
     double *A, *B;
-    int lda, n, band, nt, ncols, ntc;
-    pick(d, which, A, lda, n, band, nt, B, ncols, ntc);
+    int lda, n, band, nt, ldb, ncols, ntc;
+    pick(d, which, A, lda, n, band, nt, B, ldb, ncols, ntc);
     const int i = step + 1 + bx;
     if (i >= nt || i > step + band) return;
     const int k0 = step * TILE, i0 = i * TILE;
@@ -668,67 +749,58 @@ __global__ void __launch_bounds__(256) k_potrf_panel(const DenseDesc *D, int whi
     diag_update(o, lds, A + i0 + (size_t)i0 * lda, lda, mi);
 }
 
+// the same, one wave per panel tile: the diagonal update takes -L from the
+// accumulators (value v of acc[r][c] is L(16 c + l16, 16 r + kq + 4 v), an A and a B
+// operand of the k-step over columns 16 r + 4 v .. + 3)
+__global__ void __launch_bounds__(64, 2) k_potrf_panel_w(const DenseDesc *D, int which, int step) {
+    int bx, by;
+    xcd_tile(bx, by);
+    const DenseDesc &d = D[by];
+    double *A, *B;
+    int lda, n, band, nt, ldb, ncols, ntc;
+    pick(d, which, A, lda, n, band, nt, B, ldb, ncols, ntc);
+    const int i = step + 1 + bx;
+    if (i >= nt || i > step + band) return;
+    const int k0 = step * TILE, i0 = i * TILE;
+    const int nb = min(TILE, n - k0), mi = min(TILE, n - i0);
+    const int j0 = max(0, i - band) * TILE;
+    d4 acc[4][4];
+    double *C = A + i0 + (size_t)k0 * lda;
+    wave_start<true>(acc, C, lda, nb, mi);
+    if (k0 > j0)
+        wave_gemm<false, false>(acc, A + k0 + (size_t)j0 * lda, lda, A + i0 + (size_t)j0 * lda, lda, nb, mi, k0 - j0);
+    wave_finish<true>(acc, C, lda, nb, mi, d.Dinv + (size_t)step * TILE * TILE);
+    double *Aii = A + i0 + (size_t)i0 * lda;
+    const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
+#pragma unroll
+    for (int ib = 0; ib < 4; ib++)
+#pragma unroll
+        for (int jb = 0; jb <= ib; jb++) {
+            d4 s = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    s = __builtin_amdgcn_mfma_f64_16x16x4f64(acc[r][ib][v], acc[r][jb][v], s, 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int p = 16 * ib + kq + 4 * v, q = 16 * jb + l16;
+                if (p < mi && q < mi) Aii[p + (size_t)q * lda] -= s[v];
+            }
+        }
+}
+
 // ---- left-looking forward substitution X = L^-1 B, block row i ----
 // X_iJ = inv(L_ii) (B_iJ - L_iw X_wJ), window w = [max(first nonzero tile of
 // column tile J, i - band), i)
-__global__ void __launch_bounds__(256, 3) k_trsm_row(const DenseDesc *D, int which, int step) {
+// four waves per tile (few tiles)
+__global__ void __launch_bounds__(256, 4) k_trsm_row(const DenseDesc *D, int which, int step) {
     int bx, by;
     xcd_tile(bx, by);
     const DenseDesc &d = D[by];
     double *A, *B;
-    int lda, n, band, nt, ncols, ntc;
-    pick(d, which, A, lda, n, band, nt, B, ncols, ntc);
-    const int J0 = 2 * bx, i = step;
-    if (J0 >= ntc || i >= nt) return;
-    const int i0 = i * TILE, c0 = J0 * TILE;
-    const int mi = min(TILE, n - i0), N = min(2 * TILE, ncols - c0);
-    const double *Di = d.Dinv + (size_t)i * TILE * TILE;
-    bool valid[2];
-    int jst[2], jmin = n;
-#pragma unroll
-    for (int t = 0; t < 2; t++) {
-        const int J = J0 + t;
-        valid[t] = J < ntc;
-        const int cs = which == 0 ? (valid[t] ? d.colstart[J] : i + 1) : J;
-        if (cs > i) valid[t] = false;
-        if (valid[t] && which == 1 && J == i) {
-            // W = L^-1 I: the right-hand side is the identity, so the diagonal tile is inv(L_ii)
-            const int nj = min(TILE, ncols - J * TILE);
-            double *Cd = B + i0 + (size_t)J * TILE * n;
-            for (int q = threadIdx.x; q < TILE * TILE; q += 256) {
-                const int r = q & 63, c = q >> 6;
-                if (r < mi && c < nj) Cd[r + (size_t)c * n] = Di[q];
-            }
-            valid[t] = false;
-        }
-        jst[t] = max(cs, i - band) * TILE;
-        if (valid[t]) jmin = min(jmin, jst[t]);
-    }
-    if (!valid[0] && !valid[1]) return;  // uniform over the workgroup
-    __shared__ double lds[FUSED2_LDS];
-    d4 acc[2][4];
-#pragma unroll
-    for (int t = 0; t < 2; t++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) acc[t][r] = d4{0.0, 0.0, 0.0, 0.0};
-    double *C = B + i0 + (size_t)c0 * n;
-    if (i0 > jmin) {
-        const int kfirst[2] = {valid[0] ? jst[0] - jmin : i0 - jmin, valid[1] ? jst[1] - jmin : i0 - jmin};
-        strip2_gemm(acc, lds, A + i0 + (size_t)jmin * lda, lda, B + jmin + (size_t)c0 * n, n, mi, N, i0 - jmin,
-                    kfirst);
-    }
-    // which 1: the identity has no entries off the diagonal tile (beta 0)
-    strip2_finish(acc, lds, C, n, mi, N, Di, which == 1 ? 0.0 : 1.0, valid);
-}
-
-// one column tile per workgroup (few subdomains: twice the workgroups of the pairs)
-__global__ void __launch_bounds__(256, 4) k_trsm_row1(const DenseDesc *D, int which, int step) {
-    int bx, by;
-    xcd_tile(bx, by);
-    const DenseDesc &d = D[by];
-    double *A, *B;
-    int lda, n, band, nt, ncols, ntc;
-    pick(d, which, A, lda, n, band, nt, B, ncols, ntc);
+    int lda, n, band, nt, ldb, ncols, ntc;
+    pick(d, which, A, lda, n, band, nt, B, ldb, ncols, ntc);
     const int J = bx, i = step;
     if (J >= ntc || i >= nt) return;
     const int cs = which == 0 ? d.colstart[J] : J;
@@ -736,23 +808,90 @@ __global__ void __launch_bounds__(256, 4) k_trsm_row1(const DenseDesc *D, int wh
     const int i0 = i * TILE, c0 = J * TILE;
     const int mi = min(TILE, n - i0), nj = min(TILE, ncols - c0);
     const int j0 = max(cs, i - band) * TILE;
-    double *C = B + i0 + (size_t)c0 * n;
+    double *C = B + i0 + (size_t)c0 * ldb;
     if (which == 1 && J == i) {
         // W = L^-1 I: the right-hand side is the identity, so the diagonal tile is inv(L_ii)
         const double *Di = d.Dinv + (size_t)i * TILE * TILE;
         for (int q = threadIdx.x; q < TILE * TILE; q += 256) {
             const int r = q & 63, c = q >> 6;
-            if (r < mi && c < nj) C[r + (size_t)c * n] = Di[q];
+            if (r < mi && c < nj) C[r + (size_t)c * ldb] = Di[q];
         }
         return;
     }
     __shared__ double lds[FUSED_LDS];
     d4 acc[4] = {d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}};
     if (i0 > j0)
-        strip_gemm<false, false>(acc, lds, A + i0 + (size_t)j0 * lda, lda, B + j0 + (size_t)c0 * n, n, mi, nj,
+        strip_gemm<false, false>(acc, lds, A + i0 + (size_t)j0 * lda, lda, B + j0 + (size_t)c0 * ldb, ldb, mi, nj,
                                  i0 - j0);
     // which 1: the identity has no entries off the diagonal tile (beta 0)
-    strip_finish<false>(acc, lds, C, n, mi, nj, d.Dinv + (size_t)i * TILE * TILE, which == 1 ? 0.0 : 1.0);
+    strip_finish<false>(acc, lds, C, ldb, mi, nj, d.Dinv + (size_t)i * TILE * TILE, which == 1 ? 0.0 : 1.0);
+}
+
+// one tile per wave
+__global__ void __launch_bounds__(64, 2) k_trsm_row_w(const DenseDesc *D, int which, int step) {
+    int bx, by;
+    xcd_tile(bx, by);
+    const DenseDesc &d = D[by];
+    double *A, *B;
+    int lda, n, band, nt, ldb, ncols, ntc;
+    pick(d, which, A, lda, n, band, nt, B, ldb, ncols, ntc);
+    const int J = bx, i = step;
+    if (J >= ntc || i >= nt) return;
+    const int cs = which == 0 ? d.colstart[J] : J;
+    if (cs > i) return;
+    const int i0 = i * TILE, c0 = J * TILE;
+    const int mi = min(TILE, n - i0), nj = min(TILE, ncols - c0);
+    const int j0 = max(cs, i - band) * TILE;
+    double *C = B + i0 + (size_t)c0 * ldb;
+    const double *Di = d.Dinv + (size_t)i * TILE * TILE;
+    if (which == 1 && J == i) {
+        // W = L^-1 I: the right-hand side is the identity, so the diagonal tile is inv(L_ii)
+        for (int c = 0; c < nj; c++)
+            if ((int)threadIdx.x < mi) C[threadIdx.x + (size_t)c * ldb] = Di[threadIdx.x + c * TILE];
+        return;
+    }
+    d4 acc[4][4];
+    // which 1: the identity has no entries off the diagonal tile
+    if (which == 1) wave_zero(acc);
+    else wave_start<false>(acc, C, ldb, mi, nj);
+    if (i0 > j0)
+        wave_gemm<false, true>(acc, A + i0 + (size_t)j0 * lda, lda, B + j0 + (size_t)c0 * ldb, ldb, mi, nj, i0 - j0);
+    wave_finish<false>(acc, C, ldb, mi, nj, Di);
+}
+
+// lower tiles of the products below, one per wave.  The operands are swapped (the
+// accumulator rows are the tile's columns), so that the 16 lanes of a store write 16
+// consecutive rows of a column.
+__global__ void __launch_bounds__(64, 2) k_syrk_w(const DenseDesc *D, int which) {
+    int bx, by;
+    xcd_tile(bx, by);
+    const DenseDesc &d = D[by];
+    const int q = bx;
+    int I = (int)((sqrtf(8.0f * q + 1.0f) - 1.0f) * 0.5f);
+    while ((I + 1) * (I + 2) / 2 <= q) I++;
+    while (I * (I + 1) / 2 > q) I--;
+    const int J = q - I * (I + 1) / 2;
+    if (I >= d.ntm) return;
+    const int m = d.m, i0 = I * TILE, j0 = J * TILE;
+    const int mi = min(TILE, m - i0), mj = min(TILE, m - j0);
+    const double *Y = which == 0 ? d.Kib : d.W;
+    const int ld = which == 0 ? d.ldb : d.lds, n = which == 0 ? d.ni : m;
+    const int ks = which == 0 ? min(max(d.colstart[I], d.colstart[J]) * TILE, d.ni) : i0;
+    const double sign = which == 0 ? -1.0 : 1.0;
+    d4 acc[4][4];
+    wave_zero(acc);
+    wave_gemm<true, true>(acc, Y + ks + (size_t)j0 * ld, ld, Y + ks + (size_t)i0 * ld, ld, mj, mi, n - ks);
+    const int lane = threadIdx.x & 63, l16 = lane & 15, kq = lane >> 4;
+    double *C = d.S + i0 + (size_t)j0 * d.lds;
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int i = 16 * c + l16, j = 16 * r + kq + 4 * v;
+                if (i < mi && j < mj) C[i + (size_t)j * d.lds] = sign * acc[r][c][v];
+            }
 }
 
 // lower tiles of  S = -Y^T Y  (which 0)  or  S = W^T W  (which 1)
@@ -768,18 +907,18 @@ __global__ void __launch_bounds__(256) k_syrk(const DenseDesc *D, int which) {
     if (I >= d.ntm) return;
     const int m = d.m, i0 = I * TILE, j0 = J * TILE;
     const int mi = min(TILE, m - i0), mj = min(TILE, m - j0);
-    double *C = d.S + i0 + (size_t)j0 * m;
+    double *C = d.S + i0 + (size_t)j0 * d.lds;
     if (which == 0) {
         // S = -Y^T Y (K_bb is added by k_add_kbb); a tile with no coupled
         // interior rows (K = 0) is written as zeros
         const int ks = min(max(d.colstart[I], d.colstart[J]) * TILE, d.ni);
         const double *Y = d.Kib;
-        tile_gemm<true, false>(C, m, Y + ks + (size_t)i0 * d.ni, d.ni, Y + ks + (size_t)j0 * d.ni, d.ni, mi, mj,
-                               d.ni - ks, -1.0, 0.0);
+        tile_gemm<true, false>(C, d.lds, Y + ks + (size_t)i0 * d.ldb, d.ldb, Y + ks + (size_t)j0 * d.ldb, d.ldb, mi,
+                               mj, d.ni - ks, -1.0, 0.0);
     } else {
         int ks = i0;  // W is lower triangular: rows < max(I,J)*64 of these columns vanish
-        tile_gemm<true, false>(C, m, d.W + ks + (size_t)i0 * m, m, d.W + ks + (size_t)j0 * m, m, mi, mj, m - ks,
-                               1.0, 0.0);
+        tile_gemm<true, false>(C, d.lds, d.W + ks + (size_t)i0 * d.lds, d.lds, d.W + ks + (size_t)j0 * d.lds, d.lds,
+                               mi, mj, m - ks, 1.0, 0.0);
     }
 }
 
@@ -803,10 +942,10 @@ __global__ void __launch_bounds__(256) k_trtri_diag(const DenseDesc *D) {
     if (i >= d.ntm) return;
     const int r0 = i * TILE, mi = min(TILE, d.m - r0);
     const double *Di = d.Dinv + (size_t)i * TILE * TILE;
-    double *W = d.W + r0 + (size_t)r0 * d.m;
+    double *W = d.W + r0 + (size_t)r0 * d.lds;
     for (int q = threadIdx.x; q < TILE * TILE; q += 256) {
         const int r = q & 63, c = q >> 6;
-        if (r < mi && c < mi) W[r + (size_t)c * d.m] = Di[q];
+        if (r < mi && c < mi) W[r + (size_t)c * d.lds] = Di[q];
     }
 }
 
@@ -814,7 +953,7 @@ __global__ void __launch_bounds__(256) k_trtri_level(const DenseDesc *D, int t, 
     int bx, by;
     xcd_tile(bx, by);
     const DenseDesc &d = D[by];
-    const int nt = d.ntm, m = d.m, tt = t * t;
+    const int nt = d.ntm, m = d.m, ld = d.lds, tt = t * t;
     const int p = bx / tt, i = (bx % tt) / t, j = bx % t;  // pair, tile row in block 2, tile column in block 1
     const int b1 = 2 * t * p, b2 = b1 + t;
     if (b2 + i >= nt) return;
@@ -822,12 +961,12 @@ __global__ void __launch_bounds__(256) k_trtri_level(const DenseDesc *D, int t, 
     const int mi = min(TILE, m - r2);
     if (phase == 0) {
         // T(r2.., c1..) = L(r2.., c1..k2) W(c1..k2, c1..), stored as S[c1 + x, r2 + y] = T(y, x)
-        tile_gemm<true, true>(d.S + c1 + (size_t)r2 * m, m, d.W + c1 + (size_t)c1 * m, m, d.S + r2 + (size_t)c1 * m, m,
-                              TILE, mi, k2 - c1, 1.0, 0.0);
+        tile_gemm<true, true>(d.S + c1 + (size_t)r2 * ld, ld, d.W + c1 + (size_t)c1 * ld, ld,
+                              d.S + r2 + (size_t)c1 * ld, ld, TILE, mi, k2 - c1, 1.0, 0.0);
     } else {
         // W(r2.., c1..) = -W(r2.., k2..r2+mi) T(k2..r2+mi, c1..)
-        tile_gemm<false, true>(d.W + r2 + (size_t)c1 * m, m, d.W + r2 + (size_t)k2 * m, m, d.S + c1 + (size_t)k2 * m, m,
-                               mi, TILE, r2 + mi - k2, -1.0, 0.0);
+        tile_gemm<false, true>(d.W + r2 + (size_t)c1 * ld, ld, d.W + r2 + (size_t)k2 * ld, ld,
+                               d.S + c1 + (size_t)k2 * ld, ld, mi, TILE, r2 + mi - k2, -1.0, 0.0);
     }
 }
 
@@ -966,7 +1105,7 @@ __device__ __forceinline__ double block_max(double v) {
 __global__ void k_rho(const DenseDesc *D, double *rho) {
     const DenseDesc &d = D[blockIdx.x];
     double v = 0.0;
-    for (int i = threadIdx.x; i < d.m; i += 256) v = fmax(v, d.S[i + (size_t)i * d.m]);
+    for (int i = threadIdx.x; i < d.m; i += 256) v = fmax(v, d.S[i + (size_t)i * d.lds]);
     v = block_max(v);
     if (threadIdx.x == 0) rho[blockIdx.x] = v;
 }
@@ -1003,7 +1142,7 @@ __global__ void __launch_bounds__(256) k_kernel_reg(const DenseDesc *D, const do
 #pragma unroll
         for (int a = 0; a < KR; a++) s += qr[a][x] * qc[a][y];
         for (int a = KR; a < k; a++) s += q[i + (size_t)a * m] * q[j + (size_t)a * m];
-        d.S[i + (size_t)j * m] += r * s;
+        d.S[i + (size_t)j * d.lds] += r * s;
     }
 }
 
@@ -1013,8 +1152,8 @@ __global__ void k_hf(const DenseDesc *D, const double *fb, double *hf, const int
     const int lane = threadIdx.x & 63;
     const int j = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (j >= d.m) return;
-    const double *y = d.Kib + (size_t)j * d.ni;
-    const double *yf = d.Kib + (size_t)d.m * d.ni;
+    const double *y = d.Kib + (size_t)j * d.ldb;
+    const double *yf = d.Kib + (size_t)d.m * d.ldb;
     double s = 0.0;
     // Y(:, j) is zero above its column tile's first coupled row (not stored)
     for (int r = d.colstart[j / TILE] * TILE + lane; r < d.ni; r += 64) s += y[r] * yf[r];
@@ -1034,7 +1173,7 @@ __global__ void k_absmax(const DenseDesc *D, float *scale) {
     const int64_t mm = (int64_t)d.m * d.m;
     for (int64_t e = threadIdx.x; e < mm; e += 256) {
         int i = (int)(e % d.m), j = (int)(e / d.m);
-        if (i >= j) v = fmax(v, fabs(d.S[e]));
+        if (i >= j) v = fmax(v, fabs(d.S[i + (size_t)j * d.lds]));
     }
     v = block_max(v);
     if (threadIdx.x == 0) scale[blockIdx.x] = v > 0.0 ? (float)v : 1.0f;
@@ -1050,7 +1189,7 @@ __global__ void k_absmax(const DenseDesc *D, float *scale) {
 // starts at zero.
 __global__ void __launch_bounds__(256) k_rownorm(const DenseDesc *D, double *nrm) {
     const DenseDesc &d = D[blockIdx.y];
-    const int m = d.m;
+    const int m = d.m, ld = d.lds;
     const int c0 = blockIdx.x * 256;
     if (c0 >= m) return;
     __shared__ double below[256], wm[4];
@@ -1060,7 +1199,7 @@ __global__ void __launch_bounds__(256) k_rownorm(const DenseDesc *D, double *nrm
         const int c = c0 + q;
         double v = 0.0;
         if (c < m)
-            for (int i = c + 1 + lane; i < m; i += 64) v += fabs(S[i + (size_t)c * m]);
+            for (int i = c + 1 + lane; i < m; i += 64) v += fabs(S[i + (size_t)c * ld]);
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
         if (lane == 0) below[q] = v;
@@ -1069,7 +1208,7 @@ __global__ void __launch_bounds__(256) k_rownorm(const DenseDesc *D, double *nrm
     const int c = c0 + tid;
     double r = 0.0;
     if (c < m) {
-        for (int k = 0; k <= c; k++) r += fabs(S[c + (size_t)k * m]);
+        for (int k = 0; k <= c; k++) r += fabs(S[c + (size_t)k * ld]);
         r += below[tid];
     }
 #pragma unroll
@@ -1109,7 +1248,7 @@ __global__ void k_pack(const DenseDesc *D, T *pool, const int64_t *off, const fl
             const int row = r0 + g * VEC + u;
             double v = 0.0;
             if (row < m && row <= c) {
-                v = d.S[c + (size_t)row * m];
+                v = d.S[c + (size_t)row * d.lds];
                 if (row == c) v *= 0.5;
             }
             v *= inv;
@@ -1132,7 +1271,7 @@ __global__ void k_band_extract(const DenseDesc *D, double *band, const int64_t *
         dst[e] = (c + dd < d.ni) ? d.Kii[(c + dd) + (size_t)c * d.ldk] : 0.0;
     }
     for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < d.ni; r += (int64_t)gridDim.x * blockDim.x)
-        yf[yf_off[blockIdx.y] + r] = d.Kib[r + (size_t)d.m * d.ni];
+        yf[yf_off[blockIdx.y] + r] = d.Kib[r + (size_t)d.m * d.ldb];
 }
 
 template <int R, typename T>
@@ -1181,7 +1320,7 @@ __global__ void __launch_bounds__(256) k_materialize(const DenseDesc *D, const i
     const int *ip = iperm + perm_off[b];
     const int *pm = perm + perm_off[b];
     if (c == n) {  // f column, permuted
-        double *dst = d.Kib + (size_t)m * ni;
+        double *dst = d.Kib + (size_t)m * d.ldb;
         for (int r = lane; r < ni; r += 64) dst[r] = f[perm_off[b] + pm[r]];
         return;
     }
@@ -1212,7 +1351,7 @@ __global__ void __launch_bounds__(256) k_materialize(const DenseDesc *D, const i
             if (pr >= w0 && pr < w1) cb[pr - w0] = kv[q];
         }
         wave_lds_sync();
-        double *dst = c < ni ? d.Kii + (size_t)c * d.ldk : d.Kib + (size_t)(c - ni) * ni;
+        double *dst = c < ni ? d.Kii + (size_t)c * d.ldk : d.Kib + (size_t)(c - ni) * d.ldb;
         for (int r = w0 + lane; r < w1; r += 64) dst[r] = cb[r - w0];
         wave_lds_sync();  // the window is read before the next one clears it
     }
@@ -1235,7 +1374,7 @@ __global__ void __launch_bounds__(256) k_add_kbb(const DenseDesc *D, const int *
     const int *ip = iperm + perm_off[b];
     const int l = perm[perm_off[b] + ni + j];
     const int s0 = ni + (j / TILE) * TILE;  // first S row of the column's lower tiles, permuted
-    double *col = d.S + (size_t)j * m - ni;
+    double *col = d.S + (size_t)j * d.lds - ni;
     for (int q = rp[l] + lane; q < rp[l + 1]; q += 64) {
         const int pr = ip[ci[q]];
         if (pr >= s0) col[pr] += kv[q];
@@ -1259,7 +1398,7 @@ __global__ void k_b0_columns(const DenseDesc *D, const int *nq, const int64_t *q
         double v = 0.0;
         for (int64_t k = qe_ptr[slot]; k < qe_ptr[slot + 1]; k++) {
             const int c = qe_j[k];
-            v += qe_c[k] * ((sym || j >= c) ? d.S[j + (size_t)c * m] : d.S[c + (size_t)j * m]);
+            v += qe_c[k] * ((sym || j >= c) ? d.S[j + (size_t)c * d.lds] : d.S[c + (size_t)j * d.lds]);
         }
         fb[e] = v;
     }
@@ -1290,7 +1429,7 @@ __global__ void k_symmetrize_desc(const DenseDesc *D) {
     const int64_t nn = (int64_t)m * m;
     for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < nn; e += (int64_t)gridDim.x * blockDim.x) {
         const int i = (int)(e % m), j = (int)(e / m);
-        if (i < j) d.S[e] = d.S[j + (int64_t)i * m];
+        if (i < j) d.S[i + (int64_t)j * d.lds] = d.S[j + (int64_t)i * d.lds];
     }
 }
 
@@ -1429,6 +1568,17 @@ void launch_probe_gemm(int ta, int tb, int M, int N, int K, const double *A, int
 // ------------------------------------------------------------ launchers ----
 static inline unsigned cdiv(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
 
+// From how many tiles a launch takes one wave per tile instead of a workgroup of
+// four.  Two waves fit a SIMD (2048 tiles fill the GPU once) and a tile's serial
+// time is four times longer, so few tiles lose.  Assembly times, wave tiles in that
+// kernel / four-wave tiles: substitution 8 subdomains of 12^3 elasticity (328 tiles)
+// 23.5 / 18.6 ms, 64 of 12^3 heat (900) 7.6 / 6.8, 64 of 10^3 elasticity (1700)
+// 24.2 / 24.1, 216 of 7^3 (3900) 10.7 / 11.2, 512 of 8^3 heat (4000) 4.95 / 5.8;
+// panel 8 of 12^3 (40-330) 23.5 / 21.3, 64 of 12^3 heat (190-900) 7.6 / 7.0, 512 of
+// 8^3 heat (1500) 4.95 / 5.2; SYRK 64 of 5^3 (2900) 2.4 / 2.2, 8 of 12^3 (6900)
+// 23.5 / 23.3, 64 of 10^3 (21 thousand) 24.2 / 25.0, 216 of 12^3 156 / 173.
+constexpr int64_t WAVE_TRSM = 2048, WAVE_PANEL = 1024, WAVE_SYRK = 8192;
+
 void launch_widen_runs(const uint16_t *img, const int64_t *pos, const int64_t *off, int nsub, int64_t max_n, int *d,
                        hipStream_t st) {
     if (nsub <= 0 || max_n <= 0) return;
@@ -1469,8 +1619,13 @@ void launch_potrf_diag(const DenseDesc *desc, int nb, int which, int step, hipSt
 }
 
 void launch_potrf_panel(const DenseDesc *desc, int nb, int which, int step, int max_band, hipStream_t st) {
-    if (max_band <= 0) return;
-    hipLaunchKernelGGL(k_potrf_panel, dim3(max_band, nb), dim3(256), 0, st, desc, which, step);
+    // which 1: the band is the whole matrix, rows below the diagonal tile
+    const int rows = which == 1 ? max_band - 1 - step : max_band;
+    if (rows <= 0) return;
+    if ((int64_t)rows * nb >= WAVE_PANEL)
+        hipLaunchKernelGGL(k_potrf_panel_w, dim3(rows, nb), dim3(64), 0, st, desc, which, step);
+    else
+        hipLaunchKernelGGL(k_potrf_panel, dim3(rows, nb), dim3(256), 0, st, desc, which, step);
 }
 
 void launch_potrf_rl(const DenseDesc *desc, int nb, int max_ntm, hipStream_t st) {
@@ -1483,19 +1638,15 @@ void launch_potrf_rl(const DenseDesc *desc, int nb, int max_ntm, hipStream_t st)
     }
 }
 
-void launch_potrf_step(const DenseDesc *desc, int nb, int which, int step, int max_band, hipStream_t st) {
-    launch_potrf_diag(desc, nb, which, step, st);
-    launch_potrf_panel(desc, nb, which, step, max_band, st);
-}
-
 void launch_trsm_step(const DenseDesc *desc, int nb, int which, int step, int max_band, int max_ntc,
                       hipStream_t st) {
     (void)max_band;
-    // pairs of column tiles when they still fill the GPU (256 CUs, 3 workgroups each)
-    if ((int64_t)nb * ((max_ntc + 1) / 2) >= 768)
-        hipLaunchKernelGGL(k_trsm_row, dim3((max_ntc + 1) / 2, nb), dim3(256), 0, st, desc, which, step);
+    // which 1: W is lower triangular, column tiles up to the block row
+    const int cols = which == 1 ? std::min(max_ntc, step + 1) : max_ntc;
+    if ((int64_t)cols * nb >= WAVE_TRSM)
+        hipLaunchKernelGGL(k_trsm_row_w, dim3(cols, nb), dim3(64), 0, st, desc, which, step);
     else
-        hipLaunchKernelGGL(k_trsm_row1, dim3(max_ntc, nb), dim3(256), 0, st, desc, which, step);
+        hipLaunchKernelGGL(k_trsm_row, dim3(cols, nb), dim3(256), 0, st, desc, which, step);
 }
 
 void launch_trtri(const DenseDesc *desc, int nb, int max_ntm, hipStream_t st) {
@@ -1508,7 +1659,11 @@ void launch_trtri(const DenseDesc *desc, int nb, int max_ntm, hipStream_t st) {
 }
 
 void launch_syrk(const DenseDesc *desc, int nb, int which, int max_ntm, hipStream_t st) {
-    hipLaunchKernelGGL(k_syrk, dim3(max_ntm * (max_ntm + 1) / 2, nb), dim3(256), 0, st, desc, which);
+    const int tiles = max_ntm * (max_ntm + 1) / 2;
+    if ((int64_t)tiles * nb >= WAVE_SYRK)
+        hipLaunchKernelGGL(k_syrk_w, dim3(tiles, nb), dim3(64), 0, st, desc, which);
+    else
+        hipLaunchKernelGGL(k_syrk, dim3(tiles, nb), dim3(256), 0, st, desc, which);
 }
 
 

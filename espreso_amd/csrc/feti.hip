@@ -729,6 +729,7 @@ struct espreso_feti_s {
     std::vector<StepGraph> step_graphs;
     double *asm_pool = nullptr;  // assembly workspace, reused by later set-ups
     size_t asm_pool_n = 0;
+    int asm_pad = 16;            // rows of [K_ib | f] and S rounded up to this many values
     std::vector<int> wave_plan;  // end subdomain of each assembly wave
     bool use_graphs = true;
     void compute_b();
@@ -1611,11 +1612,17 @@ void espreso_feti_s::assemble(const double *d_f, const double *d_Q, const std::v
     // per-subdomain workspace (doubles): K_ii in band storage, [K_ib | f], S,
     // W (in [K_ib | f]'s storage when it fits there), diagonal inverses
     auto kii_rows = [](const SubHost &h) { return std::min<int64_t>((int64_t)(h.band_tiles + 2) * TILE, h.ni + TILE); };
-    auto w_apart = [](const SubHost &h) { return (int64_t)h.m * h.m > (int64_t)h.ni * (h.m + 1); };
+    // columns of [K_ib | f], S and W start on 128-byte lines (asm_pad 16 values;
+    // 1, unpadded, when the device memory does not hold the padded workspace of
+    // the largest subdomain), the arrays themselves always do with the padding
+    auto up = [this](int64_t v) { return (v + asm_pad - 1) / asm_pad * asm_pad; };
+    auto ldb = [&](const SubHost &h) { return up(h.ni); };
+    auto lds = [&](const SubHost &h) { return up(h.m); };
+    auto w_apart = [&](const SubHost &h) { return lds(h) * h.m > ldb(h) * (h.m + 1); };
     auto ws = [&](const SubHost &h) {
         const int64_t nt = std::max((h.ni + TILE - 1) / TILE, (h.m + TILE - 1) / TILE);
-        return (int64_t)h.ni * kii_rows(h) + (int64_t)h.ni * (h.m + 1) + (int64_t)h.m * h.m +
-               (w_apart(h) ? (int64_t)h.m * h.m : 0) + nt * TILE * TILE;
+        return up((int64_t)h.ni * kii_rows(h)) + ldb(h) * (h.m + 1) + lds(h) * h.m + (w_apart(h) ? lds(h) * h.m : 0) +
+               nt * TILE * TILE;
     };
     // wave plan and workspace: planned once at the first set-up and kept
     // (re-planning and reallocating a multi-GB workspace costs more than the
@@ -1639,12 +1646,21 @@ void espreso_feti_s::assemble(const double *d_f, const double *d_Q, const std::v
         double budget = std::max(0.85 * ((double)freeb + pool_free), 0.85 * (double)totalb - (double)held_bytes);
         if (opt.memory_budget_gb > 0) budget = std::min(budget, opt.memory_budget_gb * 1e9);
         double need = 0, largest = 0;
-        for (int s = 0; s < nsub; s++) {
-            need += 8.0 * ws(sub[s]);
-            largest = std::max(largest, 8.0 * ws(sub[s]));
-        }
+        auto measure_need = [&] {
+            need = largest = 0;
+            for (int s = 0; s < nsub; s++) {
+                need += 8.0 * ws(sub[s]);
+                largest = std::max(largest, 8.0 * ws(sub[s]));
+            }
+        };
+        measure_need();
         budget = std::min(budget, need);
         for (;;) {
+            if (largest > budget && asm_pad > 1) {
+                asm_pad = 1;
+                measure_need();
+                budget = std::min(budget, need);
+            }
             ESP_CHECK(largest <= budget, ESPRESO_ERR_MEMORY,
                       "one subdomain's assembly workspace exceeds the device memory left");
             wave_plan.clear();
@@ -1690,10 +1706,12 @@ void espreso_feti_s::assemble(const double *d_f, const double *d_Q, const std::v
             d.ntc = (h.m + 1 + TILE - 1) / TILE;
             d.band_ii = h.band_tiles;
             d.ldk = (int)kii_rows(h) - 1;
-            d.Kii = cur + (TILE - 1); cur += (int64_t)h.ni * kii_rows(h);
-            d.Kib = cur; cur += (int64_t)h.ni * (h.m + 1);
-            d.S = cur; cur += (int64_t)h.m * h.m;
-            if (w_apart(h)) { d.W = cur; cur += (int64_t)h.m * h.m; }
+            d.ldb = (int)ldb(h);
+            d.lds = (int)lds(h);
+            d.Kii = cur + (TILE - 1); cur += up((int64_t)h.ni * kii_rows(h));
+            d.Kib = cur; cur += ldb(h) * (h.m + 1);
+            d.S = cur; cur += lds(h) * h.m;
+            if (w_apart(h)) { d.W = cur; cur += lds(h) * h.m; }
             else d.W = d.Kib;
             d.Dinv = cur; cur += (int64_t)std::max(d.ntii, d.ntm) * TILE * TILE;
             cs_off[b] = (int64_t)cs_all.size();
@@ -1857,6 +1875,7 @@ void espreso_feti_s::coarse() {
     d.info = info;
     d.ni = 0;
     d.m = nc;
+    d.lds = nc;
     d.ntm = nt;
     d.ntc = nt;
     DenseDesc *dd = upload(std::vector<DenseDesc>{d});
@@ -2934,6 +2953,7 @@ void espreso_feti_s::invert_spd_batched(double *pool, const std::vector<int64_t>
         d.info = info + b;
         d.ni = 0;
         d.m = n[i];
+        d.lds = n[i];
         d.ntm = d.ntc = (n[i] + TILE - 1) / TILE;
         wo += (int64_t)n[i] * n[i];
         dofs += (int64_t)d.ntm * TILE * TILE;

@@ -73,15 +73,18 @@ struct DenseDesc {
     // window the kernels read, address like a column-major matrix of leading
     // dimension ldk; the storage is ni (ldk + 1) values instead of ni^2.
     double *Kii;
-    double *Kib;          // ni x (m+1), ld ni: [K_ib | f_i]  ->  [Y | y_f] = L^-1 [K_ib | f_i]
-    double *S;            // m x m, ld m (lower): K_bb - Y^T Y -> + rho Q Q^T -> L_s -> F
-    double *W;            // m x m, ld m: L_s^-1 (lower tiles); may reuse Kib's storage
+    double *Kib;          // ni x (m+1), ld ldb: [K_ib | f_i]  ->  [Y | y_f] = L^-1 [K_ib | f_i]
+    double *S;            // m x m, ld lds (lower): K_bb - Y^T Y -> + rho Q Q^T -> L_s -> F
+    double *W;            // m x m, ld lds: L_s^-1 (lower tiles); may reuse Kib's storage
                           // (Y and y_f are no longer read once S_D and the band are out)
     double *Dinv;         // max(ntii, ntm) x 64 x 64: inverses of diagonal blocks
     const int *colstart;  // ntc: first tile row of a nonzero in each column tile of K_ib
     int *info;            // factorisation status (0 = ok, else 1-based failing column)
     int ni, m;
     int ldk;              // leading dimension of Kii (band storage, see above)
+    int ldb, lds;         // leading dimensions of Kib and of S and W: in the assembly ni and m
+                          // rounded up to 16, so that a column starts on a 128-byte line (the
+                          // wave tiles read four lanes' consecutive rows of a column as one line)
     int band_ii;          // block bandwidth of K_ii in tiles
     int ntii, ntm, ntc;   // tile counts: ceil(ni/64), ceil(m/64), ceil((m+1)/64)
 };
@@ -101,8 +104,7 @@ void launch_expand_sym(const double *img, const int64_t *pos, const int64_t *nz_
                        double *vals, int *err, hipStream_t st);
 void launch_copy_runs(const double *img, const int64_t *pos, const int64_t *off, int nsub, int64_t max_n, double *d,
                       hipStream_t st);
-void launch_potrf_step(const DenseDesc *desc, int nb, int which, int step, int max_band, hipStream_t st);
-// the two halves of a step: factor and invert the diagonal tile, then the panel below it
+// the two halves of a Cholesky step: factor and invert the diagonal tile, then the panel below it
 void launch_potrf_diag(const DenseDesc *desc, int nb, int which, int step, hipStream_t st);
 void launch_potrf_panel(const DenseDesc *desc, int nb, int which, int step, int max_band, hipStream_t st);
 // whole right-looking Cholesky of S (which 1) for a few large matrices: per

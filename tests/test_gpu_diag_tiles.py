@@ -75,3 +75,33 @@ def test_breakdown_column(col):
     with pytest.raises(RuntimeError, match=f"subdomain 1 at column {col + 1}$"):
         g.setup()
     g.close()
+
+
+# wave tiles take over from four waves per tile at 2048 substitution, 1024 panel and
+# 8192 SYRK tiles in a launch: 512 to 1000 subdomains whose interiors and interfaces
+# end just before, on and after a tile, checked in the first, an inner and the last one
+@pytest.mark.parametrize("physics,domains,elements", [
+    (1, (10, 10, 10), (6, 6, 6)), (1, (8, 8, 8), (7, 6, 5)), (0, (8, 8, 8), (3, 4, 4)), (0, (8, 8, 8), (5, 5, 4)),
+    (0, (6, 6, 6), (7, 7, 7))])
+def test_wave_tiles(physics, domains, elements):
+    spec = dict(row(physics, *elements), domains=domains, length=(1.0, 1.0, 1.0))
+    print("case: wave tiles", physics, domains, elements, flush=True)
+    n = int(np.prod(domains))
+    g = core.GridFETI(spec, preconditioner="dirichlet")
+    g.setup()
+    for i in (0, n // 2 + domains[0] // 2, n - 1):
+        d = core.grid_export(spec, i)
+        K = np.zeros((d["n"], d["n"]))
+        for r in range(d["n"]):
+            q = slice(d["rowptr"][r], d["rowptr"][r + 1])
+            K[r, d["colidx"][q]] = d["vals"][q]
+        b = g.boundary(i)
+        o = np.setdiff1d(np.arange(d["n"]), b)
+        S = K[np.ix_(b, b)] - K[np.ix_(b, o)] @ np.linalg.solve(K[np.ix_(o, o)], K[np.ix_(o, b)])
+        Q, _ = np.linalg.qr(d["R"][b])
+        F = np.linalg.inv(S + np.diag(S).max() * Q @ Q.T)
+        for which, want in ((1, S), (0, F)):
+            err = np.abs(g.dense(i, which) - want).max() / np.abs(want).max()
+            print(f"  subdomain {i}: interior {len(o)}, interface {len(b)}, {'S_D' if which else 'F'} {err:.1e}", flush=True)
+            assert err < 1e-9
+    g.close()
