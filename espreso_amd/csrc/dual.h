@@ -150,6 +150,15 @@ struct PrimalDev {
     int max_ni = 0;  // largest interior DOF count (host value: launch grids)
 };
 
+// structured grid on the device: node counts, subdomain counts, boxes (6 ints per
+// subdomain: first global element and elements per direction) and, per direction and
+// node index, the last subdomain slab holding the node and how many hold it
+struct GridDev {
+    int nd = 0, NN[3] = {0, 0, 0}, NS[3] = {0, 0, 0};
+    const int *box = nullptr, *subid = nullptr;  // subid: slab coordinates (x fastest) -> subdomain
+    const int *hi[3] = {nullptr, nullptr, nullptr}, *cnt[3] = {nullptr, nullptr, nullptr};
+};
+
 // y_b (D.yb) = A x_b for every subdomain; A = S_D (sd) or F_i in storage
 // precision `prec` (0 FP64, 1 FP32, 2 BF16).  x is lambda-space and gathered
 // with sign (or sign*scale when `scaled`) if `gather`, else boundary-space.
@@ -251,5 +260,16 @@ void launch_kkt_primal(const PrimalDev &P, int nsub, int max_n, const double *u,
 void launch_b0t(const DualDev &D, const ClusterDev &C, double *bt0, hipStream_t st);
 // u <- trunc(u D) / D (FETISolver::solve output truncation); partial: 256 doubles
 void launch_truncate(double *u, int64_t n, double precision, double *partial, hipStream_t st);
+
+// ---- nodal.hip: K cases at strides (uoff: offsets of the subdomains in f and u) ----
+// f = nodal load g split over the copies of a node (*bad: a value is not finite)
+void launch_nodal_split(const GridDev &G, int nsub, int max_n, int K, const int64_t *uoff, const double *g, int64_t gstr,
+                        double *f, int64_t fstr, int *bad, hipStream_t st);
+// g = sum (average) over the copies of the subdomain fields u
+void launch_nodal_gather(const GridDev &G, int K, const int64_t *uoff, const double *u, int64_t ustr, double *g,
+                         int64_t gstr, bool average, hipStream_t st);
+// e0f = -R_s^T f_s per subdomain and e (coarse right-hand side), interleaved by case
+void launch_rhs_dots(const PrimalDev &P, const DualDev &D, int K, const double *f, int64_t fstr, double *e0f, double *e,
+                     hipStream_t st);
 
 }  // namespace esp

@@ -734,8 +734,19 @@ struct espreso_feti_s {
     bool use_graphs = true;
     void compute_b();
     void compute_b_into(const double *hf, double *ubf, const double *e0f, double *b);
-    void rhs_host(const double *f, hvec<double> &e0f, std::vector<double> &e) const;
     void resolve_rhs();
+    // structured grid: tables and nodal scratch on the device (built at first use);
+    // nodal loads set on a loaded instance stay on the device (d_fnew) until the
+    // host copies sub[s].f are asked for
+    GridDev GD;
+    double *d_fnew = nullptr, *d_fspare = nullptr, *d_nodal = nullptr;
+    int *d_bad = nullptr;
+    int64_t n_nodal = 0;      // values d_nodal holds
+    bool loads_on_device = false;
+    void grid_device();
+    double *nodal_buffer(int64_t n);
+    void host_loads();
+    void set_nodal_rhs(const double *g);
     // block re-solve of several load cases (groups of up to 16)
     struct BlockBuffers {
         int K = 0;
@@ -770,12 +781,11 @@ struct espreso_feti_s {
     void factor_solve(const DenseDesc *desc, int nb, int which, int nt, int band, int ntc);
     void block_setup(int K);
     void apply_F_block(const PcgVec &V, const double *x, double *y, bool dot);
-    bool resolve_block(int nrhs, const double *f, double *u, int32_t *iters, double *norms,
+    // nodal: f and u are nodal fields of the structured grid, else subdomain fields
+    bool resolve_block(int nrhs, const double *f, double *u, int32_t *iters, double *norms, bool nodal,
                        espreso_feti_stats *stats);
-    void resolve_group(int K, const double *f, double *u, int32_t *iters, double *norms, espreso_feti_stats &tot);
-    std::vector<double> Ns_h;                        // hybrid: N_s per subdomain (kdim x kN)
-    std::vector<int64_t> noff_h;
-    std::vector<int> ccoff_h, cblk_h;                // coarse block offset, block of each subdomain
+    void resolve_group(int K, const double *f, double *u, int32_t *iters, double *norms, bool nodal,
+                       espreso_feti_stats &tot);
     int gridNE[3] = {0, 0, 0};                       // structured grid front end
     std::vector<double> gridKe0;
     bool grid_dev = false;                           // K_i values assembled on the device
@@ -1564,46 +1574,107 @@ void espreso_feti_s::compute_b_into(const double *hf, double *ubf, const double 
     launch_axpby(b, b, d_c, nlam, 1.0, -1.0, st);
 }
 
-// host part of new loads f (all subdomains, local order): e0f = -R_s^T f_s per
-// subdomain and the coarse right-hand side e (hybrid: per cluster through N_s)
-void espreso_feti_s::rhs_host(const double *f, hvec<double> &e0f, std::vector<double> &e) const {
-    e0f.assign(asubv[nsub], 0.0);
-#pragma omp parallel for schedule(dynamic, 16)
-    for (int s = 0; s < nsub; s++) {
-        const SubHost &h = sub[s];
-        const double *fs = f + uoff[s];
-        for (int a = 0; a < h.kdim; a++) {
-            double acc = 0;
-            for (int i = 0; i < h.n; i++) acc += h.R[i + (size_t)a * h.n] * fs[i];
-            e0f[asubv[s] + a] = -acc;
-        }
-    }
-    if (hybrid) {
-        e.assign(ncoarse, 0.0);
-        for (int s = 0; s < nsub; s++) {
-            const int c = cblk_h[s], kn = (int)((noff_h[s + 1] - noff_h[s]) / std::max(1, sub[s].kdim));
-            for (int b = 0; b < kn; b++)
-                for (int a = 0; a < sub[s].kdim; a++)
-                    e[ccoff_h[c] + b] += Ns_h[noff_h[s] + a + (int64_t)b * sub[s].kdim] * e0f[asubv[s] + a];
-        }
-    } else {
-        e.assign(e0f.begin(), e0f.end());
-    }
-}
-
-// New loads (host sub[s].f) on the assembled operators: e = -R^T f (hybrid:
-// per cluster through N_s), y_f and hf by interior band solves, b.
+// New loads (set by espreso_feti_set_rhs in sub[s].f, or nodal loads on the
+// device) on the assembled operators: e = -R^T f (hybrid: per cluster through
+// N_s), y_f and hf by interior band solves, b.
 void espreso_feti_s::resolve_rhs() {
-    std::vector<double> ff(uoff[nsub]);
-    for (int s = 0; s < nsub; s++) std::copy(sub[s].f.begin(), sub[s].f.end(), ff.begin() + uoff[s]);
-    std::vector<double> e;
-    rhs_host(ff.data(), e0f_h, e);
-    ESP_HIP(hipMemcpyAsync(d_f, ff.data(), ff.size() * sizeof(double), hipMemcpyHostToDevice, st));
-    ESP_HIP(hipMemcpyAsync(d_e0f, e0f_h.data(), e0f_h.size() * sizeof(double), hipMemcpyHostToDevice, st));
-    ESP_HIP(hipMemcpyAsync(d_e, e.data(), e.size() * sizeof(double), hipMemcpyHostToDevice, st));
+    std::vector<double> ff;
+    if (loads_on_device) {
+        ESP_HIP(hipMemcpyAsync(d_f, d_fnew, uoff[nsub] * sizeof(double), hipMemcpyDeviceToDevice, st));
+    } else {
+        ff.resize(uoff[nsub]);
+        for (int s = 0; s < nsub; s++) std::copy(sub[s].f.begin(), sub[s].f.end(), ff.begin() + uoff[s]);
+        ESP_HIP(hipMemcpyAsync(d_f, ff.data(), ff.size() * sizeof(double), hipMemcpyHostToDevice, st));
+    }
+    launch_rhs_dots(P, D, 1, d_f, 0, d_e0f, d_e, st);
     launch_rhs_prepare(P, nsub, d_f, d_hf, st);
     compute_b();
     sync();
+}
+
+// tables of the structured grid: per direction the slab coordinates of the
+// subdomain boxes give the owners of every node index
+void espreso_feti_s::grid_device() {
+    if (GD.nd) return;
+    std::vector<int> start[3];
+    for (int d = 0; d < 3; d++) {
+        for (int s = 0; s < nsub; s++) start[d].push_back(grid_box[6 * (size_t)s + d]);
+        std::sort(start[d].begin(), start[d].end());
+        start[d].erase(std::unique(start[d].begin(), start[d].end()), start[d].end());
+    }
+    GridDev G;
+    std::vector<int> subid(nsub, 0);
+    for (int d = 0; d < 3; d++) {
+        G.NN[d] = gridNE[d] + 1;
+        G.NS[d] = (int)start[d].size();
+    }
+    ESP_CHECK((int64_t)G.NS[0] * G.NS[1] * G.NS[2] == nsub, ESPRESO_ERR_STATE, "grid subdomains do not form a grid");
+    for (int s = 0; s < nsub; s++) {
+        int c[3];
+        const int *b = grid_box.data() + 6 * (size_t)s;
+        for (int d = 0; d < 3; d++)
+            c[d] = (int)(std::lower_bound(start[d].begin(), start[d].end(), b[d]) - start[d].begin());
+        subid[c[0] + G.NS[0] * (c[1] + G.NS[1] * c[2])] = s;
+        ESP_CHECK((int64_t)(b[3] + 1) * (b[4] + 1) * (b[5] + 1) * ndof == sub[s].n, ESPRESO_ERR_STATE,
+                  "subdomain " + std::to_string(s) + " is not the grid's");
+    }
+    for (int d = 0; d < 3; d++) {
+        std::vector<int> hi(G.NN[d]), cnt(G.NN[d]);
+        for (int g = 0; g < G.NN[d]; g++) {
+            const int i = (int)(std::upper_bound(start[d].begin(), start[d].end(), g) - start[d].begin()) - 1;
+            // the node past the last element belongs to the last slab only
+            hi[g] = i;
+            cnt[g] = (i > 0 && g == start[d][i]) ? 2 : 1;
+        }
+        G.hi[d] = upload(hi);
+        G.cnt[d] = upload(cnt);
+    }
+    G.box = upload(grid_box);
+    G.subid = upload(subid);
+    d_bad = alloc<int>(1);
+    sync();  // the host tables above
+    G.nd = ndof;
+    GD = G;
+}
+
+// device scratch for n values of nodal fields
+double *espreso_feti_s::nodal_buffer(int64_t n) {
+    if (n > n_nodal) {
+        if (d_nodal) release(d_nodal);
+        d_nodal = nullptr;
+        n_nodal = 0;
+        d_nodal = alloc<double>(n);
+        n_nodal = n;
+    }
+    return d_nodal;
+}
+
+// the host copies of the loads, when nodal loads were set on the device
+void espreso_feti_s::host_loads() {
+    if (!loads_on_device) return;
+    std::vector<double> ff(uoff[nsub]);
+    ESP_HIP(hipMemcpyAsync(ff.data(), d_fnew, ff.size() * sizeof(double), hipMemcpyDeviceToHost, st));
+    sync();
+    for (int s = 0; s < nsub; s++) sub[s].f.assign(ff.begin() + uoff[s], ff.begin() + uoff[s + 1]);
+    loads_on_device = false;
+}
+
+// new nodal loads of a loaded grid instance, split over the copies on the device
+void espreso_feti_s::set_nodal_rhs(const double *g) {
+    grid_device();
+    const int64_t nv = (int64_t)nnodes * ndof;
+    double *dg = nodal_buffer(nv);
+    if (!d_fnew) d_fnew = alloc<double>(uoff[nsub]);
+    if (!d_fspare) d_fspare = alloc<double>(uoff[nsub]);
+    ESP_HIP(hipMemsetAsync(d_bad, 0, sizeof(int), st));
+    ESP_HIP(hipMemcpyAsync(dg, g, nv * sizeof(double), hipMemcpyHostToDevice, st));
+    launch_nodal_split(GD, nsub, kkt_max_n, 1, P.perm_off, dg, 0, d_fspare, 0, d_bad, st);
+    int bad = 0;
+    ESP_HIP(hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, st));
+    sync();
+    ESP_CHECK(!bad, ESPRESO_ERR_ARG, "non-finite load");  // the earlier loads stay in force
+    std::swap(d_fnew, d_fspare);
+    loads_on_device = true;
 }
 
 void espreso_feti_s::assemble(const double *d_f, const double *d_Q, const std::vector<int64_t> *poff,
@@ -2456,24 +2527,23 @@ void espreso_feti_s::apply_F_block(const PcgVec &V, const double *x, double *y, 
                          dot ? V.dots + 2 * (size_t)dot_blocks(nlam, K) * K : nullptr);
 }
 
-void espreso_feti_s::resolve_group(int K, const double *f, double *u, int32_t *iters, double *norms,
+void espreso_feti_s::resolve_group(int K, const double *f, double *u, int32_t *iters, double *norms, bool nodal,
                                    espreso_feti_stats &tot) {
     const double t0 = wall();
     block_setup(K);
     const PcgVec V = block_vec(K);
     const int64_t nl = nlam, nb = D.nbnd, nt = uoff[nsub], na = std::max<int64_t>(asubv[nsub], 1);
-    // loads: e0f, e on the host (interleaved by case); f, y_f, hf (one band-solve launch) and b on the device
-    ESP_HIP(hipMemcpyAsync(BB.f, f, K * nt * sizeof(double), hipMemcpyHostToDevice, st));
-    std::vector<double> e0f_all((size_t)K * asubv[nsub]), e_all((size_t)K * ncoarse);
-    for (int v = 0; v < K; v++) {
-        hvec<double> e0f;
-        std::vector<double> e;
-        rhs_host(f + v * nt, e0f, e);
-        for (size_t q = 0; q < e0f.size(); q++) e0f_all[q * K + v] = e0f[q];
-        for (size_t q = 0; q < e.size(); q++) e_all[q * K + v] = e[q];
+    // loads: f (nodal loads split over the copies), e0f, e, y_f, hf (one band-solve launch) and b on the device
+    const int64_t nv = (int64_t)nnodes * ndof;
+    if (nodal) {
+        grid_device();
+        double *dg = nodal_buffer(K * nv);
+        ESP_HIP(hipMemcpyAsync(dg, f, K * nv * sizeof(double), hipMemcpyHostToDevice, st));
+        launch_nodal_split(GD, nsub, kkt_max_n, K, P.perm_off, dg, nv, BB.f, nt, d_bad, st);
+    } else {
+        ESP_HIP(hipMemcpyAsync(BB.f, f, K * nt * sizeof(double), hipMemcpyHostToDevice, st));
     }
-    ESP_HIP(hipMemcpyAsync(BB.e0f, e0f_all.data(), e0f_all.size() * sizeof(double), hipMemcpyHostToDevice, st));
-    ESP_HIP(hipMemcpyAsync(BB.e, e_all.data(), e_all.size() * sizeof(double), hipMemcpyHostToDevice, st));
+    launch_rhs_dots(P, D, K, BB.f, nt, BB.e0f, BB.e, st);
     launch_rhs_prepare_multi(P, nsub, K, BB.f, nt, BB.hf, BB.yf, nyf, BB.work, st);
     // K^+ f on the boundary: ubf = F_i hf, hybrid + cluster correction; b = B K^+ f - c
     launch_symv_mfma(D, SB, false, K, BB.hf, BB.yb, st);
@@ -2487,7 +2557,7 @@ void espreso_feti_s::resolve_group(int K, const double *f, double *u, int32_t *i
     apply_F_block(V, BB.x, BB.Ap, false);
     launch_axpby(BB.r, BB.b, BB.Ap, K * nl, 1.0, -1.0, st);
     pcg_start(V, BB.b, 0.0);
-    sync();  // the host vectors above are in use until here
+    sync();
     const double t1 = wall();
     pcg_loop(V, 0);
     std::vector<double> tol(rec->tol, rec->tol + K), nrm(K);
@@ -2507,7 +2577,13 @@ void espreso_feti_s::resolve_group(int K, const double *f, double *u, int32_t *i
     }
     launch_alpha_combine(D, K, BB.alphaK, na, hybrid, BB.alpha_c, BB.alpha_tot, st);
     launch_primal_multi(P, nsub, K, BB.xbv, BB.yf, nyf, BB.alpha_tot, na, BB.u, nt, BB.work, st);
-    ESP_HIP(hipMemcpyAsync(u, BB.u, K * nt * sizeof(double), hipMemcpyDeviceToHost, st));
+    if (nodal) {
+        double *dg = nodal_buffer(K * nv);
+        launch_nodal_gather(GD, K, P.perm_off, BB.u, nt, dg, nv, true, st);
+        ESP_HIP(hipMemcpyAsync(u, dg, K * nv * sizeof(double), hipMemcpyDeviceToHost, st));
+    } else {
+        ESP_HIP(hipMemcpyAsync(u, BB.u, K * nt * sizeof(double), hipMemcpyDeviceToHost, st));
+    }
     sync();
     for (int v = 0; v < K; v++) {
         if (iters) iters[v] = it_v[v];
@@ -2522,7 +2598,7 @@ void espreso_feti_s::resolve_group(int K, const double *f, double *u, int32_t *i
     tot.time_primal += wall() - t2;
 }
 
-bool espreso_feti_s::resolve_block(int nrhs, const double *f, double *u, int32_t *iters, double *norms,
+bool espreso_feti_s::resolve_block(int nrhs, const double *f, double *u, int32_t *iters, double *norms, bool nodal,
                                    espreso_feti_stats *stats) {
     ESP_CHECK(ready, ESPRESO_ERR_STATE, "espreso_feti_setup not called");
     const int64_t nt = uoff[nsub];
@@ -2534,7 +2610,10 @@ bool espreso_feti_s::resolve_block(int nrhs, const double *f, double *u, int32_t
     tot.converged = 1;
     if (opt.sc_precision != 0 || D.sd_prec != 0) {
         // low-precision storage: the cases one after another (refinement per
-        // case); the instance's own solution (lambda, u, stats) is restored after
+        // case); the instance's own loads and solution (lambda, u, stats) are
+        // restored after
+        const int64_t nv = (int64_t)nnodes * ndof;
+        host_loads();
         std::vector<std::vector<double>> keep(nsub);
         for (int s = 0; s < nsub; s++) keep[s] = sub[s].f;
         double *save_x = alloc<double>(nlam), *save_u = alloc<double>(nt);
@@ -2543,12 +2622,24 @@ bool espreso_feti_s::resolve_block(int nrhs, const double *f, double *u, int32_t
         const espreso_feti_stats save_last = last;
         const bool save_solved = solved;
         for (int v = 0; v < nrhs; v++) {
-            for (int s = 0; s < nsub; s++)
-                std::copy(f + v * nt + uoff[s], f + v * nt + uoff[s] + sub[s].n, sub[s].f.begin());
+            if (nodal) {
+                set_nodal_rhs(f + v * nv);
+            } else {
+                for (int s = 0; s < nsub; s++)
+                    std::copy(f + v * nt + uoff[s], f + v * nt + uoff[s] + sub[s].n, sub[s].f.begin());
+            }
             resolve_rhs();
+            loads_on_device = false;  // the host copies are the instance's own loads
             espreso_feti_stats sv{};
             solve(&sv);
-            ESP_HIP(hipMemcpy(u + v * nt, d_u, nt * sizeof(double), hipMemcpyDeviceToHost));
+            if (nodal) {
+                double *dg = nodal_buffer(nv);
+                launch_nodal_gather(GD, 1, P.perm_off, d_u, 0, dg, 0, true, st);
+                ESP_HIP(hipMemcpyAsync(u + v * nv, dg, nv * sizeof(double), hipMemcpyDeviceToHost, st));
+                sync();
+            } else {
+                ESP_HIP(hipMemcpy(u + v * nt, d_u, nt * sizeof(double), hipMemcpyDeviceToHost));
+            }
             if (iters) iters[v] = sv.iterations;
             if (norms) norms[v] = sv.final_norm;
             tot.iterations = std::max(tot.iterations, sv.iterations);
@@ -2570,11 +2661,12 @@ bool espreso_feti_s::resolve_block(int nrhs, const double *f, double *u, int32_t
         if (stats) *stats = tot;
         return tot.converged != 0;
     }
+    const int64_t nc = nodal ? (int64_t)nnodes * ndof : nt;  // values of one case
     for (int done = 0; done < nrhs;) {
         const int rem = nrhs - done;
         const int K = std::min(rem, 16);
-        resolve_group(K, f + done * nt, u + done * nt, iters ? iters + done : nullptr, norms ? norms + done : nullptr,
-                      tot);
+        resolve_group(K, f + done * nc, u + done * nc, iters ? iters + done : nullptr, norms ? norms + done : nullptr,
+                      nodal, tot);
         done += K;
     }
     tot.time_total = tot.time_coarse + tot.time_pcg + tot.time_primal;
@@ -2890,10 +2982,6 @@ void espreso_feti_s::load_clusters() {
         }
     }
     ESP_CHECK(ncoarse > 0, ESPRESO_ERR_NUMERIC, "HYBRID_FETI: empty coarse space");
-    Ns_h = Ns;
-    noff_h = noff;
-    ccoff_h = coff;
-    cblk_h = cblk;
     D.nblk = ncl;
     D.ncoarse = ncoarse;
     D.cblk = upload(cblk);
@@ -3208,6 +3296,14 @@ int espreso_feti_set_rhs(espreso_feti *h, int32_t i, const double *f) {
     ESP_CHECK(h->sub[i].set, ESPRESO_ERR_STATE, "subdomain not set");
     SubHost &s = h->sub[i];
     for (int q = 0; q < s.n; q++) ESP_CHECK(std::isfinite(f[q]), ESPRESO_ERR_ARG, "non-finite load");
+    {
+        // subdomains may be set by several threads: one of them fetches the loads
+        std::lock_guard<std::mutex> lock(h->pin_mu);
+        if (h->loads_on_device) {
+            ESP_HIP(hipSetDevice(h->opt.device));
+            h->host_loads();
+        }
+    }
     s.f.assign(f, f + s.n);
     ESP_API_END
 }
@@ -3253,7 +3349,7 @@ int espreso_feti_resolve_block(espreso_feti *h, int32_t nrhs, const double *f, d
 #pragma omp parallel for reduction(+ : bad)
     for (int64_t q = 0; q < nf; q++) bad += !std::isfinite(f[q]);
     ESP_CHECK(bad == 0, ESPRESO_ERR_NUMERIC, "non-finite load");
-    if (!h->resolve_block(nrhs, f, u, iterations, final_norms, stats)) return ESPRESO_NOT_CONVERGED;
+    if (!h->resolve_block(nrhs, f, u, iterations, final_norms, false, stats)) return ESPRESO_NOT_CONVERGED;
     ESP_API_END
 }
 
@@ -3689,6 +3785,15 @@ int espreso_grid_nodal_load(espreso_feti *h, double *g) {
     ESP_CHECK(h && g, ESPRESO_ERR_ARG, "null argument");
     ESP_CHECK((int)h->l2g.size() == h->nsub, ESPRESO_ERR_STATE, "grid not loaded");
     const int nd = h->ndof;
+    if (h->loads_on_device) {
+        ESP_HIP(hipSetDevice(h->opt.device));
+        const int64_t nv = (int64_t)h->nnodes * nd;
+        double *dg = h->nodal_buffer(nv);
+        launch_nodal_gather(h->GD, 1, h->P.perm_off, h->d_fnew, 0, dg, 0, false, h->st);
+        ESP_HIP(hipMemcpyAsync(g, dg, nv * sizeof(double), hipMemcpyDeviceToHost, h->st));
+        h->sync();
+        return ESPRESO_OK;
+    }
     std::fill(g, g + (size_t)h->nnodes * nd, 0.0);
     for (int s = 0; s < h->nsub; s++)
         for (size_t ln = 0; ln < h->l2g[s].size(); ln++)
@@ -3710,6 +3815,11 @@ int espreso_grid_set_nodal_rhs(espreso_feti *h, const double *g) {
     ESP_CHECK(h && g, ESPRESO_ERR_ARG, "null argument");
     ESP_CHECK((int)h->l2g.size() == h->nsub, ESPRESO_ERR_STATE, "grid not loaded");
     const int nd = h->ndof;
+    if (h->loaded) {
+        ESP_HIP(hipSetDevice(h->opt.device));
+        h->set_nodal_rhs(g);
+        return ESPRESO_OK;
+    }
     std::vector<int> mult(h->nnodes, 0);
     for (int s = 0; s < h->nsub; s++)
         for (int node : h->l2g[s]) mult[node]++;
@@ -3731,44 +3841,13 @@ int espreso_grid_resolve_block(espreso_feti *h, int32_t nrhs, const double *g, d
     ESP_CHECK(h && (nrhs == 0 || (g && u_nodal)) && nrhs >= 0, ESPRESO_ERR_ARG, "null argument");
     ESP_CHECK((int)h->l2g.size() == h->nsub, ESPRESO_ERR_STATE, "grid not loaded");
     ESP_CHECK(h->ready, ESPRESO_ERR_STATE, "espreso_feti_setup not called");
-    const int nd = h->ndof, nsub = h->nsub;
-    const int64_t nt = h->uoff[nsub], nv = (int64_t)h->nnodes * nd;
-    std::vector<int> mult(h->nnodes, 0);
-    for (int s = 0; s < nsub; s++)
-        for (int node : h->l2g[s]) mult[node]++;
-    // loads split over the subdomain copies of a node (as espreso_grid_set_nodal_rhs)
-    std::vector<double> f((size_t)nrhs * nt), u((size_t)nrhs * nt);
-#pragma omp parallel for collapse(2) schedule(dynamic, 8)
-    for (int v = 0; v < nrhs; v++)
-        for (int s = 0; s < nsub; s++) {
-            double *fs = f.data() + v * nt + h->uoff[s];
-            const double *gv = g + v * nv;
-            for (size_t ln = 0; ln < h->l2g[s].size(); ln++) {
-                const int node = h->l2g[s][ln];
-                for (int c = 0; c < nd; c++) fs[ln * nd + c] = gv[(size_t)node * nd + c] / mult[node];
-            }
-        }
+    ESP_HIP(hipSetDevice(h->opt.device));
+    const int64_t nv = (int64_t)h->nnodes * h->ndof;
     int64_t bad = 0;
 #pragma omp parallel for reduction(+ : bad)
-    for (int64_t q = 0; q < (int64_t)f.size(); q++) bad += !std::isfinite(f[q]);
+    for (int64_t q = 0; q < nrhs * nv; q++) bad += !std::isfinite(g[q]);
     ESP_CHECK(bad == 0, ESPRESO_ERR_NUMERIC, "non-finite load");
-    const bool conv = h->resolve_block(nrhs, f.data(), u.data(), iterations, final_norms, stats);
-    // solutions averaged over the subdomain copies (as espreso_grid_nodal_solution)
-#pragma omp parallel for schedule(static)
-    for (int v = 0; v < nrhs; v++) {
-        double *un = u_nodal + v * nv;
-        std::fill(un, un + nv, 0.0);
-        for (int s = 0; s < nsub; s++) {
-            const double *us = u.data() + v * nt + h->uoff[s];
-            for (size_t ln = 0; ln < h->l2g[s].size(); ln++) {
-                const int node = h->l2g[s][ln];
-                for (int c = 0; c < nd; c++) un[(size_t)node * nd + c] += us[ln * nd + c];
-            }
-        }
-        for (int node = 0; node < h->nnodes; node++)
-            for (int c = 0; c < nd; c++) un[(size_t)node * nd + c] /= mult[node];
-    }
-    if (!conv) return ESPRESO_NOT_CONVERGED;
+    if (!h->resolve_block(nrhs, g, u_nodal, iterations, final_norms, true, stats)) return ESPRESO_NOT_CONVERGED;
     ESP_API_END
 }
 
@@ -3831,19 +3910,13 @@ int espreso_grid_l2g(espreso_feti *h, int32_t i, int32_t *l2g) {
 int espreso_grid_nodal_solution(espreso_feti *h, double *u_nodal) {
     ESP_API_BEGIN
     ESP_CHECK(h && h->solved && !h->l2g.empty(), ESPRESO_ERR_STATE, "no grid solution");
-    const int nd = h->ndof;
-    std::vector<double> u(h->uoff[h->nsub]);
-    ESP_HIP(hipMemcpy(u.data(), h->d_u, u.size() * sizeof(double), hipMemcpyDeviceToHost));
-    std::vector<int> cnt(h->nnodes, 0);
-    std::fill(u_nodal, u_nodal + (size_t)h->nnodes * nd, 0.0);
-    for (int s = 0; s < h->nsub; s++)
-        for (size_t ln = 0; ln < h->l2g[s].size(); ln++) {
-            const int g = h->l2g[s][ln];
-            cnt[g]++;
-            for (int d = 0; d < nd; d++) u_nodal[(size_t)g * nd + d] += u[h->uoff[s] + ln * nd + d];
-        }
-    for (int g = 0; g < h->nnodes; g++)
-        for (int d = 0; d < nd; d++) u_nodal[(size_t)g * nd + d] /= std::max(cnt[g], 1);
+    ESP_HIP(hipSetDevice(h->opt.device));
+    h->grid_device();
+    const int64_t nv = (int64_t)h->nnodes * h->ndof;
+    double *dg = h->nodal_buffer(nv);
+    launch_nodal_gather(h->GD, 1, h->P.perm_off, h->d_u, 0, dg, 0, true, h->st);
+    ESP_HIP(hipMemcpyAsync(u_nodal, dg, nv * sizeof(double), hipMemcpyDeviceToHost, h->st));
+    h->sync();
     ESP_API_END
 }
 
