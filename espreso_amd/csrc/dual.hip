@@ -170,17 +170,25 @@ __global__ void __launch_bounds__(256) k_symv(const SymvItem *__restrict__ items
 
 // Block SYMV on MFMA (v_mfma_f64_16x16x4f64): up to 16 right-hand sides, the
 // MFMA's N dimension (lanes of right-hand sides past nr carry zeros).  An
-// item is at most BLOCK_STRIPS strips of one subdomain; wave w owns the
-// 16-column blocks w, w+4, ... of the item's column range and visits every
-// strip of the item that holds the block (the 16-column grid is common to all
-// strips since strips start at multiples of 16):
+// item is at most BLOCK_STRIPS strips of one subdomain; wave w owns strips 2w
+// and 2w + 1 and walks the 16-column blocks of the item (a grid common to all
+// strips, which start at multiples of 16), the four waves in step:
 //   column product  Dc[c][v] += sum_r A[r][c] x[r][v]   (A op: lane (c, row slot))
 //   row product     Dr[r][v] += sum_c A[r][c] x[c][v]   (A op: lane (r, column slot))
-// The 16-byte loads give the first operand layout; a per-wave LDS tile
-// transposes the block for the second.  Column sums are final when the wave
-// leaves the block (written straight to the item's partial, no atomics); row
-// sums stay in registers per strip and meet in LDS at the end.  x and the
-// partials are interleaved by right-hand side with stride nr.
+// The 16-byte loads give the first operand layout; per-wave LDS tiles
+// transpose the blocks for the second.  Row sums and the x of a wave's rows stay
+// in registers; the column sums of a step meet in LDS, where thread (column, case)
+// adds the four waves' in order and writes the item's partial (fixed order, so
+// repeated applies are bitwise equal).  x and the partials are interleaved by
+// right-hand side with stride nr.
+// What bounds it is the latency of a step (load, transpose, eight chained MFMAs), so
+// the next step's blocks are loaded before the current ones are used, by loads
+// without a branch (blocks left of a strip's diagonal, past the item's strips or
+// past the last column repeat stored values and are zeroed when used: at a branch
+// the compiler waits for every load in flight), and four workgroups share a CU.
+// Waves owning columns instead of strips, one block's loads in flight, took 745 us
+// for 1.2 GB of F_i at 2000 heat subdomains and 16 cases (now 632), 421 at 512
+// uneven elasticity subdomains and 5 cases (now 333).
 typedef double v4d __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ void wave_lds_sync() {
@@ -189,108 +197,136 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__global__ void __launch_bounds__(256) k_symv_mfma(const SymvItem *__restrict__ items, const int *__restrict__ M,
-                                                   const int64_t *__restrict__ boff, const double *__restrict__ pool,
-                                                   const int64_t *__restrict__ poff, const double *__restrict__ xb,
-                                                   int nr, double *__restrict__ ypart) {
-    constexpr int R = STRIP_F64, S = BLOCK_STRIPS, TL = 18;  // TL: leading dimension of the transpose tile
-    __shared__ double xr[S * R * 16], yr[S * R * 16];        // [item row][rhs], stride 16
-    __shared__ double T[4][16 * TL];
+// workgroup barrier that orders LDS accesses only: the full barrier also waits for
+// every global load in flight
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+__global__ void __launch_bounds__(256, 4) k_symv_mfma(const SymvItem *__restrict__ items, const int *__restrict__ M,
+                                                      const int64_t *__restrict__ boff,
+                                                      const double *__restrict__ pool,
+                                                      const int64_t *__restrict__ poff, const double *__restrict__ xb,
+                                                      int nr, double *ypart) {
+    constexpr int R = STRIP_F64, W = BLOCK_STRIPS / 4, TL = 18;  // W strips per wave; TL: leading dimension of T
+    __shared__ double T[4][W][16 * TL], slot[2][4][256];
     const SymvItem it = items[blockIdx.x];
     const int s = it.sub, m = M[s];
     const int ns = it.t1 - it.t0, r0i = it.t0 * R;
-    const int nrow = min(ns * R, m - r0i);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int q = lane >> 4, l16 = lane & 15;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q = lane >> 4, l16 = lane & 15, lv = min(l16, nr - 1);
     const double *xs = xb + boff[s] * nr;
-    for (int i = tid; i < S * R * 16; i += 256) {
-        const int row = i >> 4, v = i & 15;
-        xr[i] = (row < nrow && v < nr) ? xs[(int64_t)(r0i + row) * nr + v] : 0.0;
-        yr[i] = 0.0;
-    }
-    __syncthreads();
-    const double *bs = pool + poff[s];
-    double *Tw = T[wave];
-    v4d dr[S];
-#pragma unroll
-    for (int t = 0; t < S; t++) dr[t] = (v4d){0.0, 0.0, 0.0, 0.0};
     const int nblk = (m - r0i + 15) / 16;
-    for (int cb = wave; cb < nblk; cb += 4) {
-        const int c0 = r0i + 16 * cb;
-        // row-product B operand: x[c0 + q + 4j][l16]
-        double xc[4];
+    // the wave's strips (clamped to the item's), where they start and their columns
+    const u32x4 *strip[W];
+    int r0[W];
+    double xr[W][4];  // x of the strip rows: row slot q of call (j, e) is row 2q + 8j + e
+    v4d dr[W];
+#pragma unroll
+    for (int k = 0; k < W; k++) {
+        const int t = it.t0 + min(W * wave + k, ns - 1);
+        strip[k] = (const u32x4 *)(pool + poff[s] + strip_offset(m, R, t));
+        r0[k] = t * R;
+        dr[k] = (v4d){0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const int c = c0 + q + 4 * j;
-            xc[j] = (c < m && l16 < nr) ? xs[(int64_t)c * nr + l16] : 0.0;
+            const int row = r0[k] + 2 * q + 8 * (j >> 1) + (j & 1);
+            const double v = xs[(int64_t)min(row, m - 1) * nr + lv];
+            xr[k][j] = (row < m && l16 < nr) ? v : 0.0;
         }
-        v4d dc = {0.0, 0.0, 0.0, 0.0};
-        const int tl = min(ns, cb + 1);  // strips holding the block (upper triangle)
+    }
+    // column block cb of the wave's strips: rows 2q, 2q+1 and 2q+8, 2q+9 of column
+    // c0 + l16; and the row product's B operand x[c0 + q + 4j][l16]
+    struct Step {
+        u32x4 p[W][2];
+        double x[4];
+    } st[2];
+    auto load = [&](Step &n, int cb) {
+        const int c0 = r0i + 16 * min(cb, nblk - 1);
 #pragma unroll
-        for (int tt = 0; tt < S; tt++) {
-            if (tt < tl) {
-                const int t = it.t0 + tt, r0 = t * R, ncol = m - r0;
-                const int cl = c0 - r0;  // >= 0, multiple of 16
-                const int k = cl >> 6, cc = (cl & 63) + l16;
-                const int w = min(64, ncol - 64 * k);
-                const u32x4 *chunk = (const u32x4 *)(bs + strip_offset(m, R, t) + (int64_t)64 * k * R);
-                u32x4 p0 = {0u, 0u, 0u, 0u}, p1 = {0u, 0u, 0u, 0u};
-                if (cc < w) {
-                    p0 = __builtin_nontemporal_load(chunk + q * w + cc);        // rows 2q, 2q+1
-                    p1 = __builtin_nontemporal_load(chunk + (q + 4) * w + cc);  // rows 2q+8, 2q+9
-                }
-                double a[4];
-                __builtin_memcpy(&a[0], &p0, 16);
-                __builtin_memcpy(&a[2], &p1, 16);
-                // column product: row slot q of call (j, e) is row 2q + 8j + e
-                const double *xrow = xr + (r0 - r0i) * 16;
+        for (int k = 0; k < W; k++) {
+            const int cl = max(0, c0 - r0[k]), ch = cl & ~63, w = min(64, m - r0[k] - ch);
+            const int at = min(cl - ch + l16, w - 1);
+            const u32x4 *chunk = strip[k] + (int64_t)ch * (R / 2);
+            n.p[k][0] = __builtin_nontemporal_load(chunk + q * w + at);
+            n.p[k][1] = __builtin_nontemporal_load(chunk + (q + 4) * w + at);
+        }
 #pragma unroll
-                for (int j = 0; j < 2; j++)
+        for (int j = 0; j < 4; j++) n.x[j] = xs[(int64_t)min(c0 + q + 4 * j, m - 1) * nr + lv];
+    };
+    auto step = [&](Step &c, int cb, int buf) {
+        const int c0 = r0i + 16 * cb;
+        if (cb < BLOCK_STRIPS || c0 + 16 > m || ns < BLOCK_STRIPS) {  // uniform: values to zero
+            const u32x4 zero = {0u, 0u, 0u, 0u};
 #pragma unroll
-                    for (int e = 0; e < 2; e++)
-                        dc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[2 * j + e], xrow[(2 * q + 8 * j + e) * 16 + l16],
-                                                                  dc, 0, 0, 0);
-                // transpose through the wave's tile: T[c][r]
-                *(u32x4 *)(Tw + l16 * TL + 2 * q) = p0;
-                *(u32x4 *)(Tw + l16 * TL + 2 * q + 8) = p1;
-                wave_lds_sync();
-                // row product: column slot q of call j is column q + 4j
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-                    dr[tt] = __builtin_amdgcn_mfma_f64_16x16x4f64(Tw[(q + 4 * j) * TL + l16], xc[j], dr[tt], 0, 0, 0);
-                wave_lds_sync();
+            for (int k = 0; k < W; k++) {
+                const bool in = W * wave + k <= min(cb, ns - 1) && c0 + l16 < m;
+                c.p[k][0] = in ? c.p[k][0] : zero;
+                c.p[k][1] = in ? c.p[k][1] : zero;
             }
+#pragma unroll
+            for (int j = 0; j < 4; j++) c.x[j] = c0 + q + 4 * j < m ? c.x[j] : 0.0;
         }
-        // column sums of the block: lane holds D[c0 + q + 4i][l16]
+        v4d dc[W];  // a chain per strip
+#pragma unroll
+        for (int k = 0; k < W; k++) {
+            dc[k] = (v4d){0.0, 0.0, 0.0, 0.0};
+            *(u32x4 *)(T[wave][k] + l16 * TL + 2 * q) = c.p[k][0];
+            *(u32x4 *)(T[wave][k] + l16 * TL + 2 * q + 8) = c.p[k][1];
+        }
+        double a[W][4];
+        __builtin_memcpy(a, c.p, sizeof(a));
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int k = 0; k < W; k++)
+                dc[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k][j], xr[k][j], dc[k], 0, 0, 0);
+        wave_lds_sync();
+        // row product: column slot q of call j is column q + 4j
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int k = 0; k < W; k++)
+                dr[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(T[wave][k][(q + 4 * j) * TL + l16], c.x[j], dr[k], 0, 0, 0);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int c = c0 + q + 4 * i;
-            if (c < m && l16 < nr) {
-                const int j = c - r0i;
-                if (j < nrow) yr[j * 16 + l16] = dc[i];  // the only column sum of j
-                else ypart[(it.part_off + j) * nr + l16] = dc[i];
-            }
+            double v = dc[0][i];
+#pragma unroll
+            for (int k = 1; k < W; k++) v += dc[k][i];
+            slot[buf][wave][(q + 4 * i) * 16 + l16] = v;
         }
+        lds_barrier();  // a slot is written again two steps on, behind the next barrier
+        const int col = c0 + (tid >> 4), v = tid & 15;
+        if (col < m && v < nr)
+            ypart[(it.part_off + col - r0i) * nr + v] =
+                (slot[buf][0][tid] + slot[buf][1][tid]) + (slot[buf][2][tid] + slot[buf][3][tid]);
+    };
+    load(st[0], 0);
+    for (int cb = 0; cb < nblk; cb += 2) {
+        load(st[1], cb + 1);
+        step(st[0], cb, 0);
+        if (cb + 1 >= nblk) break;
+        load(st[0], cb + 2);
+        step(st[1], cb + 1, 1);
     }
-    // row sums: lane holds D[strip row q + 4i][l16] per strip; the waves add
-    // them in turn (a fixed order, so repeated applies are bitwise equal)
+    // the row sums join the column sums of the item's own rows: lane holds D[strip row q + 4i][l16]
     __syncthreads();
-    for (int w = 0; w < 4; w++) {
-        if (wave == w) {
+    double own[W][4];
 #pragma unroll
-            for (int tt = 0; tt < S; tt++)
+    for (int k = 0; k < W; k++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int row = tt * R + q + 4 * i;
-                    if (tt < ns && row < nrow && l16 < nr) yr[row * 16 + l16] += dr[tt][i];
-                }
+        for (int i = 0; i < 4; i++)
+            own[k][i] = ypart[(it.part_off + min(r0[k] + q + 4 * i, m - 1) - r0i) * nr + lv];
+#pragma unroll
+    for (int k = 0; k < W; k++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int row = r0[k] + q + 4 * i;
+            if (W * wave + k < ns && row < m && l16 < nr)
+                ypart[(it.part_off + row - r0i) * nr + l16] = own[k][i] + dr[k][i];
         }
-        __syncthreads();
-    }
-    for (int i = tid; i < nrow * 16; i += 256) {
-        const int j = i >> 4, v = i & 15;
-        if (v < nr) ypart[(it.part_off + j) * nr + v] = yr[i];
-    }
 }
 
 __device__ __forceinline__ double block_sum(double v, double *red) {
