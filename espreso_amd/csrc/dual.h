@@ -140,6 +140,7 @@ struct ClusterDev {
     double *rho_s = nullptr;   // per subdomain: max diag S_i (the scale of the kernel regularisation)
 };
 
+constexpr int BAND_PAD = 72;  // columns past the last subdomain's band (at the largest width), read and not used
 struct PrimalDev {
     int *ni = nullptr, *m = nullptr, *n = nullptr, *bw = nullptr, *kdim = nullptr, *coff = nullptr;
     int64_t *band_off = nullptr, *yf_off = nullptr, *perm_off = nullptr, *rp_off = nullptr, *nz_off = nullptr;
@@ -147,7 +148,7 @@ struct PrimalDev {
     double *band = nullptr, *yf = nullptr, *vals = nullptr, *R = nullptr, *alpha = nullptr, *work = nullptr;
     int64_t *asub = nullptr;
     int *perm = nullptr, *iperm = nullptr, *rowptr = nullptr, *colidx = nullptr;
-    int max_ni = 0;  // largest interior DOF count (host value: launch grids)
+    int max_ni = 0, max_m = 0, max_n = 0;  // largest interior, boundary and total DOF counts (host values: launch grids)
 };
 
 // structured grid on the device: node counts, subdomain counts, boxes (6 ints per
@@ -226,15 +227,14 @@ void launch_alpha_combine(const DualDev &D, int K, const double *alphaK, int64_t
 void launch_dot(const double *a, const double *b, int64_t n, double *partial, double *out, hipStream_t st);
 void launch_axpby(double *y, const double *a, const double *b, int64_t n, double alpha, double beta, hipStream_t st);
 void launch_symmetrize(double *A, int n, hipStream_t st);
-void launch_primal(const PrimalDev &P, int nsub, const double *ub, double *u, hipStream_t st);
-// new loads f (local DOF order, all subdomains): P.yf = L^-1 f_int, hf = f_b - K_bi K_ii^-1 f_int
-void launch_rhs_prepare(const PrimalDev &P, int nsub, const double *f, double *hf, hipStream_t st);
-// nr load vectors at once (strides fstr, ystr; hf and ub interleaved; work:
-// 16 values per interior row, P.work_off layout)
-void launch_rhs_prepare_multi(const PrimalDev &P, int nsub, int nr, const double *f, int64_t fstr, double *hf,
-                              double *yf, int64_t ystr, double *work, hipStream_t st);
-void launch_primal_multi(const PrimalDev &P, int nsub, int nr, const double *ub, const double *yf, int64_t ystr,
-                         const double *alpha, int64_t astr, double *u, int64_t ustr, double *work, hipStream_t st);
+// nr cases at once (strides fstr, ystr, astr, ustr; hf and ub interleaved in lines of nr; work: min(nr, 16)
+// values per interior row, P.work_off layout).  New loads f (local DOF order, all subdomains):
+// yf = L^-1 f_int, hf = f_b - K_bi K_ii^-1 f_int
+void launch_rhs_prepare(const PrimalDev &P, int nsub, int nr, const double *f, int64_t fstr, double *hf, double *yf,
+                        int64_t ystr, double *work, hipStream_t st);
+// u = [K_ii^-1 (f_int - K_ib u_b); u_b] + R alpha in local DOF order
+void launch_primal(const PrimalDev &P, int nsub, int nr, double *ub, double *yf, int64_t ystr, const double *alpha,
+                   int64_t astr, double *u, int64_t ustr, double *work, hipStream_t st);
 // sens[e] = -w_e^T Ke0 u_e over the NE[0] x NE[1] x NE[2] HEXA8 grid (nodal fields, ndof nd)
 void launch_element_sensitivity(const int *NE, int nd, const double *Ke0, const double *u, const double *w,
                                 double *sens, hipStream_t st);

@@ -1015,7 +1015,7 @@ void espreso_feti_s::load() {
             bw = std::max(bw, r - fr);
             bt = std::max(bt, r / TILE - fr / TILE);
         }
-        h.bw = bw;
+        h.bw = std::max(bw, TILE - 1);  // the inverses of the diagonal blocks are kept in the band
         h.band_tiles = std::max(bt, 1);
         const int ntc = (h.m + 1 + TILE - 1) / TILE;
         h.colstart.assign(ntc, 0);
@@ -1407,7 +1407,11 @@ void espreso_feti_s::load() {
         P.iperm = upload_pieces<int>(n_off, [&](int s) { return sub[s].iperm.data(); });
         P.R = upload_pieces<double>(r_off, [&](int s) { return sub[s].R.data(); });
         P.ni = upload(niv);
-        P.max_ni = nsub ? *std::max_element(niv.begin(), niv.end()) : 0;
+        for (const SubHost &h : sub) {
+            P.max_ni = std::max(P.max_ni, h.ni);
+            P.max_m = std::max(P.max_m, h.m);
+            P.max_n = std::max(P.max_n, h.n);
+        }
         P.n = upload(nv);
         P.bw = upload(bwv);
         P.m = D.m;
@@ -1419,7 +1423,9 @@ void espreso_feti_s::load() {
         P.yf_off = upload(yf_off);
         P.work_off = P.yf_off;
         P.r_off = upload(r_off);
-        P.band = alloc<double>(band_off[nsub]);
+        int max_bw = 0;
+        for (int b : bwv) max_bw = std::max(max_bw, b);
+        P.band = alloc<double>(band_off[nsub] + BAND_PAD * (int64_t)(max_bw + 1));
         P.yf = alloc<double>(yf_off[nsub]);
         P.work = alloc<double>(yf_off[nsub]);
         nyf = yf_off[nsub];
@@ -1587,7 +1593,7 @@ void espreso_feti_s::resolve_rhs() {
         ESP_HIP(hipMemcpyAsync(d_f, ff.data(), ff.size() * sizeof(double), hipMemcpyHostToDevice, st));
     }
     launch_rhs_dots(P, D, 1, d_f, 0, d_e0f, d_e, st);
-    launch_rhs_prepare(P, nsub, d_f, d_hf, st);
+    launch_rhs_prepare(P, nsub, 1, d_f, 0, d_hf, P.yf, 0, P.work, st);
     compute_b();
     sync();
 }
@@ -2364,7 +2370,7 @@ void espreso_feti_s::solve(espreso_feti_stats *out) {
         launch_cluster_correction(D, CL, d_e0s, D.xb, 0, st);
     }
     launch_alpha_combine(D, 1, CL.alphaK, 0, hybrid, d_alpha_c, d_alpha_tot, st);
-    launch_primal(P, nsub, D.xb, d_u, st);
+    launch_primal(P, nsub, 1, D.xb, P.yf, 0, P.alpha, 0, d_u, 0, P.work, st);
     // KKT report of the solution (GetSolution_Primal_singular_parallel, itersolver.cpp:171-370)
     kkt(d_x, last);
     if (opt.truncate_output) truncate_primal();
@@ -2488,7 +2494,7 @@ void espreso_feti_s::block_setup(int K) {
     BB.yf = alloc<double>(K * std::max<int64_t>(nyf, 1));
     BB.u = alloc<double>(K * uoff[nsub]);
     BB.scal = alloc<double>((size_t)PCG_SLOTS * K);
-    BB.work = alloc<double>(16 * std::max<int64_t>(nyf, 1));
+    BB.work = alloc<double>(std::min<int64_t>(K, 16) * std::max<int64_t>(nyf, 1));
     BB.e0s = alloc<double>(K * n_e0s);
     BB.lam0 = alloc<double>(K * n_lambda0);
     BB.alphaK = alloc<double>(K * na);
@@ -2544,7 +2550,7 @@ void espreso_feti_s::resolve_group(int K, const double *f, double *u, int32_t *i
         ESP_HIP(hipMemcpyAsync(BB.f, f, K * nt * sizeof(double), hipMemcpyHostToDevice, st));
     }
     launch_rhs_dots(P, D, K, BB.f, nt, BB.e0f, BB.e, st);
-    launch_rhs_prepare_multi(P, nsub, K, BB.f, nt, BB.hf, BB.yf, nyf, BB.work, st);
+    launch_rhs_prepare(P, nsub, K, BB.f, nt, BB.hf, BB.yf, nyf, BB.work, st);
     // K^+ f on the boundary: ubf = F_i hf, hybrid + cluster correction; b = B K^+ f - c
     launch_symv_mfma(D, SB, false, K, BB.hf, BB.yb, st);
     ESP_HIP(hipMemcpyAsync(BB.ubf, BB.yb, K * nb * sizeof(double), hipMemcpyDeviceToDevice, st));
@@ -2576,7 +2582,7 @@ void espreso_feti_s::resolve_group(int K, const double *f, double *u, int32_t *i
         launch_cluster_correction_multi(D, CL, K, BB.e0s, BB.lam0, n_lambda0, BB.alphaK, na, BB.xbv, 0, st);
     }
     launch_alpha_combine(D, K, BB.alphaK, na, hybrid, BB.alpha_c, BB.alpha_tot, st);
-    launch_primal_multi(P, nsub, K, BB.xbv, BB.yf, nyf, BB.alpha_tot, na, BB.u, nt, BB.work, st);
+    launch_primal(P, nsub, K, BB.xbv, BB.yf, nyf, BB.alpha_tot, na, BB.u, nt, BB.work, st);
     if (nodal) {
         double *dg = nodal_buffer(K * nv);
         launch_nodal_gather(GD, K, P.perm_off, BB.u, nt, dg, nv, true, st);

@@ -135,7 +135,8 @@ void launch_hf(const DenseDesc *desc, int nb, const double *fb, double *hf, cons
 void launch_rownorm(const DenseDesc *desc, int nb, double *nrm, int max_m, hipStream_t st);
 void launch_pack(const DenseDesc *desc, int nb, int prec, void *pool, const int64_t *off, float *scale,
                  int max_m, hipStream_t st);
-// copy band of L (ni x (bw+1), column c holds L[c..c+bw][c]) and y_f out of the workspace
+// copy band of L (ni x (bw+1), column c holds L[c..c+bw][c], bw >= 63; 64 x 64 diagonal blocks: their inverses)
+// and y_f out of the workspace
 void launch_band_extract(const DenseDesc *desc, int nb, double *band, const int64_t *band_off, const int *bw,
                          double *yf, const int64_t *yf_off, int max_ni, hipStream_t st);
 // unpack one strip-packed matrix into dense m x m (column-major, full)
