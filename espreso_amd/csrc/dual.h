@@ -90,7 +90,8 @@ struct DualDev {
     int sd_prec = 0;
     double *GGinv = nullptr;
     // SYMV work lists per storage precision (F_i and S_D of one precision share them)
-    SymvItem *items[3] = {nullptr, nullptr, nullptr};
+    SymvItem *items[3] = {nullptr, nullptr, nullptr};         // by subdomain
+    SymvItem *launch_items[3] = {nullptr, nullptr, nullptr};  // largest first
     int n_items[3] = {0, 0, 0};
     int *item0[3] = {nullptr, nullptr, nullptr}, *nitems[3] = {nullptr, nullptr, nullptr};
     double *ypart = nullptr;

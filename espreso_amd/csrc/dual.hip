@@ -707,7 +707,7 @@ static inline unsigned vgrid(int64_t n) { return (unsigned)std::max<int64_t>(1, 
 void launch_symv(const DualDev &D, bool sd, int prec, const double *x, int gather, bool scaled, hipStream_t st,
                  hipEvent_t ev0, hipEvent_t ev1) {
     if (sd) prec = D.sd_prec;
-    const SymvItem *items = D.items[prec];
+    const SymvItem *items = D.launch_items[prec];
     const int n_items = D.n_items[prec];
     const double *coef = scaled ? D.bl_sscale : D.bl_sign;
     const double *nrm = sd ? D.sdnrm : D.fnrm;
@@ -728,7 +728,7 @@ void launch_symv(const DualDev &D, bool sd, int prec, const double *x, int gathe
                            D.bl_lam, coef, x, gather, D.ypart);
     }
     if (ev1) (void)hipEventRecord(ev1, st);
-    launch_part_reduce(D, items, D.item0[prec], D.nitems[prec], strip_rows(prec), 1, D.ypart, D.yb, st);
+    launch_part_reduce(D, D.items[prec], D.item0[prec], D.nitems[prec], strip_rows(prec), 1, D.ypart, D.yb, st);
 }
 
 void launch_symv_mfma(const DualDev &D, const SymvBlock &B, bool sd, int nr, const double *xb, double *yb,
@@ -859,8 +859,8 @@ void launch_copy(const double *src, double *dst, int64_t n, hipStream_t st) {
 // direction at bw = 270; 16 waves a workgroup gain nothing (943 against 890 us at 64
 // subdomains, 2010 against 1780 at 512).  Chains of 64 divisions and one row a thread
 // took, for the two directions: 3.7 ms at 512 subdomains of 2187 interior DOFs (now
-// 1.78), 2.95 ms at 64 of them (now 0.89), 13.2 ms at 2000 heat subdomains of 729 and
-// 16 cases (now 1.3 and, without the gather, 1.1).
+// 1.78), 2.95 ms at 64 of them (now 0.89), 13.2 ms at 2000 uneven heat subdomains
+// (4 to 14 elements an edge) and 16 cases (now 1.3 and, without the gather, 1.1).
 // PRIMAL: z = K_ib u_b on entry; z <- L^-T (yf - L^-1 z).  Else z = f_int,
 // yf = L^-1 z, z <- L^-T yf.
 // p[off] with a scalar base: the offset of a lane is the same for every load of a step
