@@ -106,6 +106,7 @@ struct DualDev {
     double *Rt = nullptr, *N = nullptr, *dsub = nullptr;
     double *RbT = nullptr, *RtT = nullptr;  // R_b and Rt with row-major subdomain blocks
     LamCoarse *le_coarse = nullptr;         // per lambda entry (2 per lambda)
+    int max_k = 0;                          // most kernel or coarse columns of a subdomain
     bool coarse_direct = false;             // dsub is the coarse vector (one subdomain per block, in order)
     int64_t *asub = nullptr;          // offset of kernel amplitudes of subdomain s (sum of kdim)
 };
@@ -160,6 +161,32 @@ struct GridDev {
     const int *box = nullptr, *subid = nullptr;  // subid: slab coordinates (x fastest) -> subdomain
     const int *hi[3] = {nullptr, nullptr, nullptr}, *cnt[3] = {nullptr, nullptr, nullptr};
 };
+
+// transpose-reduce R per-lane accumulators over the 64 lanes of a wave; on
+// return lane l holds the total of row (l / (64/R)) in v[0]
+template <int R, typename A>
+__device__ __forceinline__ A wave_rows_reduce(A *v, int lane) {
+    int n = R;
+#pragma unroll
+    for (int o = 32; o >= 64 / R; o >>= 1) {
+        const bool up = lane & o;
+        const int h = n >> 1;
+#pragma unroll
+        for (int i = 0; i < h; i++) {
+            // select values, not addresses: a conditional over the two array
+            // elements would index the array dynamically and push it to scratch
+            const A lo = v[i], hi = v[i + h];
+            const A send = up ? (A)lo : (A)hi;
+            const A keep = up ? (A)hi : (A)lo;
+            v[i] = keep + __shfl_xor(send, o, 64);
+        }
+        n = h;
+    }
+    A s = v[0];
+#pragma unroll
+    for (int o = 64 / R / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    return s;
+}
 
 // y_b (D.yb) = A x_b for every subdomain; A = S_D (sd) or F_i in storage
 // precision `prec` (0 FP64, 1 FP32, 2 BF16).  x is lambda-space and gathered

@@ -32,32 +32,6 @@ __device__ __forceinline__ A load_cvt(T v) { return (A)v; }
 template <>
 __device__ __forceinline__ float load_cvt<uint16_t, float>(uint16_t v) { return __uint_as_float(((uint32_t)v) << 16); }
 
-// transpose-reduce R per-lane accumulators over the 64 lanes of a wave; on
-// return lane l holds the total of row (l / (64/R)) in v[0]
-template <int R, typename A>
-__device__ __forceinline__ A wave_rows_reduce(A *v, int lane) {
-    int n = R;
-#pragma unroll
-    for (int o = 32; o >= 64 / R; o >>= 1) {
-        const bool up = lane & o;
-        const int h = n >> 1;
-#pragma unroll
-        for (int i = 0; i < h; i++) {
-            // select values, not addresses: a conditional over the two array
-            // elements would index the array dynamically and push it to scratch
-            const A lo = v[i], hi = v[i + h];
-            const A send = up ? (A)lo : (A)hi;
-            const A keep = up ? (A)hi : (A)lo;
-            v[i] = keep + __shfl_xor(send, o, 64);
-        }
-        n = h;
-    }
-    A s = v[0];
-#pragma unroll
-    for (int o = 64 / R / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    return s;
-}
-
 // Fixed-point accumulation of the SYMV: value v enters the accumulators as
 // rint(v 2^k).  With 2^e <= 2 ||F_s||_inf max|x| (the bound of every partial
 // sum, doubled against the rounding of the stored values) and k = 60 - e,

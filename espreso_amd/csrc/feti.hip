@@ -1292,6 +1292,7 @@ void espreso_feti_s::load() {
     for (int s = 0; s < nsub; s++) { mv[s] = sub[s].m; kd[s] = sub[s].kdim; }
     D.m = upload(mv);
     D.kdim = upload(kd);
+    D.max_k = nsub ? *std::max_element(kd.begin(), kd.end()) : 0;
     D.asub = upload(asubv);
     D.boff = upload(boff);
     D.rboff = upload(rboff);
@@ -3002,6 +3003,7 @@ void espreso_feti_s::load_clusters() {
         }
     }
     ESP_CHECK(ncoarse > 0, ESPRESO_ERR_NUMERIC, "HYBRID_FETI: empty coarse space");
+    D.max_k = std::max(D.max_k, *std::max_element(ck.begin(), ck.end()));
     D.nblk = ncl;
     D.ncoarse = ncoarse;
     D.cblk = upload(cblk);

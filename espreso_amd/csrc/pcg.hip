@@ -22,63 +22,139 @@ typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
 
 static inline unsigned cdiv(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
 
-// threads of a workgroup as lines of K values: thread (li, v), li < per
+// Threads of a workgroup as lines of K values, W consecutive cases a thread (W = 2:
+// 16-byte accesses, K even): thread (li, v), li < per, v the first case of the thread,
+// `width` threads a line, K / W or (pad) the next power of two, so that no line straddles
+// a wave.  Pairs of cases halve the instructions and requests of a pass, which is what
+// bounds it once thousands of workgroups are in flight: at 669000 lines of 16 cases (86
+// MB a vector) lambda gather 100 -> 48 us, boundary gather 99 -> 79, projector finish
+// 152 -> 52, partial sums 128 -> 79 (5 TB/s); several lines a thread gain nothing more.
+constexpr int LINE_CASES = 16;  // largest K
+template <int W>
 struct Lines {
-    int per, li, v;
+    int per, li, v, width;
     bool on;
-};
-__device__ __forceinline__ Lines lines_of(int K) {
-    Lines L;
-    if (K == 1) {
-        L.per = blockDim.x;
-        L.li = threadIdx.x;
-        L.v = 0;
-        L.on = true;
-    } else {
-        L.per = blockDim.x / K;
-        L.li = threadIdx.x / K;
-        L.v = threadIdx.x - L.li * K;
-        L.on = L.li < L.per;
+    __device__ __forceinline__ explicit Lines(int K, bool pad = false) {
+        width = K / W;
+        if (pad) width = width > 8 ? 16 : width > 4 ? 8 : width > 2 ? 4 : width;
+        per = blockDim.x;
+        li = threadIdx.x;
+        v = 0;
+        if (width > 1) {
+            per = blockDim.x / width;
+            li = threadIdx.x / width;
+            v = (threadIdx.x - li * width) * W;
+        }
+        on = li < per && v < K;
+        if (!on) v = 0;
     }
-    return L;
+};
+template <int W>
+struct Vals {
+    double d[W];
+};
+template <int W>
+__device__ __forceinline__ Vals<W> line_load(const double *p) {
+    Vals<W> r;
+    if constexpr (W == 2) {
+        const double2 x = *(const double2 *)p;
+        r.d[0] = x.x;
+        r.d[1] = x.y;
+    } else {
+        r.d[0] = *p;
+    }
+    return r;
+}
+template <int W>
+__device__ __forceinline__ void line_store(double *p, const Vals<W> &x) {
+    if constexpr (W == 2) *(double2 *)p = make_double2(x.d[0], x.d[1]);
+    else *p = x.d[0];
 }
 
-// sum of `val` over the lines of the workgroup, per case: sh[v] (blockDim
-// doubles of LDS), in a fixed order; every thread may read sh[v] afterwards
-__device__ __forceinline__ void lines_sum(double val, const Lines &L, int K, double *sh) {
-    __syncthreads();
-    sh[threadIdx.x] = L.on ? val : 0.0;
-    __syncthreads();
-    int h = 1;
-    while (2 * h < L.per) h *= 2;
-    for (; h > 0; h >>= 1) {
-        if (L.on && L.li < h && L.li + h < L.per) sh[threadIdx.x] += sh[threadIdx.x + h * K];
+// sum of `val` over the lines of the workgroup, per case, into sh[v], in a fixed
+// order (lines that divide a wave: a butterfly, then the waves; else a tree in LDS);
+// every thread may read sh[v] afterwards.  sh: LINE_SUM doubles of LDS
+constexpr int LINE_SUM = 512 + LINE_CASES;
+template <int W>
+__device__ __forceinline__ void lines_sum(Vals<W> val, const Lines<W> &L, int K, double *sh) {
+    if ((L.width & (L.width - 1)) == 0) {
+        const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+#pragma unroll
+        for (int i = 0; i < W; i++)
+            for (int o = 32; o >= L.width; o >>= 1) val.d[i] += __shfl_xor(val.d[i], o, 64);
         __syncthreads();
+        if (lane < L.width)
+#pragma unroll
+            for (int i = 0; i < W; i++) sh[(w + 1) * K + L.v + i] = val.d[i];
+        __syncthreads();
+        if ((int)threadIdx.x < K) {
+            double s = 0.0;
+            for (int i = 1; i <= nw; i++) s += sh[i * K + threadIdx.x];
+            sh[threadIdx.x] = s;
+        }
+        __syncthreads();
+        return;
     }
+    // at most 512 threads: the second value of a thread in a second turn
+    double *t = sh + LINE_CASES;
+    double sum[W];
+#pragma unroll
+    for (int i = 0; i < W; i++) {
+        __syncthreads();
+        t[threadIdx.x] = L.on ? val.d[i] : 0.0;
+        __syncthreads();
+        int h = 1;
+        while (2 * h < L.per) h *= 2;
+        for (; h > 0; h >>= 1) {
+            if (L.on && L.li < h && L.li + h < L.per) t[threadIdx.x] += t[threadIdx.x + h * L.width];
+            __syncthreads();
+        }
+        sum[i] = t[threadIdx.x];
+    }
+    if (L.li == 0)
+#pragma unroll
+        for (int i = 0; i < W; i++) sh[L.v + i] = sum[i];
+    __syncthreads();
 }
 
 // sum of np partials per case, part[b K + v], into sh[v]
-__device__ __forceinline__ void partials_sum(const double *__restrict__ part, int np, const Lines &L, int K,
+template <int W>
+__device__ __forceinline__ void partials_sum(const double *__restrict__ part, int np, const Lines<W> &L, int K,
                                              double *sh) {
-    double a = 0.0;
+    Vals<W> a = {};
     if (L.on)
-        for (int b = L.li; b < np; b += L.per) a += part[(int64_t)b * K + L.v];
+#pragma unroll 4
+        for (int b = L.li; b < np; b += L.per) {
+            const Vals<W> x = line_load<W>(part + (int64_t)b * K + L.v);
+#pragma unroll
+            for (int i = 0; i < W; i++) a.d[i] += x.d[i];
+        }
     lines_sum(a, L, K, sh);
 }
 
 constexpr int LINE_THREADS_1 = 256, LINE_THREADS_K = 512;
 static inline int line_threads(int K) { return K == 1 ? LINE_THREADS_1 : LINE_THREADS_K; }
+// lines per workgroup
+static inline int64_t line_per(int K) { return line_threads(K) / (K % 2 ? K : K / 2); }
 // workgroups of a pass over n lines that sums a dot product: one partial each.
 // At most 4 (K = 1) or 2 workgroups per CU: the consumer of the partials reads
 // them all in every workgroup
 int dot_blocks(int64_t n, int K) {
-    const int64_t per = line_threads(K) / K;
+    const int64_t per = line_per(K);
     return (int)std::max<int64_t>(1, std::min<int64_t>((n + per - 1) / per, K == 1 ? 1024 : 512));
 }
 static inline unsigned line_grid(int64_t n, int K) {
-    const int64_t per = line_threads(K) / K;
+    const int64_t per = line_per(K);
     return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + per - 1) / per, 4096));
 }
+// kernel<W> for K cases
+#define ESP_LINES(KERNEL, K, grid, ...)                                                                            \
+    do {                                                                                                           \
+        if ((K) % 2)                                                                                               \
+            hipLaunchKernelGGL(KERNEL<1>, dim3(grid), dim3(line_threads(K)), 0, st, __VA_ARGS__);                  \
+        else                                                                                                       \
+            hipLaunchKernelGGL(KERNEL<2>, dim3(grid), dim3(line_threads(K)), 0, st, __VA_ARGS__);                  \
+    } while (0)
 
 // ---- set-up of the derived maps ----
 // bl_row[q]: boundary DOF of entry q of the boundary -> lambda CSR
@@ -131,7 +207,10 @@ void launch_lambda_coarse(const DualDev &D, LamCoarse *le, hipStream_t st) {
 // yb[(boff + j) K + v] = sum of the partials of the items of subdomain s that
 // cover j.  A partial starts at its item's first row j0, so the interleaved
 // index i = j K + v of the item's own values is i - j0 K: no division, and the
-// item list is uniform over the workgroup (scalar loads).  grid (chunks, subdomains)
+// item list is uniform over the workgroup (scalar loads).  An item that starts
+// below i is read at its start and left out (no branch between the loads).  grid
+// (chunks, subdomains); bound by the partials (16 cases: 2.4 times the result)
+template <int W>
 __global__ void __launch_bounds__(256) k_part_reduce(const SymvItem *__restrict__ items, const int *__restrict__ item0,
                                                      const int *__restrict__ nitems, const int *__restrict__ M,
                                                      const int64_t *__restrict__ boff, int R, int K,
@@ -140,32 +219,44 @@ __global__ void __launch_bounds__(256) k_part_reduce(const SymvItem *__restrict_
     const int64_t n = (int64_t)M[s] * K;
     const int i0 = item0[s], ni = nitems[s];
     double *y = yb + boff[s] * K;
-    for (int64_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-        double v = 0.0;
+    for (int64_t i = (blockIdx.x * 256 + threadIdx.x) * W; i < n; i += (int64_t)gridDim.x * 256 * W) {
+        Vals<W> v = {};
+#pragma unroll 4
         for (int q = 0; q < ni; q++) {
             const SymvItem it = items[i0 + q];
             const int64_t lo = (int64_t)it.t0 * R * K;
-            if (i >= lo) v += ypart[it.part_off * K + i - lo];
+            const Vals<W> x = line_load<W>(ypart + it.part_off * K + (i >= lo ? i - lo : 0));
+#pragma unroll
+            for (int k = 0; k < W; k++) v.d[k] += i >= lo ? x.d[k] : 0.0;
         }
-        y[i] = v;
+        line_store<W>(y + i, v);
     }
 }
 
-// y[l K + v] = sum_e coef_e yb[b_e K + v]; with `a`, part gets the partial dot
-// products of y with a
+// y[l K + v] = sum_e coef_e yb[b_e K + v] (one or two entries); with `a`, part gets
+// the partial dot products of y with a
+template <int W>
 __global__ void k_lambda_gather(int nlam, int K, const int *__restrict__ cnt, const int64_t *__restrict__ lb,
                                 const double *__restrict__ coef, const double *__restrict__ yb, double *__restrict__ y,
                                 const double *__restrict__ a, double *__restrict__ part) {
-    extern __shared__ double sh[];
-    const Lines L = lines_of(K);
-    double dot = 0.0;
+    __shared__ double sh[LINE_SUM];
+    const Lines<W> L(K);
+    Vals<W> dot = {};
     if (L.on)
         for (int64_t l = (int64_t)blockIdx.x * L.per + L.li; l < nlam; l += (int64_t)gridDim.x * L.per) {
-            double v = 0.0;
-            const int c = cnt[l];
-            for (int e = 0; e < c; e++) v += coef[2 * l + e] * yb[lb[2 * l + e] * K + L.v];
-            y[l * K + L.v] = v;
-            if (a) dot += v * a[l * K + L.v];
+            const bool two = cnt[l] > 1;
+            const int64_t b0 = lb[2 * l], b1 = lb[2 * l + 1];
+            const double c0 = coef[2 * l], c1 = coef[2 * l + 1];
+            const Vals<W> x0 = line_load<W>(yb + b0 * K + L.v), x1 = line_load<W>(yb + (two ? b1 : b0) * K + L.v);
+            Vals<W> v, av = {};
+            if (a) av = line_load<W>(a + l * K + L.v);
+#pragma unroll
+            for (int i = 0; i < W; i++) {
+                v.d[i] = c0 * x0.d[i];
+                if (two) v.d[i] += c1 * x1.d[i];
+                dot.d[i] += v.d[i] * av.d[i];
+            }
+            line_store<W>(y + l * K + L.v, v);
         }
     if (!a) return;  // uniform
     lines_sum(dot, L, K, sh);
@@ -173,16 +264,22 @@ __global__ void k_lambda_gather(int nlam, int K, const int *__restrict__ cnt, co
 }
 
 // xb[j K + v] = sum coef x[lambda K + v]
+template <int W>
 __global__ void k_boundary_gather(int64_t nb, int K, const int64_t *__restrict__ bl_ptr,
                                   const int *__restrict__ bl_lam, const double *__restrict__ coef,
                                   const double *__restrict__ x, double *__restrict__ xb) {
-    const Lines L = lines_of(K);
+    const Lines<W> L(K);
     if (!L.on) return;
     for (int64_t j = (int64_t)blockIdx.x * L.per + L.li; j < nb; j += (int64_t)gridDim.x * L.per) {
-        double v = 0.0;
+        Vals<W> v = {};
         const int64_t q1 = bl_ptr[j + 1];
-        for (int64_t q = bl_ptr[j]; q < q1; q++) v += coef[q] * x[(int64_t)bl_lam[q] * K + L.v];
-        xb[j * K + L.v] = v;
+        for (int64_t q = bl_ptr[j]; q < q1; q++) {
+            const double c = coef[q];
+            const Vals<W> xl = line_load<W>(x + (int64_t)bl_lam[q] * K + L.v);
+#pragma unroll
+            for (int i = 0; i < W; i++) v.d[i] += c * xl.d[i];
+        }
+        line_store<W>(xb + j * K + L.v, v);
     }
 }
 
@@ -205,7 +302,7 @@ __global__ void __launch_bounds__(256) k_kbb_rows(int64_t nb, const int64_t *__r
 }
 __global__ void k_kbb_lines(int64_t nb, int K, const int64_t *__restrict__ ptr, const int64_t *__restrict__ col,
                             const double *__restrict__ val, const double *__restrict__ xb, double *__restrict__ yb) {
-    const Lines L = lines_of(K);
+    const Lines<1> L(K);
     if (!L.on) return;
     for (int64_t j = (int64_t)blockIdx.x * L.per + L.li; j < nb; j += (int64_t)gridDim.x * L.per) {
         double v = 0.0;
@@ -220,7 +317,7 @@ __global__ void k_kbb_lines(int64_t nb, int K, const int64_t *__restrict__ ptr, 
 // DOFs next to the boundary, then y_b = K_bb x_b - K_bn t
 __global__ void k_superdir_near(int64_t n_near, int K, const int64_t *ptr, const int64_t *col, const double *val,
                                 const double *diag, const double *xb, double *t) {
-    const Lines L = lines_of(K);
+    const Lines<1> L(K);
     if (!L.on) return;
     for (int64_t g = (int64_t)blockIdx.x * L.per + L.li; g < n_near; g += (int64_t)gridDim.x * L.per) {
         double v = 0.0;
@@ -231,7 +328,7 @@ __global__ void k_superdir_near(int64_t n_near, int K, const int64_t *ptr, const
 __global__ void k_superdir_bnd(int64_t nb, int K, const int64_t *kptr, const int64_t *kcol, const double *kval,
                                const int64_t *ptr, const int64_t *col, const double *val, const double *xb,
                                const double *t, double *yb) {
-    const Lines L = lines_of(K);
+    const Lines<1> L(K);
     if (!L.on) return;
     for (int64_t j = (int64_t)blockIdx.x * L.per + L.li; j < nb; j += (int64_t)gridDim.x * L.per) {
         double v = 0.0;
@@ -252,61 +349,89 @@ __global__ void k_superdir_bnd(int64_t nb, int K, const int64_t *kptr, const int
 // 40 us at 2000 heat subdomains of ~330 entries).  One workgroup per subdomain.
 // stop != null (first pass of an iteration): workgroup 0 copies the stop flags
 // that the previous iteration decided (slot PCG_NEXT) to the ones this one obeys.
-template <bool ONE>
+// KB columns of the basis per pass (heat has one, elasticity six); one case reduces
+// them together (a butterfly per column is 6 shuffles each).  Bound by the gather of x
+// and the rows: 16 cases at 2000 heat subdomains 140 -> 47 us, 5 cases at 512 elasticity
+// subdomains 56 -> 28 us (rows as 16-byte loads without a branch, cases in pairs, one LDS
+// exchange for all columns), one case at 512 of 1806 boundary DOFs 25.6 -> 18.3 us.
+template <int W, int KB>
 __global__ void k_apply_G(const int *__restrict__ M, const int64_t *__restrict__ boff, const int *__restrict__ kcols,
                           const int64_t *__restrict__ outoff, const int64_t *__restrict__ roff,
                           const double *__restrict__ RT, const int64_t *__restrict__ bl_ptr,
                           const int *__restrict__ bl_lam, const int *__restrict__ bl_row,
                           const double *__restrict__ sign, int K, const double *__restrict__ x,
                           double *__restrict__ out, double *stop) {
-    constexpr int KB = 8;  // columns per pass
-    extern __shared__ double sh[];
+    __shared__ double sh[KB * 16 * LINE_CASES];  // [column][wave][case]
     const int s = blockIdx.x, k = kcols[s];
     if (stop && s == 0 && (int)threadIdx.x < K)
         stop[threadIdx.x * PCG_SLOTS + PCG_STOP] = stop[threadIdx.x * PCG_SLOTS + PCG_NEXT];
-    const int64_t b0 = boff[s], q0 = bl_ptr[b0], q1 = bl_ptr[b0 + M[s]];
+    const int64_t b0 = boff[s], q0 = bl_ptr[b0];
+    const int n = (int)(bl_ptr[b0 + M[s]] - q0);
     const double *Rs = RT + roff[s];
-    const Lines L = lines_of(ONE ? 1 : K);
+    const Lines<W> L(K, true);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    constexpr int UNR = W == 2 ? 2 : 4;  // four pairs take so many registers that one workgroup fits a CU (62 us, not 47)
     for (int a0 = 0; a0 < k; a0 += KB) {
         const int kb = min(KB, k - a0);
-        double acc[KB];
-#pragma unroll
-        for (int a = 0; a < KB; a++) acc[a] = 0.0;
+        Vals<W> acc[KB] = {};
         if (L.on) {
-#pragma unroll 4
-            for (int64_t q = q0 + L.li; q < q1; q += L.per) {
-                const double xv = sign[q] * x[(int64_t)bl_lam[q] * (ONE ? 1 : K) + L.v];
-                const double *r = Rs + (bl_row[q] - b0) * k + a0;
+            auto entry = [&](int q, bool full) {
+                const double sg = sign[q0 + q];
+                const Vals<W> xv = line_load<W>(x + (int64_t)bl_lam[q0 + q] * K + L.v);
+                const double *r = Rs + (bl_row[q0 + q] - b0) * k + a0;
+                double ra[KB];
+                if (full) {
+                    if constexpr (KB % 2 == 0) {
+#pragma unroll
+                        for (int a = 0; a < KB; a += 2) {
+                            const d2u rr = *(const d2u *)(r + a);
+                            ra[a] = rr[0];
+                            ra[a + 1] = rr[1];
+                        }
+                    } else {
+                        ra[0] = r[0];
+                    }
+                } else {
+#pragma unroll
+                    for (int a = 0; a < KB; a++) ra[a] = a < kb ? r[a] : 0.0;
+                }
 #pragma unroll
                 for (int a = 0; a < KB; a++)
-                    if (a < kb) acc[a] += r[a] * xv;
+#pragma unroll
+                    for (int i = 0; i < W; i++) acc[a].d[i] += ra[a] * (sg * xv.d[i]);
+            };
+            // no branch between the loads of the usual case
+            if (kb == KB) {
+#pragma unroll UNR
+                for (int q = L.li; q < n; q += L.per) entry(q, true);
+            } else {
+                for (int q = L.li; q < n; q += L.per) entry(q, false);
             }
         }
-        if constexpr (ONE) {
-            const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+        __syncthreads();
+        if (KB == 6 && W == 1 && L.width == 1) {
+            double v[8];
 #pragma unroll
-            for (int a = 0; a < KB; a++) {
-                if (a >= kb) break;
-                double v = acc[a];
-                for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-                if (lane == 0) sh[a * 16 + w] = v;
-            }
-            __syncthreads();
-            if ((int)threadIdx.x < kb) {
-                double v = 0.0;
-                for (int q = 0; q < nw; q++) v += sh[threadIdx.x * 16 + q];
-                out[outoff[s] + a0 + threadIdx.x] = -v;
-            }
-            __syncthreads();
+            for (int a = 0; a < 8; a++) v[a] = a < KB ? acc[a % KB].d[0] : 0.0;
+            const double t = wave_rows_reduce<8, double>(v, lane);
+            if ((lane & 7) == 0 && lane < 8 * KB) sh[(lane >> 3) * 16 + w] = t;
         } else {
-            for (int a = 0; a < kb; a++) {
-                double v = 0.0;
 #pragma unroll
-                for (int b = 0; b < KB; b++)
-                    if (b == a) v = acc[b];
-                lines_sum(v, L, K, sh);
-                if ((int)threadIdx.x < K) out[(outoff[s] + a0 + a) * K + threadIdx.x] = -sh[threadIdx.x];
-            }
+            for (int a = 0; a < KB; a++)
+                if (a < kb)
+#pragma unroll
+                    for (int i = 0; i < W; i++) {
+                        double v = acc[a].d[i];
+                        for (int o = 32; o >= L.width; o >>= 1) v += __shfl_xor(v, o, 64);
+                        if (lane < L.width && L.on) sh[(a * 16 + w) * K + L.v + i] = v;
+                    }
+        }
+        __syncthreads();
+        for (int c = threadIdx.x; c < kb * K; c += blockDim.x) {
+            const int a = c / K, v = c - a * K;
+            double t = 0.0;
+            for (int q = 0; q < nw; q++) t += sh[(a * 16 + q) * K + v];
+            out[(outoff[s] + a0 + a) * K + v] = -t;
         }
     }
 }
@@ -342,19 +467,20 @@ __global__ void __launch_bounds__(256) k_coarse_gemv(int nc, const double *__res
 }
 
 // e = GGinv d for K <= 16 cases on MFMA (the N dimension of v_mfma_f64_16x16x4f64):
-// GGinv is read once for all cases.  One workgroup per 16 rows, its four waves
-// take every fourth chunk of 16 columns and meet in LDS in a fixed order.  A lane
+// GGinv is read once for all cases.  One workgroup per 16 rows, its 16 waves
+// take every 16th chunk of 16 columns and meet in LDS in a fixed order (four waves
+// leave too little in flight with one workgroup a CU: 47 us at 3072 columns, now 32).  A lane
 // loads four consecutive columns of its row (32 B of the 128 B line that four
 // lanes share) and the matching rows of d; products of columns past nc are zero.
-__global__ void __launch_bounds__(256) k_coarse_block(int nc, int K, const double *__restrict__ Ginv,
+__global__ void __launch_bounds__(1024) k_coarse_block(int nc, int K, const double *__restrict__ Ginv,
                                                       const double *__restrict__ d, double *__restrict__ e) {
-    __shared__ double sum[4][256];
+    __shared__ double sum[16][256];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, l16 = lane & 15, kq = lane >> 4;
     const int i0 = blockIdx.x * 16;
     const double *row = Ginv + (int64_t)min(i0 + l16, nc - 1) * nc;
     const int v = min(l16, K - 1);
     v4d acc = {0.0, 0.0, 0.0, 0.0};
-    for (int k0 = 16 * w; k0 < nc; k0 += 64) {
+        for (int k0 = 16 * w; k0 < nc; k0 += 256) {
         double a[4], b[4];
 #pragma unroll
         for (int s = 0; s < 4; s++) {
@@ -370,41 +496,78 @@ __global__ void __launch_bounds__(256) k_coarse_block(int nc, int K, const doubl
 #pragma unroll
     for (int q = 0; q < 4; q++) sum[w][(kq + 4 * q) * 16 + l16] = acc[q];
     __syncthreads();
+    if (threadIdx.x >= 256) return;
     const int r = threadIdx.x >> 4, c = threadIdx.x & 15;
-    if (i0 + r < nc && c < K)
-        e[(int64_t)(i0 + r) * K + c] =
-            (sum[0][threadIdx.x] + sum[1][threadIdx.x]) + (sum[2][threadIdx.x] + sum[3][threadIdx.x]);
+    double v2 = 0.0;
+#pragma unroll
+    for (int q = 0; q < 16; q++) v2 += sum[q][threadIdx.x];
+    if (i0 + r < nc && c < K) e[(int64_t)(i0 + r) * K + c] = v2;
 }
 
 // mode 0: y = x - G^T e ; mode 1: y = G^T e, (G^T e)_l = -sum_entries sign Rt(row) e_blk.
 // with `part`: partial dot products of y with a (a == null: with y itself)
+template <int W>
 __global__ void k_project_finish(int nlam, int K, const int *__restrict__ cnt, const LamCoarse *__restrict__ lc,
                                  const double *__restrict__ sign, const double *__restrict__ RT,
                                  const double *__restrict__ e, const double *x, double *y, int mode,
                                  const double *__restrict__ a, double *__restrict__ part) {
-    extern __shared__ double sh[];
-    const Lines L = lines_of(K);
-    double dot = 0.0;
+    __shared__ double sh[LINE_SUM];
+    const Lines<W> L(K);
+    Vals<W> dot = {};
     if (L.on)
         for (int64_t l = (int64_t)blockIdx.x * L.per + L.li; l < nlam; l += (int64_t)gridDim.x * L.per) {
-            double g = 0.0;
-            const int c = cnt[l];
-            for (int q = 0; q < c; q++) {
-                const LamCoarse t = lc[2 * l + q];
-                const double *r = RT + t.row, *es = e + (int64_t)t.off * K + L.v;
-                double acc = 0.0;
-                if (t.k == 6) {  // rigid motions in space: the row as three 16-byte loads
-                    const d2u r0 = *(const d2u *)r, r1 = *(const d2u *)(r + 2), r2 = *(const d2u *)(r + 4);
-                    acc = r0[0] * es[0] + r0[1] * es[K] + r1[0] * es[2 * K] + r1[1] * es[3 * K] + r2[0] * es[4 * K] +
-                          r2[1] * es[5 * K];
-                } else {
-                    for (int b = 0; b < t.k; b++) acc += r[b] * es[(int64_t)b * K];
+            // both entries, x and a are loaded before the first is used
+            LamCoarse t[2] = {lc[2 * l], lc[2 * l + 1]};
+            if (cnt[l] < 2) t[1].k = 0;
+            const double sg[2] = {sign[2 * l], sign[2 * l + 1]};
+            Vals<W> g = {}, v = {}, av = {};
+            if (mode == 0) v = line_load<W>(x + l * K + L.v);
+            if (a) av = line_load<W>(a + l * K + L.v);
+            if (t[0].k <= 1 && t[1].k <= 1) {  // one column (heat) or none (any value is read, and not used)
+                double r[2];
+                Vals<W> ev[2];
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    const bool on = t[q].k > 0;
+                    r[q] = *(on ? RT + t[q].row : sign);
+                    ev[q] = line_load<W>(on ? e + (int64_t)t[q].off * K + L.v : y + l * K + L.v);
                 }
-                g -= sign[2 * l + q] * acc;
+#pragma unroll
+                for (int q = 0; q < 2; q++)
+                    if (t[q].k > 0)
+#pragma unroll
+                        for (int i = 0; i < W; i++) g.d[i] -= sg[q] * (r[q] * ev[q].d[i]);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 2; q++) {
+                    const double *r = RT + t[q].row, *es = e + (int64_t)t[q].off * K + L.v;
+                    Vals<W> acc = {};
+                    if (t[q].k == 6) {  // rigid motions in space: the row as three 16-byte loads
+                        const d2u rr[3] = {*(const d2u *)r, *(const d2u *)(r + 2), *(const d2u *)(r + 4)};
+                        Vals<W> ev[6];
+#pragma unroll
+                        for (int b = 0; b < 6; b++) ev[b] = line_load<W>(es + b * K);
+#pragma unroll
+                        for (int b = 0; b < 6; b++)
+#pragma unroll
+                            for (int i = 0; i < W; i++) acc.d[i] += rr[b >> 1][b & 1] * ev[b].d[i];
+                    } else {
+                        for (int b = 0; b < t[q].k; b++) {
+                            const Vals<W> ev = line_load<W>(es + b * K);
+#pragma unroll
+                            for (int i = 0; i < W; i++) acc.d[i] += r[b] * ev.d[i];
+                        }
+                    }
+#pragma unroll
+                    for (int i = 0; i < W; i++) g.d[i] -= sg[q] * acc.d[i];
+                }
             }
-            const double v = mode == 0 ? x[l * K + L.v] - g : g;
-            y[l * K + L.v] = v;
-            if (part) dot += v * (a ? a[l * K + L.v] : v);
+#pragma unroll
+            for (int i = 0; i < W; i++) {
+                v.d[i] = mode == 0 ? v.d[i] - g.d[i] : g.d[i];
+                if (part) dot.d[i] += v.d[i] * (a ? av.d[i] : v.d[i]);
+            }
+            line_store<W>(y + l * K + L.v, v);
         }
     if (!part) return;  // uniform
     lines_sum(dot, L, K, sh);
@@ -412,14 +575,18 @@ __global__ void k_project_finish(int nlam, int K, const int *__restrict__ cnt, c
 }
 
 // ---- dots and updates ----
+template <int W>
 __global__ void k_dot_lines(int64_t n, int K, const double *__restrict__ a, const double *__restrict__ b,
                             double *__restrict__ part) {
-    extern __shared__ double sh[];
-    const Lines L = lines_of(K);
-    double dot = 0.0;
+    __shared__ double sh[LINE_SUM];
+    const Lines<W> L(K);
+    Vals<W> dot = {};
     if (L.on)
-        for (int64_t l = (int64_t)blockIdx.x * L.per + L.li; l < n; l += (int64_t)gridDim.x * L.per)
-            dot += a[l * K + L.v] * b[l * K + L.v];
+        for (int64_t l = (int64_t)blockIdx.x * L.per + L.li; l < n; l += (int64_t)gridDim.x * L.per) {
+            const Vals<W> x = line_load<W>(a + l * K + L.v), z = line_load<W>(b + l * K + L.v);
+#pragma unroll
+            for (int i = 0; i < W; i++) dot.d[i] += x.d[i] * z.d[i];
+        }
     lines_sum(dot, L, K, sh);
     if ((int)threadIdx.x < K) part[(int64_t)blockIdx.x * K + threadIdx.x] = sh[threadIdx.x];
 }
@@ -428,8 +595,8 @@ __global__ void k_dot_lines(int64_t n, int K, const double *__restrict__ a, cons
 // tol = precision min(||P r0||, ||b||), or tol_abs when that is positive
 __global__ void __launch_bounds__(256) k_pcg_init(int K, const double *part_r, const double *part_b, int np,
                                                   double precision, double tol_abs, double *scal, PcgRecord *rec) {
-    __shared__ double sh[256], rr[16];
-    const Lines L = lines_of(K);
+    __shared__ double sh[LINE_SUM], rr[LINE_CASES];
+    const Lines<1> L(K);
     partials_sum(part_r, np, L, K, sh);
     const int v = threadIdx.x;
     if (v < K) rr[v] = sh[v];
@@ -449,18 +616,32 @@ __global__ void __launch_bounds__(256) k_pcg_init(int K, const double *part_r, c
 // of the next iteration (||w|| < tol, or not finite) and reports to the host
 // record (pinned memory): the host queues the next iteration, or not, while the
 // dual operator of this one runs, so the stop test costs no wait on either side.
+template <int W>
 __global__ void k_p_update(int64_t n, int K, double *__restrict__ p, const double *__restrict__ y,
                            const double *__restrict__ part_yw, const double *__restrict__ part_ww, int np, int first,
                            double *scal, PcgRecord *rec) {
-    extern __shared__ double sh[];
-    const Lines L = lines_of(K);
+    __shared__ double sh[LINE_SUM], yws[LINE_CASES];
+    const Lines<W> L(K);
     partials_sum(part_yw, np, L, K, sh);
-    const double yw = sh[L.v], prev = scal[L.v * PCG_SLOTS + PCG_YW_PREV];
-    const bool run = L.on && scal[L.v * PCG_SLOTS + PCG_STOP] == 0.0;
-    const double beta = first ? 0.0 : yw / prev;
-    if (run)
-        for (int64_t l = (int64_t)blockIdx.x * L.per + L.li; l < n; l += (int64_t)gridDim.x * L.per)
-            p[l * K + L.v] = first ? y[l * K + L.v] : y[l * K + L.v] + beta * p[l * K + L.v];
+    if ((int)threadIdx.x < K) yws[threadIdx.x] = sh[threadIdx.x];
+    double beta[W];
+    bool run[W], any_run = false;
+#pragma unroll
+    for (int i = 0; i < W; i++) {
+        const double *s = scal + (L.v + i) * PCG_SLOTS;
+        run[i] = L.on && s[PCG_STOP] == 0.0;
+        beta[i] = first ? 0.0 : sh[L.v + i] / s[PCG_YW_PREV];
+        any_run |= run[i];
+    }
+    if (any_run)
+        for (int64_t l = (int64_t)blockIdx.x * L.per + L.li; l < n; l += (int64_t)gridDim.x * L.per) {
+            const Vals<W> yv = line_load<W>(y + l * K + L.v);
+            Vals<W> pv = line_load<W>(p + l * K + L.v);
+#pragma unroll
+            for (int i = 0; i < W; i++)
+                if (run[i]) pv.d[i] = first ? yv.d[i] : yv.d[i] + beta[i] * pv.d[i];
+            line_store<W>(p + l * K + L.v, pv);
+        }
     if (blockIdx.x) return;
     partials_sum(part_ww, np, L, K, sh);
     if (threadIdx.x >= 64) return;
@@ -468,10 +649,10 @@ __global__ void k_p_update(int64_t n, int K, double *__restrict__ p, const doubl
     int active = 0;
     if (v < K) {
         double *s = scal + v * PCG_SLOTS;
-        if (run) {
+        if (s[PCG_STOP] == 0.0) {
             const double ww = sh[v];
             const bool stop = sqrt(ww) < s[PCG_TOL] || !isfinite(ww);
-            s[PCG_YW] = yw;
+            s[PCG_YW] = yws[v];
             s[PCG_WW] = ww;
             s[PCG_ITERS] += 1.0;
             s[PCG_NEXT] = stop ? 1.0 : 0.0;
@@ -490,28 +671,48 @@ __global__ void k_p_update(int64_t n, int K, double *__restrict__ p, const doubl
 }
 
 // alpha = yw / pAp; x += alpha p; r -= alpha Ap of the cases that still run
+template <int W>
 __global__ void k_xr_update(int64_t n, int K, double *__restrict__ x, double *__restrict__ r,
                             const double *__restrict__ p, const double *__restrict__ Ap,
                             const double *__restrict__ part_pAp, int np, double *scal) {
-    extern __shared__ double sh[];
-    const Lines L = lines_of(K);
+    __shared__ double sh[LINE_SUM];
+    const Lines<W> L(K);
     partials_sum(part_pAp, np, L, K, sh);
-    const double yw = scal[L.v * PCG_SLOTS + PCG_YW], alpha = yw / sh[L.v];
-    const bool run = L.on && scal[L.v * PCG_SLOTS + PCG_STOP] == 0.0;
-    if (!run) return;
-    for (int64_t l = (int64_t)blockIdx.x * L.per + L.li; l < n; l += (int64_t)gridDim.x * L.per) {
-        x[l * K + L.v] += alpha * p[l * K + L.v];
-        r[l * K + L.v] -= alpha * Ap[l * K + L.v];
+    double alpha[W];
+    bool run[W], any = false;
+#pragma unroll
+    for (int i = 0; i < W; i++) {
+        const double *s = scal + (L.v + i) * PCG_SLOTS;
+        run[i] = L.on && s[PCG_STOP] == 0.0;
+        alpha[i] = s[PCG_YW] / sh[L.v + i];
+        any |= run[i];
     }
+    if (any)
+        for (int64_t l = (int64_t)blockIdx.x * L.per + L.li; l < n; l += (int64_t)gridDim.x * L.per) {
+            const int64_t o = l * K + L.v;
+            const Vals<W> pv = line_load<W>(p + o), Av = line_load<W>(Ap + o);
+            Vals<W> xv = line_load<W>(x + o), rv = line_load<W>(r + o);
+#pragma unroll
+            for (int i = 0; i < W; i++)
+                if (run[i]) {
+                    xv.d[i] += alpha[i] * pv.d[i];
+                    rv.d[i] -= alpha[i] * Av.d[i];
+                }
+            line_store<W>(x + o, xv);
+            line_store<W>(r + o, rv);
+        }
     if (blockIdx.x == 0 && (int)threadIdx.x < K) {
-        scal[threadIdx.x * PCG_SLOTS + PCG_PAP] = sh[threadIdx.x];
-        scal[threadIdx.x * PCG_SLOTS + PCG_YW_PREV] = yw;  // read by the next iteration only
+        double *s = scal + threadIdx.x * PCG_SLOTS;
+        if (s[PCG_STOP] == 0.0) {
+            s[PCG_PAP] = sh[threadIdx.x];
+            s[PCG_YW_PREV] = s[PCG_YW];  // read by the next iteration only
+        }
     }
 }
 
 // y_v -= c for every case
 __global__ void k_sub_lines(int64_t n, int K, double *__restrict__ y, const double *__restrict__ c) {
-    const Lines L = lines_of(K);
+    const Lines<1> L(K);
     if (!L.on) return;
     for (int64_t l = (int64_t)blockIdx.x * L.per + L.li; l < n; l += (int64_t)gridDim.x * L.per) y[l * K + L.v] -= c[l];
 }
@@ -523,22 +724,25 @@ void launch_sub_lines(int64_t n, int K, double *y, const double *c, hipStream_t 
 
 void launch_part_reduce(const DualDev &D, const SymvItem *items, const int *item0, const int *nitems, int R, int K,
                         const double *ypart, double *yb, hipStream_t st) {
-    const unsigned g = std::max(1u, std::min(cdiv((int64_t)D.max_m * K, 256), 64u));
-    hipLaunchKernelGGL(k_part_reduce, dim3(g, D.nsub), dim3(256), 0, st, items, item0, nitems, D.m, D.boff, R, K, ypart,
-                       yb);
+    const int W = K % 2 ? 1 : 2;
+    const unsigned g = std::max(1u, std::min(cdiv((int64_t)D.max_m * K, 256 * W), 64u));
+    if (W == 1)
+        hipLaunchKernelGGL(k_part_reduce<1>, dim3(g, D.nsub), dim3(256), 0, st, items, item0, nitems, D.m, D.boff, R, K,
+                           ypart, yb);
+    else
+        hipLaunchKernelGGL(k_part_reduce<2>, dim3(g, D.nsub), dim3(256), 0, st, items, item0, nitems, D.m, D.boff, R, K,
+                           ypart, yb);
 }
 
 void launch_lambda_gather(const DualDev &D, int K, const double *yb, bool scaled, double *y, hipStream_t st,
                           const double *a, double *part) {
-    const int T = line_threads(K);
-    hipLaunchKernelGGL(k_lambda_gather, dim3(part ? (unsigned)dot_blocks(D.nlam, K) : line_grid(D.nlam, K)), dim3(T),
-                       part ? T * sizeof(double) : 0, st, D.nlam, K, D.le_cnt, D.le_b,
-                       scaled ? D.le_sscale : D.le_sign, yb, y, a, part);
+    ESP_LINES(k_lambda_gather, K, part ? (unsigned)dot_blocks(D.nlam, K) : line_grid(D.nlam, K), D.nlam, K, D.le_cnt,
+              D.le_b, scaled ? D.le_sscale : D.le_sign, yb, y, a, part);
 }
 
 void launch_boundary_gather(const DualDev &D, int K, const double *x, bool scaled, double *xb, hipStream_t st) {
-    hipLaunchKernelGGL(k_boundary_gather, dim3(line_grid(D.nbnd, K)), dim3(line_threads(K)), 0, st, D.nbnd, K, D.bl_ptr,
-                       D.bl_lam, scaled ? D.bl_sscale : D.bl_sign, x, xb);
+    ESP_LINES(k_boundary_gather, K, line_grid(D.nbnd, K), D.nbnd, K, D.bl_ptr, D.bl_lam,
+              scaled ? D.bl_sscale : D.bl_sign, x, xb);
 }
 
 void launch_kbb(const DualDev &D, int K, const double *xb, double *yb, hipStream_t st) {
@@ -568,12 +772,17 @@ static void apply_G(const DualDev &D, int K, const int *kcols, const int64_t *ou
                     const double *RT, const double *x, double *out, double *stop, hipStream_t st) {
     const int64_t e = D.nle * K / std::max(D.nsub, 1) / 2;
     const int T = e <= 256 ? 256 : e <= 512 ? 512 : 1024;
-    if (K == 1)
-        hipLaunchKernelGGL(k_apply_G<true>, dim3(D.nsub), dim3(T), 8 * 16 * sizeof(double), st, D.m, D.boff, kcols,
-                           outoff, roff, RT, D.bl_ptr, D.bl_lam, D.bl_row, D.bl_sign, 1, x, out, stop);
-    else
-        hipLaunchKernelGGL(k_apply_G<false>, dim3(D.nsub), dim3(T), T * sizeof(double), st, D.m, D.boff, kcols, outoff,
-                           roff, RT, D.bl_ptr, D.bl_lam, D.bl_row, D.bl_sign, K, x, out, stop);
+#define ESP_APPLY_G(W, KB)                                                                                          \
+    hipLaunchKernelGGL((k_apply_G<W, KB>), dim3(D.nsub), dim3(T), 0, st, D.m, D.boff, kcols, outoff, roff, RT, D.bl_ptr, \
+                       D.bl_lam, D.bl_row, D.bl_sign, K, x, out, stop)
+    if (D.max_k == 1) {
+        if (K % 2) ESP_APPLY_G(1, 1);
+        else ESP_APPLY_G(2, 1);
+    } else {
+        if (K % 2) ESP_APPLY_G(1, 6);
+        else ESP_APPLY_G(2, 6);
+    }
+#undef ESP_APPLY_G
 }
 
 void launch_project(const DualDev &D, int K, const double *x, double *y, int mode, hipStream_t st, const double *a,
@@ -594,13 +803,11 @@ void launch_project(const DualDev &D, int K, const double *x, double *y, int mod
     if (K == 1)
         hipLaunchKernelGGL(k_coarse_gemv, dim3(D.ncoarse), dim3(256), 0, st, D.ncoarse, D.GGinv, din, eout);
     else
-        hipLaunchKernelGGL(k_coarse_block, dim3(cdiv(D.ncoarse, 16)), dim3(256), 0, st, D.ncoarse, K, D.GGinv, din,
+        hipLaunchKernelGGL(k_coarse_block, dim3(cdiv(D.ncoarse, 16)), dim3(1024), 0, st, D.ncoarse, K, D.GGinv, din,
                            eout);
     if (mode == 2) return;
-    const int T = line_threads(K);
-    hipLaunchKernelGGL(k_project_finish, dim3(part ? (unsigned)dot_blocks(D.nlam, K) : line_grid(D.nlam, K)), dim3(T),
-                       part ? T * sizeof(double) : 0, st, D.nlam, K, D.le_cnt, D.le_coarse, D.le_sign, D.RtT, D.ce, x,
-                       y, mode, a, part);
+    ESP_LINES(k_project_finish, K, part ? (unsigned)dot_blocks(D.nlam, K) : line_grid(D.nlam, K), D.nlam, K, D.le_cnt,
+              D.le_coarse, D.le_sign, D.RtT, D.ce, x, y, mode, a, part);
 }
 
 void launch_subdomain_kernel_dots(const DualDev &D, int K, const double *x, double *out, hipStream_t st) {
@@ -608,8 +815,7 @@ void launch_subdomain_kernel_dots(const DualDev &D, int K, const double *x, doub
 }
 
 void launch_dot_lines(int64_t n, int K, const double *a, const double *b, double *part, hipStream_t st) {
-    const int T = line_threads(K);
-    hipLaunchKernelGGL(k_dot_lines, dim3(dot_blocks(n, K)), dim3(T), T * sizeof(double), st, n, K, a, b, part);
+    ESP_LINES(k_dot_lines, K, dot_blocks(n, K), n, K, a, b, part);
 }
 
 void launch_pcg_init(int K, const double *part_r, const double *part_b, int np, double precision, double tol_abs,
@@ -622,16 +828,12 @@ static unsigned update_grid(int64_t n, int K) { return std::min(line_grid(n, K),
 
 void launch_p_update(int64_t n, int K, double *p, const double *y, const double *part_yw, const double *part_ww,
                      int np, bool first, double *scal, PcgRecord *rec, hipStream_t st) {
-    const int T = line_threads(K);
-    hipLaunchKernelGGL(k_p_update, dim3(update_grid(n, K)), dim3(T), T * sizeof(double), st, n, K, p, y, part_yw,
-                       part_ww, np, first ? 1 : 0, scal, rec);
+    ESP_LINES(k_p_update, K, update_grid(n, K), n, K, p, y, part_yw, part_ww, np, first ? 1 : 0, scal, rec);
 }
 
 void launch_xr_update(int64_t n, int K, double *x, double *r, const double *p, const double *Ap,
                       const double *part_pAp, int np, double *scal, hipStream_t st) {
-    const int T = line_threads(K);
-    hipLaunchKernelGGL(k_xr_update, dim3(update_grid(n, K)), dim3(T), T * sizeof(double), st, n, K, x, r, p, Ap,
-                       part_pAp, np, scal);
+    ESP_LINES(k_xr_update, K, update_grid(n, K), n, K, x, r, p, Ap, part_pAp, np, scal);
 }
 
 }  // namespace esp
