@@ -466,7 +466,7 @@ class FETISolver:
         (u of the same shape, iterations per case, final ||P r|| per case)."""
         f = np.ascontiguousarray(f, dtype=np.float64)
         nrhs = f.shape[0]
-        u = np.zeros_like(f)
+        u = np.empty_like(f)
         it = np.zeros(nrhs, np.int32)
         nr = np.zeros(nrhs)
         st = Stats()
@@ -609,7 +609,7 @@ class GridFETI(FETISolver):
         Returns (u (nrhs, n_nodes, ndof), iterations, final norms)."""
         loads = np.ascontiguousarray(loads, dtype=np.float64).reshape(len(loads), self.n_nodes, self.ndof)
         nrhs = loads.shape[0]
-        un = np.zeros_like(loads)
+        un = np.empty_like(loads)
         it = np.zeros(nrhs, np.int32)
         nr = np.zeros(nrhs)
         st = Stats()
