@@ -20,7 +20,8 @@ struct SymvItem {
 // partials (plen x Kmax)
 constexpr int BLOCK_STRIPS = 8;
 struct SymvBlock {
-    SymvItem *items = nullptr;
+    SymvItem *items = nullptr;         // by subdomain
+    SymvItem *launch_items = nullptr;  // longest first
     int n_items = 0;
     int *item0 = nullptr, *nitems = nullptr;
     int64_t plen = 0;

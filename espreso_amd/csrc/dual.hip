@@ -155,15 +155,30 @@ __global__ void __launch_bounds__(256) k_symv(const SymvItem *__restrict__ items
 // adds the four waves' in order and writes the item's partial (fixed order, so
 // repeated applies are bitwise equal).  x and the partials are interleaved by
 // right-hand side with stride nr.
-// What bounds it is the latency of a step (load, transpose, eight chained MFMAs), so
-// the next step's blocks are loaded before the current ones are used, by loads
-// without a branch (blocks left of a strip's diagonal, past the item's strips or
-// past the last column repeat stored values and are zeroed when used: at a branch
-// the compiler waits for every load in flight), and four workgroups share a CU.
-// Waves owning columns instead of strips, one block's loads in flight, took 745 us
-// for 1.2 GB of F_i at 2000 heat subdomains and 16 cases (now 632), 421 at 512
-// uneven elasticity subdomains and 5 cases (now 333).
+// What bounds it is the latency of a step and the start and end of an item (11 us of
+// an item's 37 at 18 steps), not bandwidth (F_i of 2000 uneven heat subdomains is 2.0 GB:
+// 303 us) nor the MFMAs (216 us).  So the next step's blocks are loaded before the
+// current ones are used, by loads without a branch (blocks left of a strip's diagonal,
+// past the item's strips or past the last column repeat stored values and are zeroed
+// when used: at a branch the compiler waits for every load in flight) and without
+// 64-bit address arithmetic per lane, four workgroups share a CU, waves whose strips
+// start right of a block only keep step, and items are launched longest first.  x is
+// read up to 15 lines past the last column: its buffers are that much longer.
+// Waves owning columns instead of strips, one block's loads in flight, took 745 us at
+// those subdomains and 16 cases (now 596), 421 at 512 uneven elasticity subdomains and 5
+// cases (now 290).  Two steps ahead, 64 columns a load, two waves with four strips or
+// eight with one and x in LDS all take 594 to 635 and 290 to 327 us.
 typedef double v4d __attribute__((ext_vector_type(4)));
+
+// loads with a scalar base and one 32-bit lane offset (no 64-bit address arithmetic per lane)
+__device__ __forceinline__ u32x4 stream_load(const u32x4 *p, unsigned at) {
+    asm volatile("" : "+s"(p));
+    return __builtin_nontemporal_load((const __attribute__((address_space(1))) u32x4 *)p + at);
+}
+__device__ __forceinline__ double line_value(const double *p, unsigned at) {
+    asm volatile("" : "+s"(p));
+    return ((const __attribute__((address_space(1))) double *)p)[at];
+}
 
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -217,18 +232,25 @@ __global__ void __launch_bounds__(256, 4) k_symv_mfma(const SymvItem *__restrict
         u32x4 p[W][2];
         double x[4];
     } st[2];
+    int qw[W];  // q times the width of the last chunk of columns
+    unsigned xo[4];
+#pragma unroll
+    for (int k = 0; k < W; k++) qw[k] = q * (((m - r0[k] - 1) & 63) + 1);
+#pragma unroll
+    for (int j = 0; j < 4; j++) xo[j] = (q + 4 * j) * nr + lv;
     auto load = [&](Step &n, int cb) {
         const int c0 = r0i + 16 * min(cb, nblk - 1);
 #pragma unroll
         for (int k = 0; k < W; k++) {
             const int cl = max(0, c0 - r0[k]), ch = cl & ~63, w = min(64, m - r0[k] - ch);
-            const int at = min(cl - ch + l16, w - 1);
+            const unsigned at = (w == 64 ? 64 * q : qw[k]) + min(cl - ch + l16, w - 1);
             const u32x4 *chunk = strip[k] + (int64_t)ch * (R / 2);
-            n.p[k][0] = __builtin_nontemporal_load(chunk + q * w + at);
-            n.p[k][1] = __builtin_nontemporal_load(chunk + (q + 4) * w + at);
+            n.p[k][0] = stream_load(chunk, at);
+            n.p[k][1] = stream_load(chunk + 4 * w, at);
         }
+        const double *x = xs + (int64_t)c0 * nr;  // past the last column: not used
 #pragma unroll
-        for (int j = 0; j < 4; j++) n.x[j] = xs[(int64_t)min(c0 + q + 4 * j, m - 1) * nr + lv];
+        for (int j = 0; j < 4; j++) n.x[j] = line_value(x, xo[j]);
     };
     auto step = [&](Step &c, int cb, int buf) {
         const int c0 = r0i + 16 * cb;
@@ -243,34 +265,33 @@ __global__ void __launch_bounds__(256, 4) k_symv_mfma(const SymvItem *__restrict
 #pragma unroll
             for (int j = 0; j < 4; j++) c.x[j] = c0 + q + 4 * j < m ? c.x[j] : 0.0;
         }
-        v4d dc[W];  // a chain per strip
+        // waves whose strips start right of the block only keep step
+        double dc[4] = {0.0, 0.0, 0.0, 0.0};
+        if (W * wave <= min(cb, ns - 1)) {
+            v4d d = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int k = 0; k < W; k++) {
-            dc[k] = (v4d){0.0, 0.0, 0.0, 0.0};
-            *(u32x4 *)(T[wave][k] + l16 * TL + 2 * q) = c.p[k][0];
-            *(u32x4 *)(T[wave][k] + l16 * TL + 2 * q + 8) = c.p[k][1];
+            for (int k = 0; k < W; k++) {
+                *(u32x4 *)(T[wave][k] + l16 * TL + 2 * q) = c.p[k][0];
+                *(u32x4 *)(T[wave][k] + l16 * TL + 2 * q + 8) = c.p[k][1];
+            }
+            double a[W][4];
+            __builtin_memcpy(a, c.p, sizeof(a));
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int k = 0; k < W; k++) d = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k][j], xr[k][j], d, 0, 0, 0);
+            wave_lds_sync();
+            // row product: column slot q of call j is column q + 4j
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int k = 0; k < W; k++)
+                    dr[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(T[wave][k][(q + 4 * j) * TL + l16], c.x[j], dr[k], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) dc[i] = d[i];
         }
-        double a[W][4];
-        __builtin_memcpy(a, c.p, sizeof(a));
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-            for (int k = 0; k < W; k++)
-                dc[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k][j], xr[k][j], dc[k], 0, 0, 0);
-        wave_lds_sync();
-        // row product: column slot q of call j is column q + 4j
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-            for (int k = 0; k < W; k++)
-                dr[k] = __builtin_amdgcn_mfma_f64_16x16x4f64(T[wave][k][(q + 4 * j) * TL + l16], c.x[j], dr[k], 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            double v = dc[0][i];
-#pragma unroll
-            for (int k = 1; k < W; k++) v += dc[k][i];
-            slot[buf][wave][(q + 4 * i) * 16 + l16] = v;
-        }
+        for (int i = 0; i < 4; i++) slot[buf][wave][(q + 4 * i) * 16 + l16] = dc[i];
         lds_barrier();  // a slot is written again two steps on, behind the next barrier
         const int col = c0 + (tid >> 4), v = tid & 15;
         if (col < m && v < nr)
@@ -711,7 +732,7 @@ void launch_symv_mfma(const DualDev &D, const SymvBlock &B, bool sd, int nr, con
     const double *pool = sd ? D.SD : D.Fd;
     const int64_t *off = sd ? D.sdoff : D.foff;
     if (ev0) (void)hipEventRecord(ev0, st);
-    hipLaunchKernelGGL(k_symv_mfma, dim3(B.n_items), dim3(256), 0, st, B.items, D.m, D.boff, pool, off, xb, nr,
+    hipLaunchKernelGGL(k_symv_mfma, dim3(B.n_items), dim3(256), 0, st, B.launch_items, D.m, D.boff, pool, off, xb, nr,
                        B.ypart);
     if (ev1) (void)hipEventRecord(ev1, st);
     launch_part_reduce(D, B.items, B.item0, B.nitems, STRIP_F64, nr, B.ypart, yb, st);

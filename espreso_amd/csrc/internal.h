@@ -37,7 +37,7 @@ constexpr int STRIP_B16 = 64;   // BF16 storage
 // SYMV work-item sizes (matrix elements per workgroup): default and autotuner candidates.  An
 // operator too small to give every CU four workgroups of that size is cut finer, down to
 // SYMV_MIN_ITEM elements, where the gather of x per workgroup outweighs the split: 64
-// elasticity subdomains of 456 boundary DOFs (53 MB) take 31.9 us in 128 workgroups, 18.1 at
+// elasticity subdomains of 456 boundary DOFs (41 MB) take 31.9 us in 128 workgroups, 18.1 at
 // 48 K elements, 14.3 at 32 K, 15.3 at 20 K, 14.2 at 12 K and 15.8 at 8 K.
 constexpr int64_t SYMV_DEFAULT_TARGET = 320 * 1024;
 constexpr int64_t SYMV_TUNE_TARGETS[5] = {96 * 1024, 192 * 1024, 320 * 1024, 640 * 1024, 1280 * 1024};
