@@ -140,6 +140,7 @@ struct ClusterDev {
     float *FB0f = nullptr;     // FB0 in FP32 (FP32/BF16 storage of F_i only)
     double *Fcc = nullptr;     // nq x nq per subdomain: B0_i F_i B0_i^T
     double *lambda0 = nullptr, *alphaK = nullptr;
+    double *g0 = nullptr;      // B0 y_b of one case
     double *rho_s = nullptr;   // per subdomain: max diag S_i (the scale of the kernel regularisation)
 };
 

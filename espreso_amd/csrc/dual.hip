@@ -155,9 +155,10 @@ __global__ void __launch_bounds__(256) k_symv(const SymvItem *__restrict__ items
 // adds the four waves' in order and writes the item's partial (fixed order, so
 // repeated applies are bitwise equal).  x and the partials are interleaved by
 // right-hand side with stride nr.
-// What bounds it is the latency of a step and the start and end of an item (11 us of
-// an item's 37 at 18 steps), not bandwidth (F_i of 2000 uneven heat subdomains is 2.0 GB:
-// 303 us) nor the MFMAs (216 us).  So the next step's blocks are loaded before the
+// What bounds it: a step of 16 columns moves 16 KB of F_i, 2 KB of x and, at 16 cases,
+// 2 KB of partials, and takes 0.93 us a CU, 5 TB/s like a copy; 71 of the 596 us below
+// are the starts and ends of items.  (F_i of 2000 uneven heat subdomains is 2.0 GB: 303 us
+// read alone; the MFMAs take 216.)  So the next step's blocks are loaded before the
 // current ones are used, by loads without a branch (blocks left of a strip's diagonal,
 // past the item's strips or past the last column repeat stored values and are zeroed
 // when used: at a branch the compiler waits for every load in flight) and without
@@ -345,42 +346,75 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// t = F0^-1 g0: 32 rows per workgroup (8 per wave, accumulated together for
-// memory-level parallelism), each row a dot over a column of the symmetric
-// F0^-1; g0 is gathered from the SYMV output.
-__global__ void __launch_bounds__(256) k_cluster_t(const ClusterDev C, const double *yb, double *t) {
-    extern __shared__ double g0[];
-    const int c = blockIdx.y;
-    const int n0 = C.n0[c];
-    const int rb = blockIdx.x * 32;
-    if (rb >= n0) return;  // uniform over the workgroup
+// One case, first kernel: g0 gathered from the SYMV output and alpha = Sa^-1 (H^T g0 - e0)
+// (H^T = G0 F0^-1), one workgroup per cluster, so that t is not needed before alpha
+// and the kernel that computes t finishes lambda0.  Both are chains of latency beside
+// the few MB of F0^-1: 38 us (t, each workgroup with the gather) + 28 us (alpha from t, one
+// column a thread, then lambda0) at 64 clusters of 8 subdomains of 10^3 elasticity, now 18 + 21.
+__global__ void __launch_bounds__(1024) k_cluster_alpha_one(const ClusterDev C, const double *yb, const double *e0s) {
+    extern __shared__ double t2[];
+    const int c = blockIdx.x;
+    const int n0 = C.n0[c], kt = C.kt[c];
     const int64_t ro = C.rowoff[c];
-    for (int r = threadIdx.x; r < n0; r += 256) {
+    double *g0 = C.g0 + ro;
+    for (int r = threadIdx.x; r < n0; r += 1024) {
         double v = 0.0;
         for (int64_t e = C.re_ptr[ro + r]; e < C.re_ptr[ro + r + 1]; e++) v += C.re_c[e] * yb[C.re_b[e]];
         g0[r] = v;
     }
     __syncthreads();
-    const double *F = C.F0inv + C.f0off[c];
+    const double *H = C.H + C.g0off[c];  // n0 x kt
+    const double *e0 = e0s + C.eoff[c];  // cluster-contiguous subdomain partials
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int a = w; a < kt; a += 16) {
+        double v = 0.0;
+#pragma unroll 4
+        for (int r = lane; r < n0; r += 64) v += H[r + (int64_t)a * n0] * g0[r];
+        v = wave_sum(v);
+        if (lane == 0) t2[a] = v - e0[a];
+    }
+    __syncthreads();
+    const double *Sai = C.Sainv + C.saoff[c];  // symmetric: column a is row a
+    for (int a = w; a < kt; a += 16) {
+        double v = 0.0;
+        for (int b = lane; b < kt; b += 64) v += Sai[b + (int64_t)a * kt] * t2[b];
+        v = wave_sum(v);
+        if (lane == 0) C.alphaK[C.eoff[c] + a] = v;
+    }
+}
+
+// lambda0 = F0^-1 g0 - H alpha: 32 rows per workgroup (8 per wave, accumulated together
+// for memory-level parallelism), each row a dot over a column of the symmetric F0^-1
+__global__ void __launch_bounds__(256) k_cluster_lambda0(const ClusterDev C) {
+    extern __shared__ double g0[];
+    const int c = blockIdx.y;
+    const int n0 = C.n0[c], kt = C.kt[c];
+    const int rb = blockIdx.x * 32;
+    if (rb >= n0) return;  // uniform over the workgroup
+    const int64_t ro = C.rowoff[c];
+    for (int r = threadIdx.x; r < n0; r += 256) g0[r] = C.g0[ro + r];
+    __syncthreads();
+    const double *F = C.F0inv + C.f0off[c], *H = C.H + C.g0off[c], *al = C.alphaK + C.eoff[c];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int r0 = rb + w * 8;
     double v[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) v[i] = 0.0;
+    for (int a = lane; a < kt; a += 64) {
+        const double x = al[a];
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] -= H[min(r0 + i, n0 - 1) + (int64_t)a * n0] * x;
+    }
     for (int q = lane; q < n0; q += 64) {
         const double gq = g0[q];
 #pragma unroll
-        for (int i = 0; i < 8; i++)
-            if (r0 + i < n0) v[i] += F[q + (int64_t)(r0 + i) * n0] * gq;
+        for (int i = 0; i < 8; i++) v[i] += F[q + (int64_t)min(r0 + i, n0 - 1) * n0] * gq;
     }
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const double sv = wave_sum(v[i]);
-        if (lane == 0 && r0 + i < n0) t[ro + r0 + i] = sv;
-    }
+    const double s = wave_rows_reduce<8, double>(v, lane);
+    if ((lane & 7) == 0 && r0 + (lane >> 3) < n0) C.lambda0[ro + r0 + (lane >> 3)] = s;
 }
 
-// one workgroup per cluster and case: alpha = Sa^-1 (G0 t - e0), lambda0 = t - H alpha (in place over t);
+// Several cases: one workgroup per cluster and case: alpha = Sa^-1 (G0 t - e0), lambda0 = t - H alpha (in place over t);
 // e0s interleaved by case, lam0 and alphaK at strides lstr and astr
 __global__ void __launch_bounds__(1024) k_cluster_alpha(const ClusterDev C, const double *e0s, double *lam0,
                                                         int64_t lstr, double *alphaK, int64_t astr) {
@@ -740,11 +774,9 @@ void launch_symv_mfma(const DualDev &D, const SymvBlock &B, bool sd, int nr, con
 
 void launch_cluster_correction(const DualDev &D, const ClusterDev &C, const double *e0s, double *yb, int addR,
                                hipStream_t st, bool lowp) {
+    hipLaunchKernelGGL(k_cluster_alpha_one, dim3(C.ncl), dim3(1024), (size_t)std::max(C.max_kt, 1) * 8, st, C, yb, e0s);
     if (C.max_n0 > 0)
-        hipLaunchKernelGGL(k_cluster_t, dim3((C.max_n0 + 31) / 32, C.ncl), dim3(256), (size_t)C.max_n0 * 8, st, C, yb,
-                           C.lambda0);
-    hipLaunchKernelGGL(k_cluster_alpha, dim3(C.ncl), dim3(1024), 2 * (size_t)std::max(C.max_kt, 1) * 8, st, C, e0s,
-                       C.lambda0, (int64_t)0, C.alphaK, (int64_t)0);
+        hipLaunchKernelGGL(k_cluster_lambda0, dim3((C.max_n0 + 31) / 32, C.ncl), dim3(256), (size_t)C.max_n0 * 8, st, C);
     if (lowp && C.FB0f)
         hipLaunchKernelGGL(k_cluster_apply<float>, dim3((D.max_m + 255) / 256, D.nsub), dim3(256), 0, st, C,
                            (const float *)C.FB0f, D.m, D.boff, D.kdim, D.rboff, D.Rb, C.lambda0, C.alphaK, addR, yb);

@@ -3090,6 +3090,7 @@ void espreso_feti_s::load_clusters() {
     CL.Fcc = alloc<double>(std::max<int64_t>(1, fccoff_h[nsub]));
     n_lambda0 = std::max<int64_t>(1, rowoff[ncl]);
     CL.lambda0 = alloc<double>(n_lambda0);
+    CL.g0 = alloc<double>(n_lambda0);
     CL.alphaK = alloc<double>(asubv[nsub]);
     CL.rho_s = alloc<double>(nsub);
     d_Fcc = CL.Fcc;
