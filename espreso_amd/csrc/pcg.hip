@@ -467,31 +467,37 @@ __global__ void __launch_bounds__(256) k_coarse_gemv(int nc, const double *__res
 }
 
 // e = GGinv d for K <= 16 cases on MFMA (the N dimension of v_mfma_f64_16x16x4f64):
-// GGinv is read once for all cases.  One workgroup per 16 rows, its 16 waves
-// take every 16th chunk of 16 columns and meet in LDS in a fixed order (four waves
-// leave too little in flight with one workgroup a CU: 47 us at 3072 columns, now 32).  A lane
-// loads four consecutive columns of its row (32 B of the 128 B line that four
-// lanes share) and the matching rows of d; products of columns past nc are zero.
+// GGinv is read once for all cases.  One workgroup per 16 rows, its 16 waves take every
+// 16th chunk of 16 columns, four chunks' loads at a time, and meet in LDS in a fixed
+// order; products of columns past nc are zero.  GGinv is symmetric, so 16 lanes read 128
+// consecutive bytes of a column; lanes along a row touch 16 lines a load, and one workgroup
+// a CU then gets 12 GB/s: 47 us with four waves and 32 with 16 at 3072 columns (75 MB) and 5
+// cases, now 20; 33, 23 and 15 at 2000 and 16.
 __global__ void __launch_bounds__(1024) k_coarse_block(int nc, int K, const double *__restrict__ Ginv,
                                                       const double *__restrict__ d, double *__restrict__ e) {
     __shared__ double sum[16][256];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, l16 = lane & 15, kq = lane >> 4;
     const int i0 = blockIdx.x * 16;
-    const double *row = Ginv + (int64_t)min(i0 + l16, nc - 1) * nc;
+    const double *col = Ginv + min(i0 + l16, nc - 1);
     const int v = min(l16, K - 1);
     v4d acc = {0.0, 0.0, 0.0, 0.0};
-        for (int k0 = 16 * w; k0 < nc; k0 += 256) {
-        double a[4], b[4];
+    constexpr int U = 4;  // chunks loaded before the first is used
+    for (int k0 = 16 * w; k0 < nc; k0 += 256 * U) {
+        double a[U][4], b[U][4];
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const int k = k0 + 4 * kq + s;
-            const bool ok = k < nc;
-            const double av = row[ok ? k : 0], bv = d[(int64_t)(ok ? k : 0) * K + v];
-            a[s] = ok ? av : 0.0;
-            b[s] = ok ? bv : 0.0;
-        }
+        for (int u = 0; u < U; u++)
 #pragma unroll
-        for (int s = 0; s < 4; s++) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[s], acc, 0, 0, 0);
+            for (int s = 0; s < 4; s++) {
+                const int k = k0 + 256 * u + 4 * s + kq;
+                const bool ok = k < nc;
+                const double av = col[(int64_t)(ok ? k : 0) * nc], bv = d[(int64_t)(ok ? k : 0) * K + v];
+                a[u][s] = ok ? av : 0.0;
+                b[u][s] = ok ? bv : 0.0;
+            }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int s = 0; s < 4; s++) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u][s], b[u][s], acc, 0, 0, 0);
     }
 #pragma unroll
     for (int q = 0; q < 4; q++) sum[w][(kq + 4 * q) * 16 + l16] = acc[q];
