@@ -1278,11 +1278,13 @@ __global__ void __launch_bounds__(256) k_band_extract(const DenseDesc *D, double
         double *dst = band + band_off[blockIdx.y] + (int64_t)c * w;
         const double *src = d.Kii + c + (size_t)c * d.ldk;
         const int diag = c & (TILE - 1);
+        // the factor is zero, and its storage not written, past the column's band tiles
+        const int end = min(d.ni, (c / TILE + d.band_ii + 1) * TILE);
         const double *inv = d.Dinv + (size_t)(c / TILE) * TILE * TILE + diag * (TILE + 1);
 #pragma unroll 4
         for (int r = lane; r < w; r += 64) {
-            const double v = (diag + r < TILE ? inv : src)[min(r, d.ni - 1 - c)];
-            dst[r] = c + r < d.ni ? v : 0.0;
+            const double v = (diag + r < TILE ? inv : src)[min(r, end - 1 - c)];
+            dst[r] = c + r < end ? v : 0.0;
         }
         if (lane == 0) yf[yf_off[blockIdx.y] + c] = d.Kib[c + (size_t)d.m * d.ldb];
     }
