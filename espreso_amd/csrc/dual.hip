@@ -1,9 +1,8 @@
 // Dual-space kernels of the FETI iteration: the dual operator
-// F x = sum_i B_i F_i B_i^T x (itersolvercpu.cpp:9-114), the preconditioners
-// (itersolvercpu.cpp:520-602), the projector P = I - G^T (G G^T)^-1 G
-// (itersolver.cpp:5541-5623), PCG vector updates and dot products
-// (itersolver.cpp:1537-1684, 6427-6467), and the primal recovery
-// (itersolver.cpp:372-431).
+// F x = sum_i B_i F_i B_i^T x (itersolvercpu.cpp:9-114) for one and for several
+// cases, the cluster correction of hybrid FETI, new loads and the primal recovery
+// (itersolver.cpp:372-431) with their interior band solves, and the KKT report.
+// The passes of the PCG between two operator applies are in pcg.hip.
 //
 // F_i and S_D live in HBM in the packed-strip layout (see internal.h): one
 // pass over the upper triangle applies both triangles.  A workgroup owns a
