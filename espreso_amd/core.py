@@ -521,7 +521,7 @@ class FETISolver:
 
     def symv_items(self):
         """SYMV work-item sizes chosen by the autotuner: (FP64, FP32, BF16),
-        0 for a precision nothing is stored in."""
+        0 for a precision nothing is stored in, sizes under 98304 as 98304."""
         t = (C.c_int64 * 3)()
         _check(lib().espreso_feti_symv_items(self.h, t))
         return tuple(int(v) for v in t)

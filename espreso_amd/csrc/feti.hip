@@ -928,10 +928,11 @@ struct espreso_feti_s {
     // precision (FP64, FP32, BF16); 0 for a precision nothing is stored in;
     // chosen by tune_symv
     int64_t symv_target[3] = {0, 0, 0};
-    bool symv_fill = true;  // items also small enough for SYMV_MIN_ITEMS of them (unless the size is fixed)
+    bool symv_fixed = false;  // by ESPRESO_SYMV_ITEM
     bool symv_tuned = false;
     int max_m_h = 0;
     bool prec_used(int p) const { return p == 0 || p == opt.sc_precision || p == opt.sd_precision; }
+    int64_t symv_elements(int prec) const;
     void upload_items(int prec, int64_t target);
     void tune_symv();
     // dual operators on device vectors
@@ -1577,8 +1578,7 @@ void espreso_feti_s::load() {
         int64_t target = SYMV_DEFAULT_TARGET;
         if (const char *e = std::getenv("ESPRESO_SYMV_ITEM")) {
             target = std::max<int64_t>(4096, std::atoll(e));
-            symv_tuned = true;
-            symv_fill = false;
+            symv_tuned = symv_fixed = true;
         }
         // partial vectors sized for the smallest item size any candidate uses
         std::vector<SymvItem> it;
@@ -1586,7 +1586,8 @@ void espreso_feti_s::load() {
         int64_t plen_max = 1, pl = 0;
         for (int p = 0; p < 3; p++) {
             if (!prec_used(p)) continue;
-            build_items(p, std::min(target, SYMV_TUNE_TARGETS[0]), it, i0, ni, pl);
+            const int64_t smallest = symv_elements(p) < SYMV_FINE_BELOW ? SYMV_TUNE_TARGETS[0] : SYMV_COARSE;
+            build_items(p, std::min(target, smallest), it, i0, ni, pl);
             plen_max = std::max(plen_max, pl);
         }
         D.ypart = alloc<double>(plen_max);
@@ -2172,11 +2173,6 @@ void espreso_feti_s::build_items(int prec, int64_t target, std::vector<SymvItem>
     item0.assign(nsub, 0);
     nit.assign(nsub, 0);
     plen = 0;
-    if (symv_fill) {
-        int64_t all = 0;
-        for (const SubHost &h : sub) all += strip_size(h.m, R);
-        target = std::min(target, std::max(SYMV_MIN_ITEM, all / SYMV_MIN_ITEMS));
-    }
     for (int s = 0; s < nsub; s++) {
         const int m = sub[s].m;
         const int nst = (int)strip_count(m, R);
@@ -2202,6 +2198,13 @@ void espreso_feti_s::build_items(int prec, int64_t target, std::vector<SymvItem>
     }
 }
 
+// packed elements of all subdomains
+int64_t espreso_feti_s::symv_elements(int prec) const {
+    int64_t all = 0;
+    for (const SubHost &h : sub) all += strip_size(h.m, strip_rows(prec));
+    return all;
+}
+
 // (re)build and upload the SYMV work list of a storage precision
 void espreso_feti_s::upload_items(int prec, int64_t target) {
     std::vector<SymvItem> it;
@@ -2224,10 +2227,13 @@ void espreso_feti_s::upload_items(int prec, int64_t target) {
     symv_target[prec] = target;
 }
 
-// Autotuner of the SYMV work-item size, keyed on the subdomain size: at the
-// first set-up every candidate is timed on the assembled F_i (HIP events, 2
-// applies each after one warm-up apply) and the fastest kept; the choice is cached for the process by
-// (storage precision, largest interface size rounded to 64).  ESPRESO_SYMV_ITEM
+// Autotuner of the SYMV work-item size: at the first set-up every candidate is
+// timed on the assembled F_i (HIP events, 2 applies each after one warm-up
+// apply, 4 of the short ones of a small operator) and the fastest kept; the
+// choice is cached for the process by (storage precision, largest interface
+// size rounded to 64, packed elements to the power of two below): how many
+// subdomains share the CUs decides as much as their size.  Candidates that
+// give the list of the one before are not timed again.  ESPRESO_SYMV_ITEM
 // fixes the size, ESPRESO_AUTOTUNE=0 keeps the default.
 void espreso_feti_s::tune_symv() {
     if (symv_tuned) return;
@@ -2235,10 +2241,12 @@ void espreso_feti_s::tune_symv() {
     if (const char *e = std::getenv("ESPRESO_AUTOTUNE"))
         if (std::atoi(e) == 0) return;
     static std::mutex mu;
-    static std::map<std::pair<int, int>, int64_t> cache;
+    static std::map<std::array<int, 3>, int64_t> cache;
     for (int prec = 0; prec < 3; prec++) {
         if (!prec_used(prec)) continue;
-        const std::pair<int, int> key{prec, (max_m_h + 63) / 64};
+        const int64_t all = symv_elements(prec);
+        const bool fine = all < SYMV_FINE_BELOW;
+        const std::array<int, 3> key{prec, (max_m_h + 63) / 64, std::ilogb((double)all)};
         {
             std::lock_guard<std::mutex> lk(mu);
             auto f = cache.find(key);
@@ -2254,11 +2262,15 @@ void espreso_feti_s::tune_symv() {
         ESP_HIP(hipEventCreate(&e1));
         int64_t best = symv_target[prec];
         float best_ms = 1e30f;
+        int items = 0;
         launch_symv(D, sd, prec, d_b, 1, false, st);  // warm
         for (const int64_t target : SYMV_TUNE_TARGETS) {
+            if (target < SYMV_COARSE && !fine) continue;
             upload_items(prec, target);
+            if (D.n_items[prec] == items) continue;  // not fewer items: the list of the one before
+            items = D.n_items[prec];
             ESP_HIP(hipEventRecord(e0, st));
-            for (int r = 0; r < 2; r++) launch_symv(D, sd, prec, d_b, 1, false, st);
+            for (int r = 0; r < (fine ? 4 : 2); r++) launch_symv(D, sd, prec, d_b, 1, false, st);
             ESP_HIP(hipEventRecord(e1, st));
             ESP_HIP(hipEventSynchronize(e1));
             float ms = 0;
@@ -2270,7 +2282,10 @@ void espreso_feti_s::tune_symv() {
         }
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
-        upload_items(prec, best);
+        if (best != symv_target[prec]) upload_items(prec, best);
+        if (measure)
+            std::fprintf(stderr, "espreso: SYMV items tuned: precision %d, %lld of %lld elements\n", prec,
+                         (long long)best, (long long)all);
         std::lock_guard<std::mutex> lk(mu);
         cache[key] = best;
     }
@@ -3476,7 +3491,10 @@ int espreso_feti_resolve(espreso_feti *h, espreso_feti_stats *st) {
 int espreso_feti_symv_items(espreso_feti *h, int64_t *targets) {
     ESP_API_BEGIN
     ESP_CHECK(h && targets, ESPRESO_ERR_ARG, "null argument");
-    for (int p = 0; p < 3; p++) targets[p] = h->symv_target[p];
+    for (int p = 0; p < 3; p++) {
+        targets[p] = h->symv_target[p];
+        if (targets[p] > 0 && !h->symv_fixed) targets[p] = std::max(targets[p], SYMV_COARSE);
+    }
     ESP_API_END
 }
 

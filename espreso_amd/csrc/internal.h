@@ -34,14 +34,16 @@ constexpr int TILE = 64;        // dense tile edge of the assembly kernels
 constexpr int STRIP_F64 = 16;   // rows per packed strip, FP64 storage
 constexpr int STRIP_F32 = 32;   // FP32 storage
 constexpr int STRIP_B16 = 64;   // BF16 storage
-// SYMV work-item sizes (matrix elements per workgroup): default and autotuner candidates.  An
-// operator too small to give every CU four workgroups of that size is cut finer, down to
-// SYMV_MIN_ITEM elements, where the gather of x per workgroup outweighs the split: 64
-// elasticity subdomains of 456 boundary DOFs (41 MB) take 31.9 us in 128 workgroups, 18.1 at
-// 48 K elements, 14.3 at 32 K, 15.3 at 20 K, 14.2 at 12 K and 15.8 at 8 K.
+// SYMV work-item sizes (matrix elements per workgroup): the default and the autotuner's candidates.
+// The sizes under SYMV_COARSE are tried only on operators of less than SYMV_FINE_BELOW elements: there
+// larger items leave CUs idle, above it the gather of x by every item and the partials of more items cost
+// more than they give.  SYMV at 48 K / at the best of 96 K and more (elasticity cubes of e^3 elements):
+// 64 of 5^3 (4.9 M elements) 22 / 33 us (16 K: 18), 216 of 5^3 (18 M) 32 / 41, 64 of 8^3 (29 M) 50 / 57,
+// 512 of 5^3 (46 M) 73 / 70, 64 of 10^3 (70 M) 124 / 103.
 constexpr int64_t SYMV_DEFAULT_TARGET = 320 * 1024;
-constexpr int64_t SYMV_TUNE_TARGETS[5] = {96 * 1024, 192 * 1024, 320 * 1024, 640 * 1024, 1280 * 1024};
-constexpr int64_t SYMV_MIN_ITEM = 16 * 1024, SYMV_MIN_ITEMS = 1024;
+constexpr int64_t SYMV_TUNE_TARGETS[8] = {16 * 1024,  32 * 1024,  48 * 1024,  96 * 1024,
+                                          192 * 1024, 320 * 1024, 640 * 1024, 1280 * 1024};
+constexpr int64_t SYMV_COARSE = 96 * 1024, SYMV_FINE_BELOW = (int64_t)64 << 20;
 
 __host__ __device__ inline int strip_rows(int prec) { return prec == 0 ? STRIP_F64 : (prec == 1 ? STRIP_F32 : STRIP_B16); }
 // LDS of a SYMV workgroup (interface up to max_m DOFs): the 64-bit fixed-point

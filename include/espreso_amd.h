@@ -309,9 +309,11 @@ int espreso_feti_vec_b(espreso_feti *h, double *b);
 /* SYMV work-item sizes in matrix elements per workgroup, targets[3]: FP64,
  * FP32 and BF16 storage (0 where neither F_i nor S_D is stored in that
  * precision).  The first espreso_feti_setup picks them by timing candidates
- * on the assembled operators (cached per process by storage precision and
- * subdomain interface size); ESPRESO_SYMV_ITEM fixes them and
- * ESPRESO_AUTOTUNE=0 keeps the default (327680).                            */
+ * on the assembled operators (cached per process by storage precision,
+ * subdomain interface size and the operator's size); ESPRESO_SYMV_ITEM fixes
+ * them and ESPRESO_AUTOTUNE=0 keeps the default (327680).  An operator of less
+ * than 2^26 elements may take 49152, 32768 or 16384; these are reported as
+ * 98304 (no item is larger).                                                 */
 int espreso_feti_symv_items(espreso_feti *h, int64_t *targets);
 /* K_i CSR values of subdomain i as the device holds them (after setup; the
  * CSR of espreso_feti_set_subdomain, or of the grid builder with
