@@ -3560,6 +3560,7 @@ int espreso_feti_dual(espreso_feti *h, double *lambda) {
 static int dual_op(espreso_feti *h, const double *x, double *y, int which) {
     ESP_API_BEGIN
     ESP_CHECK(h && h->ready, ESPRESO_ERR_STATE, "setup not done");
+    ESP_CHECK(x && y, ESPRESO_ERR_ARG, "null argument");
     const size_t bytes = h->nlam * sizeof(double);
     copy_from_host(h->opt.device, h->d_z, x, bytes, h->st);
     if (which == 0) h->apply_F(h->d_z, h->d_tmp, h->opt.sc_precision);
@@ -4080,6 +4081,7 @@ int espreso_grid_l2g(espreso_feti *h, int32_t i, int32_t *l2g) {
 int espreso_grid_nodal_solution(espreso_feti *h, double *u_nodal) {
     ESP_API_BEGIN
     ESP_CHECK(h && h->solved && !h->l2g.empty(), ESPRESO_ERR_STATE, "no grid solution");
+    ESP_CHECK(u_nodal, ESPRESO_ERR_ARG, "null argument");
     ESP_HIP(hipSetDevice(h->opt.device));
     h->grid_device();
     const int64_t nv = (int64_t)h->nnodes * h->ndof;
