@@ -461,7 +461,10 @@ void copy_to_host(int device, void *dst, const void *src, size_t bytes, hipStrea
 
 // PCG records (pinned, one per instance with loaded inputs), kept for the
 // process and lent to the instances: pinning and unpinning a page costs more
-// than a small solve.  As many as instances were alive at once.
+// than a small solve.  As many as instances were alive at once.  The host polls a
+// record while the kernel that writes it still runs: only coherent memory promises
+// that what is stored before `count` is seen with it then (without the flag the
+// environment decides).
 struct RecordPool {
     std::mutex mu;
     std::vector<PcgRecord *> idle;
@@ -475,7 +478,7 @@ struct RecordPool {
             }
         }
         void *p = nullptr;
-        ESP_HIP(hipHostMalloc(&p, sizeof(PcgRecord), hipHostMallocPortable));
+        ESP_HIP(hipHostMalloc(&p, sizeof(PcgRecord), hipHostMallocPortable | hipHostMallocCoherent));
         return (PcgRecord *)p;
     }
     void give_back(PcgRecord *r) {
