@@ -298,8 +298,8 @@ struct WorkspaceCache {
     }
 };
 WorkspaceCache &workspace_cache() {
-    static WorkspaceCache c;
-    return c;
+    static WorkspaceCache *c = new WorkspaceCache;  // not destroyed: instances may be closed at exit
+    return *c;
 }
 
 // Pinned host blocks that receive the 16-bit column indices of the K_i CSR
@@ -332,8 +332,8 @@ struct PinnedPool {
     }
 };
 PinnedPool &pinned_pool() {
-    static PinnedPool p;
-    return p;
+    static PinnedPool *p = new PinnedPool;  // not destroyed: instances may be closed at exit
+    return *p;
 }
 
 // Copies between a caller's pageable vectors and the device through pinned chunks:
@@ -487,8 +487,8 @@ struct RecordPool {
     }
 };
 RecordPool &record_pool() {
-    static RecordPool p;
-    return p;
+    static RecordPool *p = new RecordPool;  // not destroyed: instances may be closed at exit
+    return *p;
 }
 
 struct espreso_feti_s {
