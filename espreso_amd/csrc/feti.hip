@@ -2512,6 +2512,7 @@ void espreso_feti_s::solve(espreso_feti_stats *out) {
         converged = norm < tol64;
     }
     check_launches("PCG");
+    sync();  // the operator and updates of the last iteration belong to the PCG's time
     double tp = wall();
     last.time_pcg = tp - t0;
     // amplitudes alpha = (GG^T)^-1 G r ; primal u = K~^+ (f - B^T lambda) + R alpha
