@@ -3985,16 +3985,25 @@ int espreso_grid_unit_element(const espreso_grid_problem *p, double *Ke) {
     ESP_API_END
 }
 
+// Subdomain values up to which new nodal loads are split on the host: the device takes 35 to 50 us
+// for the way there and back of a few kB and its check, the host loop 6 us at 384 values, 10 at 5 K, 16 at
+// 10 K (27 subdomains of 4^3 elasticity), 32 at 28 K (the later upload then eats the difference),
+// 49 at 41 K, where the device takes 51 and keeps the loads there.
+static constexpr int64_t HOST_LOADS = 16 * 1024;
+
 int espreso_grid_set_nodal_rhs(espreso_feti *h, const double *g) {
     ESP_API_BEGIN
     ESP_CHECK(h && g, ESPRESO_ERR_ARG, "null argument");
     ESP_CHECK((int)h->l2g.size() == h->nsub, ESPRESO_ERR_STATE, "grid not loaded");
     const int nd = h->ndof;
-    if (h->loaded) {
+    if (h->loaded && h->uoff[h->nsub] > HOST_LOADS) {
         ESP_HIP(hipSetDevice(h->opt.device));
         h->set_nodal_rhs(g);
         return ESPRESO_OK;
     }
+    // a refused load changes nothing
+    for (size_t q = 0; q < (size_t)h->nnodes * nd; q++)
+        ESP_CHECK(std::isfinite(g[q]), ESPRESO_ERR_ARG, "non-finite load");
     std::vector<int> mult(h->nnodes, 0);
     for (int s = 0; s < h->nsub; s++)
         for (int node : h->l2g[s]) mult[node]++;
