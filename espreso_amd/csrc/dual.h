@@ -104,8 +104,8 @@ struct DualDev {
     int nblk = 0;
     int *cblk = nullptr, *ck = nullptr, *blk_ptr = nullptr, *blk_sub = nullptr;
     int64_t *rtoff = nullptr, *dsub_off = nullptr, *noff = nullptr;
-    double *Rt = nullptr, *N = nullptr, *dsub = nullptr;
-    double *RbT = nullptr, *RtT = nullptr;  // R_b and Rt with row-major subdomain blocks
+    double *N = nullptr, *dsub = nullptr;
+    double *RbT = nullptr, *RtT = nullptr;  // R_b and the coarse basis R_b N_s with row-major subdomain blocks
     LamCoarse *le_coarse = nullptr;         // per lambda entry (2 per lambda)
     int max_k = 0;                          // most kernel or coarse columns of a subdomain
     bool coarse_direct = false;             // dsub is the coarse vector (one subdomain per block, in order)

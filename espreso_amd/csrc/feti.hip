@@ -2909,7 +2909,6 @@ void espreso_feti_s::coarse_layout_subdomains() {
     D.coff = upload(coff);
     D.blk_ptr = upload(bptr);
     D.blk_sub = upload(bsub);
-    D.Rt = D.Rb;
     D.RtT = D.RbT;
     D.coarse_direct = true;  // asub is the coarse offset
     D.rtoff = D.rboff;
@@ -3161,9 +3160,10 @@ void espreso_feti_s::load_clusters() {
     D.blk_ptr = upload(bptr);
     D.blk_sub = upload(bsub);
     D.rtoff = upload(rtoff);
-    D.Rt = upload(Rt);
     D.RtT = alloc<double>(rtoff[nsub]);
-    launch_basis_rows(nsub, D.max_m, D.m, D.ck, D.rtoff, D.Rt, D.RtT, st);
+    double *d_Rt = upload(Rt);
+    launch_basis_rows(nsub, D.max_m, D.m, D.ck, D.rtoff, d_Rt, D.RtT, st);
+    release(d_Rt);
     D.N = upload(Ns);
     D.noff = upload(noff);
     D.dsub_off = upload(dsub_off);
