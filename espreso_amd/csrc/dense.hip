@@ -551,9 +551,11 @@ __device__ __forceinline__ double read_lane(double v, int lane) {
 // runs on MFMA over the four waves.  The inverse takes the four diagonal blocks
 // at once (a column per lane) and the blocks below by distance on MFMA, the sum
 // staying in the accumulators (their layout is the B operand of the product
-// with the inverted diagonal block).  60 -> 29 us a step at 64 subdomains of 5^3;
-// beside the MFMA work of the substitution 92 -> 50 us at 64 x 10^3 (wave priority
-// raised: this chain is what the other launches of a step wait for).
+// with the inverted diagonal block).  60 -> 29 us a step at 64 subdomains of 5^3; 92 -> 40
+// at 64 x 10^3 beside the substitution's four-wave tiles (wave priority raised: this chain is
+// what the other launches of a step wait for).  Beside one-wave tiles, which leave a CU
+// no room for a workgroup of four waves until several end, a step mostly waits: 250 us at 512 x 10^3,
+// 200 at 216 x 12^3; those tiles still give the shorter assembly (156 against 173 ms there).
 __global__ void __launch_bounds__(256, 4) k_potrf_diag(const DenseDesc *D, int which, int step) {
     const DenseDesc &d = D[blockIdx.x];
     double *A, *B;

@@ -166,8 +166,8 @@ __global__ void __launch_bounds__(256) k_symv(const SymvItem *__restrict__ items
 // read up to 15 lines past the last column: its buffers are that much longer.
 // Waves owning columns instead of strips, one block's loads in flight, took 745 us at
 // those subdomains and 16 cases (now 596), 421 at 512 uneven elasticity subdomains and 5
-// cases (now 290).  Two steps ahead, 64 columns a load, two waves with four strips or
-// eight with one and x in LDS all take 594 to 635 and 290 to 327 us.
+// cases (now 290).  Two steps ahead, 64 columns a load, 16 strips an item, two waves with four
+// strips or eight with one and x in LDS all take 594 to 659 and 290 to 327 us.
 typedef double v4d __attribute__((ext_vector_type(4)));
 
 // loads with a scalar base and one 32-bit lane offset (no 64-bit address arithmetic per lane)

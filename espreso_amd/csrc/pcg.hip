@@ -28,7 +28,7 @@ static inline unsigned cdiv(int64_t a, int64_t b) { return (unsigned)((a + b - 1
 // a wave.  Pairs of cases halve the instructions and requests of a pass, which is what
 // bounds it once thousands of workgroups are in flight: at 669000 lines of 16 cases (86
 // MB a vector) lambda gather 100 -> 48 us, boundary gather 99 -> 79, projector finish
-// 152 -> 52, partial sums 128 -> 79 (5 TB/s); several lines a thread gain nothing more.
+// 152 -> 47, partial sums 128 -> 76 (5 TB/s); several lines a thread gain nothing more.
 constexpr int LINE_CASES = 16;  // largest K
 template <int W>
 struct Lines {
