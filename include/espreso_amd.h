@@ -301,9 +301,9 @@ int espreso_feti_project(espreso_feti *h, const double *x, double *y);
  * allocate device memory (code under HIP graph capture, tight serving loops).
  * It allocates nothing: its scratch (G x per subdomain and per coarse block,
  * (G G^T)^-1 G x: sum of the kernel dimensions + 2 x the coarse dimension
- * doubles) is a static device array of 2^20 doubles (8 MiB) per GPU, shared by
- * every call on that GPU, so calls that overlap on one GPU race.  A larger
- * coarse space is refused with ESPRESO_ERR_ARG. */
+ * doubles) is the instance's own, at most 2^20 doubles (8 MiB).  Calls on
+ * several instances may overlap on one GPU, those on one instance race.  A
+ * larger coarse space is refused with ESPRESO_ERR_ARG. */
 int espreso_feti_project_device(espreso_feti *h, const double *x, double *y, void *stream);
 int espreso_feti_vec_b(espreso_feti *h, double *b);
 /* SYMV work-item sizes in matrix elements per workgroup, targets[3]: FP64,
