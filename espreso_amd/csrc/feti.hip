@@ -17,6 +17,7 @@
 #include <omp.h>
 #include <map>
 #include <mutex>
+#include <shared_mutex>
 #include <cstdlib>
 #include <chrono>
 #include <cmath>
@@ -206,6 +207,19 @@ void keep_pooled_memory(int device) {
     done[device] = 1;
 }
 
+// The runtime refuses allocations in every thread while one of them captures a graph
+// ("operation not permitted when stream is capturing"), also in ThreadLocal mode: instances
+// that work in several threads allocate and capture in turn
+std::shared_mutex &capture_mutex() {
+    static std::shared_mutex *m = new std::shared_mutex;  // not destroyed: instances may be closed at exit
+    return *m;
+}
+template <class Allocate>
+hipError_t no_capture(Allocate allocate) {
+    std::shared_lock<std::shared_mutex> lock(capture_mutex());
+    return allocate();
+}
+
 // The assembly workspaces (tens to hundreds of GB) are kept for the process
 // once allocated and lent to the instances, largest first fit: memory that
 // was in use before (by an earlier instance, or a block the stream-ordered
@@ -248,7 +262,7 @@ struct WorkspaceCache {
             return best->ptr;
         }
         void *p = nullptr;
-        hipError_t e = hipMalloc(&p, bytes);
+        hipError_t e = no_capture([&] { return hipMalloc(&p, bytes); });
         if (e == hipErrorOutOfMemory) {
             // make room: give the idle blocks of the device back and retry
             (void)hipGetLastError();
@@ -260,7 +274,7 @@ struct WorkspaceCache {
                     ++it;
                 }
             }
-            e = hipMalloc(&p, bytes);
+            e = no_capture([&] { return hipMalloc(&p, bytes); });
         }
         if (e != hipSuccess) {
             (void)hipGetLastError();
@@ -320,7 +334,7 @@ struct PinnedPool {
             }
         }
         void *p = nullptr;
-        if (hipHostMalloc(&p, BLOCK, hipHostMallocDefault) != hipSuccess) {
+        if (no_capture([&] { return hipHostMalloc(&p, BLOCK, hipHostMallocDefault); }) != hipSuccess) {
             (void)hipGetLastError();
             return nullptr;
         }
@@ -422,7 +436,9 @@ struct HostStagePool {
         (void)hipGetDevice(&current);
         if (current != device && hipSetDevice(device) != hipSuccess) return nullptr;
         auto s = std::make_unique<HostStage>();
-        bool ok = hipHostMalloc((void **)&s->buf, HostStage::SLOTS * HostStage::SLOT, hipHostMallocPortable) == hipSuccess;
+        bool ok = no_capture([&] {
+            return hipHostMalloc((void **)&s->buf, HostStage::SLOTS * HostStage::SLOT, hipHostMallocPortable);
+        }) == hipSuccess;
         for (hipEvent_t &e : s->ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
         if (current != device) (void)hipSetDevice(current);
         if (ok) return s;
@@ -478,7 +494,8 @@ struct RecordPool {
             }
         }
         void *p = nullptr;
-        ESP_HIP(hipHostMalloc(&p, sizeof(PcgRecord), hipHostMallocPortable | hipHostMallocCoherent));
+        ESP_HIP(no_capture(
+            [&] { return hipHostMalloc(&p, sizeof(PcgRecord), hipHostMallocPortable | hipHostMallocCoherent); }));
         return (PcgRecord *)p;
     }
     void give_back(PcgRecord *r) {
@@ -682,7 +699,7 @@ struct espreso_feti_s {
                 return p;
             }
         }
-        auto get = [&]() { return hipMallocAsync(&p, bytes, st); };
+        auto get = [&]() { return no_capture([&] { return hipMallocAsync(&p, bytes, st); }); };
         const double ta = measure ? wall() : 0.0;
         hipError_t e = get();
         if (measure && bytes >= ((size_t)256 << 20))
@@ -724,7 +741,7 @@ struct espreso_feti_s {
     double stage_wait_s = 0, stage_copy_s = 0;  // staged uploads: waits for the copy engine, host copies
     void staging_ready() {
         for (int b = 0; b < 2; b++) {
-            if (!stage[b]) ESP_HIP(hipHostMalloc(&stage[b], STAGE_BYTES, hipHostMallocDefault));
+            if (!stage[b]) ESP_HIP(no_capture([&] { return hipHostMalloc(&stage[b], STAGE_BYTES, hipHostMallocDefault); }));
             if (!stage_ev[b]) ESP_HIP(hipEventCreateWithFlags(&stage_ev[b], hipEventDisableTiming));
         }
     }
@@ -2387,6 +2404,7 @@ void espreso_feti_s::pcg_step_graph(const PcgVec &V, int prec) {
             ESP_HIP(hipGraphLaunch(g.exec, st));
             return;
         }
+    std::unique_lock<std::shared_mutex> capture(capture_mutex());
     hipGraph_t graph = nullptr;
     ESP_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
     try {
